@@ -1280,12 +1280,15 @@ svmi_status svmi_measure(svmi_handle h, const double* uniforms, size_t shots, ui
     for (size_t i = 0; i < shots; i++)
         if (blk[i] >= 0) order.push_back(i);
     std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return blk[a] < blk[b]; });
+    // one workgroup per job {block, first draw, draws}; a block's draws are cut
+    // into jobs of kSampleDraws, one draw per thread
+    constexpr uint64_t kSampleDraws = 256;
     std::vector<uint64_t> jobs;
     std::vector<double> offs, draws(order.size());
     for (size_t j = 0; j < order.size(); j++) {
         draws[j] = uniforms[order[j]];
         const uint64_t b = uint64_t(blk[order[j]]);
-        if (jobs.empty() || jobs[jobs.size() - 3] != b) {
+        if (jobs.empty() || jobs[jobs.size() - 3] != b || jobs.back() == kSampleDraws) {
             jobs.push_back(b);
             jobs.push_back(j);
             jobs.push_back(0);
@@ -1296,18 +1299,19 @@ svmi_status svmi_measure(svmi_handle h, const double* uniforms, size_t shots, ui
     const uint32_t njobs = uint32_t(offs.size());
     std::vector<uint64_t> res(order.size());
     if (njobs) {
-        SVMI_TRY(h->scratch[0].ensure(jobs.size() * sizeof(uint64_t)));
-        SVMI_TRY(h->scratch[1].ensure(offs.size() * sizeof(double)));
-        SVMI_TRY(h->scratch[2].ensure(draws.size() * sizeof(double)));
+        // jobs | offsets | draws, all of 8-byte words, in one copy
+        std::vector<uint64_t> in(jobs.size() + offs.size() + draws.size());
+        std::memcpy(in.data(), jobs.data(), jobs.size() * 8);
+        std::memcpy(in.data() + jobs.size(), offs.data(), offs.size() * 8);
+        std::memcpy(in.data() + jobs.size() + offs.size(), draws.data(), draws.size() * 8);
+        SVMI_TRY(h->scratch[0].ensure(in.size() * sizeof(uint64_t)));
         SVMI_TRY(h->scratch[4].ensure(res.size() * sizeof(uint64_t)));
-        SVMI_HIP(hipMemcpyAsync(h->scratch[0].p, jobs.data(), jobs.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
+        SVMI_HIP(hipMemcpyAsync(h->scratch[0].p, in.data(), in.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
                                 h->stream));
-        SVMI_HIP(hipMemcpyAsync(h->scratch[1].p, offs.data(), offs.size() * sizeof(double), hipMemcpyHostToDevice,
-                                h->stream));
-        SVMI_HIP(hipMemcpyAsync(h->scratch[2].p, draws.data(), draws.size() * sizeof(double), hipMemcpyHostToDevice,
-                                h->stream));
-        SVMI_HIP(launch_sample(h->stream, h->sv, nthr, chunk, h->scratch[0].as<uint64_t>(), njobs,
-                               h->scratch[1].as<double>(), h->scratch[2].as<double>(), h->scratch[4].as<uint64_t>()));
+        const uint64_t* din = h->scratch[0].as<uint64_t>();
+        const double* doffs = reinterpret_cast<const double*>(din + jobs.size());
+        SVMI_HIP(launch_sample(h->stream, h->sv, nthr, chunk, din, njobs, doffs, doffs + offs.size(),
+                               h->scratch[4].as<uint64_t>()));
         SVMI_HIP(hipMemcpyAsync(res.data(), h->scratch[4].p, res.size() * sizeof(uint64_t), hipMemcpyDeviceToHost,
                                 h->stream));
         SVMI_HIP(hipStreamSynchronize(h->stream));

@@ -1063,6 +1063,17 @@ k_sample(const c64* __restrict__ s, uint32_t chunk, const uint64_t* __restrict__
     }
 }
 
+// The same search with the block staged in LDS and one thread per draw.  The
+// staged probabilities are replaced by the scan L_j itself, so a draw takes
+// two binary searches (8 steps over the threads' runs, lg inside one run)
+// instead of a pass of the whole workgroup over the block with three
+// barriers: 1024 draws in one 2^12-amplitude block 3365 -> 9.7 us, and the
+// draws of a block run in as many workgroups as the host cuts them into.
+// O + L_j grows along a run (p_j >= 0 and rounding is monotone), but the next
+// run starts from its own prefix and may begin an ulp lower, so the first
+// run with a match is searched in the running maximum of the runs' last
+// values: it first exceeds r where a run's own last value does, which is the
+// smallest j that the definition above asks for.
 __global__ void __launch_bounds__(256)
 k_sample_staged(const c64* __restrict__ s, uint32_t lg, const uint64_t* __restrict__ jobs,
                 const double* __restrict__ offsets, const double* __restrict__ draws,
@@ -1070,33 +1081,53 @@ k_sample_staged(const c64* __restrict__ s, uint32_t lg, const uint64_t* __restri
 {
     extern __shared__ double lp[];
     __shared__ double lds_w[4];
-    __shared__ unsigned long long best;
-    const uint32_t chunk = 1u << lg;
+    __shared__ double top[256];   // running maximum of O + L at the end of each thread's run
+    const uint32_t chunk = 1u << lg, t = threadIdx.x, nthr = blockDim.x;
     const uint64_t b = jobs[3 * blockIdx.x + 0];
     const uint64_t first = jobs[3 * blockIdx.x + 1];
     const uint64_t cnt = jobs[3 * blockIdx.x + 2];
-    const uint64_t bsize = uint64_t(blockDim.x) << lg;
+    const uint64_t bsize = uint64_t(nthr) << lg;
     stage_probs(s + b * bsize, lg, lp);
-    const double P = thread_prefix_staged(lp, lg, lds_w);
+    double acc = thread_prefix_staged(lp, lg, lds_w);
     const double O = offsets[blockIdx.x];
-    const double* mine = lp + threadIdx.x * (chunk + 1);
-    for (uint64_t q = 0; q < cnt; q++) {
+    double* mine = lp + t * (chunk + 1);
+    for (uint32_t i = 0; i < chunk; i++) {
+        acc = __dadd_rn(acc, mine[i]);
+        mine[i] = acc;
+    }
+    const int width = nthr < 64 ? int(nthr) : 64;
+    const int lane = int(t & 63u);
+    double m = __dadd_rn(O, acc);
+    for (int d = 1; d < width; d <<= 1) {
+        const double u = __shfl_up(m, d, width);
+        if (lane >= d && u > m) m = u;
+    }
+    if (lane == width - 1) lds_w[t >> 6] = m;
+    __syncthreads();
+    for (uint32_t v = 0; v < (t >> 6); v++)
+        if (lds_w[v] > m) m = lds_w[v];
+    top[t] = m;
+    __syncthreads();
+    for (uint64_t q = t; q < cnt; q += nthr) {
         const double r = draws[first + q];
-        if (threadIdx.x == 0) best = ~0ull;
-        __syncthreads();
-        double acc = P;
-        uint64_t found = ~0ull;
-        for (uint32_t i = 0; i < chunk; i++) {
-            acc = __dadd_rn(acc, mine[i]);
-            if (__dadd_rn(O, acc) > r) {
-                found = uint64_t(threadIdx.x) * chunk + i;
-                break;
-            }
+        uint32_t lo = 0, len = nthr;   // smallest run with top > r in [lo, lo + len]
+        while (len > 0) {
+            const uint32_t half = len >> 1;
+            if (top[lo + half] > r) len = half;
+            else lo += half + 1, len -= half + 1;
         }
-        if (found != ~0ull) atomicMin(&best, (unsigned long long)found);
-        __syncthreads();
-        if (threadIdx.x == 0) out[first + q] = best == ~0ull ? 0 : b * bsize + best;
-        __syncthreads();
+        uint64_t res = 0;
+        if (lo < nthr) {
+            const double* run = lp + lo * (chunk + 1);
+            uint32_t j = 0;
+            for (len = chunk - 1; len > 0;) {   // the run's last value exceeds r
+                const uint32_t half = len >> 1;
+                if (__dadd_rn(O, run[j + half]) > r) len = half;
+                else j += half + 1, len -= half + 1;
+            }
+            res = b * bsize + (uint64_t(lo) << lg) + j;
+        }
+        out[first + q] = res;
     }
 }
 
