@@ -16,6 +16,7 @@
 #include "svmi_exec.hpp"
 #include "svmi_kernels.hpp"
 #include "svmi_lower.hpp"
+#include "svmi_pauli.hpp"
 #include "svmi_plan.hpp"
 #include "svmi_jit.hpp"
 #include "svmi_qasm.hpp"
@@ -276,26 +277,6 @@ svmi_status check_terms(const svmi_pauli_term* terms, size_t n_terms, int n)
     return SVMI_OK;
 }
 
-// Group terms by X mask; coefficients absorb i^{|x&z|}.
-void group_terms(const svmi_pauli_term* terms, size_t n_terms, std::vector<PauliGroup>& groups,
-                 std::vector<PauliTerm>& out)
-{
-    std::vector<size_t> idx(n_terms);
-    std::iota(idx.begin(), idx.end(), 0);
-    std::stable_sort(idx.begin(), idx.end(), [&](size_t a, size_t b) { return terms[a].xmask < terms[b].xmask; });
-    groups.clear();
-    out.clear();
-    for (size_t i : idx) {
-        const svmi_pauli_term& t = terms[i];
-        if (groups.empty() || groups.back().xmask != t.xmask)
-            groups.push_back(PauliGroup{t.xmask, uint32_t(out.size()), uint32_t(out.size())});
-        const int ny = __builtin_popcountll(t.xmask & t.zmask) & 3;
-        const double re[4] = {1, 0, -1, 0}, im[4] = {0, 1, 0, -1};
-        out.push_back(PauliTerm{t.zmask, t.coeff * re[ny], t.coeff * im[ny]});
-        groups.back().end = uint32_t(out.size());
-    }
-}
-
 svmi_status check_params(const svmi_gate* gates, size_t n_gates, const int32_t* param_slots, size_t n_params)
 {
     if (n_gates && !param_slots) return fail(SVMI_ERR_ARG, "null param_slots");
@@ -472,7 +453,8 @@ svmi_status verify_batch(const BatchPlan& bp)
             g.dst >= uint64_t(bp.n_slots) + bp.circs.size())
             return fail(SVMI_ERR_STATE, "batch plan: bad sum segment");
     for (const BatchCircuit& c : bp.circs)
-        if (c.group_end > bp.groups.size() || c.slot_begin + c.n_slots > bp.n_slots ||
+        if (c.group_begin > c.flat_end || c.flat_end > c.tile_end || c.tile_end > c.group_end ||
+            c.group_end > bp.groups.size() || c.slot_begin + c.n_slots > bp.n_slots ||
             c.e_partial + c.n_e_partials > bp.n_e_partials)
             return fail(SVMI_ERR_STATE, "batch plan: bad circuit record");
     return SVMI_OK;
@@ -498,8 +480,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
     }
     if (total_params && !grads) return fail(SVMI_ERR_ARG, "null gradient array");
     std::vector<int> ni(n_items);
-    std::vector<std::vector<PauliGroup>> pg(n_items);
-    std::vector<std::vector<PauliTerm>> pt(n_items);
+    std::vector<PauliPlan> pauli(n_items);
     bp.fwd.resize(n_items);
     bp.adj.resize(n_items);
     {
@@ -522,7 +503,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 oa.tile_qubits = it.adj_tile ? it.adj_tile : tu.adj_tile;
                 oa.op_overhead = of.op_overhead;
                 build_adjoint_program(entries, ni[i], oa, bp.adj[i]);
-                group_terms(it.terms, it.n_terms, pg[i], pt[i]);
+                plan_pauli(it.terms, it.n_terms, ni[i], kPauliTileQubits, true, 1, pauli[i]);
             }
         };
         std::vector<std::thread> pool;
@@ -576,12 +557,14 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
         bp.state_off[i] = bp.state_bytes;
         bp.state_bytes += ((2 * dim * sizeof(c64)) + 255) & ~uint64_t(255);
         c.group_begin = uint32_t(bp.groups.size());
-        for (PauliGroup g : pg[i]) {
+        c.flat_end = c.group_begin + pauli[i].passes[0].flat_end;
+        c.tile_end = c.group_begin + pauli[i].passes[0].tile_end;
+        for (PauliGroup g : pauli[i].groups) {
             g.begin += uint32_t(bp.terms.size());
             g.end += uint32_t(bp.terms.size());
             bp.groups.push_back(g);
         }
-        bp.terms.insert(bp.terms.end(), pt[i].begin(), pt[i].end());
+        bp.terms.insert(bp.terms.end(), pauli[i].terms.begin(), pauli[i].terms.end());
         c.group_end = uint32_t(bp.groups.size());
         auto& cs = csteps[i];
         const Program& fw = bp.fwd[i];
@@ -868,46 +851,54 @@ svmi_status exec_program(svmi_handle h, const Program& prog, DeviceProgram& dp, 
 }
 
 // <psi|H|psi>, optionally writing lam = H psi.
-// The Pauli tables of `terms` into scratch[0..1] (groups / pt hold them on
-// the host and must outlive the stream's copies: the caller synchronises).
-svmi_status pauli_upload(svmi_handle h, const svmi_pauli_term* terms, size_t n_terms, std::vector<PauliGroup>& groups,
-                         std::vector<PauliTerm>& pt)
+// The plan's tables into scratch[0..1] (the plan must outlive the stream's
+// copies: the caller synchronises).
+svmi_status pauli_upload(svmi_handle h, const svmi_pauli_term* terms, size_t n_terms, bool lam, PauliPlan& plan)
 {
-    group_terms(terms, n_terms, groups, pt);
-    SVMI_TRY(h->scratch[0].ensure(std::max<size_t>(groups.size(), 1) * sizeof(PauliGroup)));
-    SVMI_TRY(h->scratch[1].ensure(std::max<size_t>(pt.size(), 1) * sizeof(PauliTerm)));
-    if (!groups.empty()) {
-        SVMI_HIP(hipMemcpyAsync(h->scratch[0].p, groups.data(), groups.size() * sizeof(PauliGroup),
+    plan_pauli(terms, n_terms, h->n_int, pauli_tile_qubits(h->n_int), lam, kMaxPauliPasses, plan);
+    SVMI_TRY(h->scratch[0].ensure(std::max<size_t>(plan.groups.size(), 1) * sizeof(PauliGroup)));
+    SVMI_TRY(h->scratch[1].ensure(std::max<size_t>(plan.terms.size(), 1) * sizeof(PauliTerm)));
+    if (!plan.groups.empty()) {
+        SVMI_HIP(hipMemcpyAsync(h->scratch[0].p, plan.groups.data(), plan.groups.size() * sizeof(PauliGroup),
                                 hipMemcpyHostToDevice, h->stream));
-        SVMI_HIP(hipMemcpyAsync(h->scratch[1].p, pt.data(), pt.size() * sizeof(PauliTerm), hipMemcpyHostToDevice,
-                                h->stream));
+        SVMI_HIP(hipMemcpyAsync(h->scratch[1].p, plan.terms.data(), plan.terms.size() * sizeof(PauliTerm),
+                                hipMemcpyHostToDevice, h->stream));
     }
     return SVMI_OK;
 }
 
-// lam = H psi (and copy = psi if given) with the uploaded tables of n_groups
-// groups; the block partials of <psi|lam> in scratch[2] (grid of them,
-// returned).
-svmi_status pauli_launch(svmi_handle h, const c64* psi, c64* lam, c64* copy, size_t n_groups, uint32_t* grid_out)
+// Block partials of a plan's passes.
+size_t pauli_partials(svmi_handle h, const PauliPlan& plan)
 {
-    const uint32_t grid = pauli_grid(h->dim);
-    SVMI_TRY(h->scratch[2].ensure(size_t(grid) * sizeof(double)));
-    SVMI_HIP(launch_pauli(h->stream, psi, lam, h->dim, h->scratch[0].as<PauliGroup>(), uint32_t(n_groups),
-                          h->scratch[1].as<PauliTerm>(), h->scratch[2].as<double>(), copy));
-    *grid_out = grid;
+    size_t np = 0;
+    for (const PauliPass& p : plan.passes) np += pauli_grid(h->dim, p);
+    return np;
+}
+
+// lam = H psi (and copy = psi if given), one launch per pass; part: the
+// pauli_partials block partials of <psi|lam>.
+svmi_status pauli_launch(svmi_handle h, const PauliPlan& plan, const PauliGroup* groups, const PauliTerm* terms,
+                         const c64* psi, c64* lam, c64* copy, double* part)
+{
+    bool first = true;
+    for (const PauliPass& p : plan.passes) {
+        SVMI_HIP(launch_pauli(h->stream, psi, lam, h->dim, p, !first, groups, terms, part, first ? copy : nullptr));
+        part += pauli_grid(h->dim, p);
+        first = false;
+    }
     return SVMI_OK;
 }
 
-svmi_status pauli_device(svmi_handle h, const c64* psi, c64* lam, const svmi_pauli_term* terms, size_t n_terms,
-                         double* out)
+svmi_status pauli_device(svmi_handle h, const c64* psi, const svmi_pauli_term* terms, size_t n_terms, double* out)
 {
-    std::vector<PauliGroup> groups;
-    std::vector<PauliTerm> pt;
-    uint32_t grid = 0;
-    SVMI_TRY(pauli_upload(h, terms, n_terms, groups, pt));
-    SVMI_TRY(pauli_launch(h, psi, lam, nullptr, groups.size(), &grid));
-    std::vector<double> part(grid);
-    SVMI_HIP(hipMemcpyAsync(part.data(), h->scratch[2].p, grid * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    PauliPlan plan;
+    SVMI_TRY(pauli_upload(h, terms, n_terms, false, plan));
+    std::vector<double> part(pauli_partials(h, plan));
+    SVMI_TRY(h->scratch[2].ensure(part.size() * sizeof(double)));
+    SVMI_TRY(pauli_launch(h, plan, h->scratch[0].as<PauliGroup>(), h->scratch[1].as<PauliTerm>(), psi, nullptr,
+                          nullptr, h->scratch[2].as<double>()));
+    SVMI_HIP(hipMemcpyAsync(part.data(), h->scratch[2].p, part.size() * sizeof(double), hipMemcpyDeviceToHost,
+                            h->stream));
     SVMI_HIP(hipStreamSynchronize(h->stream));
     double s = 0.0;
     for (double v : part) s += v;
@@ -1326,7 +1317,7 @@ svmi_status svmi_expval(svmi_handle h, const svmi_pauli_term* terms, size_t n_te
     SVMI_TRY(use_device(h));
     if (!out) return fail(SVMI_ERR_ARG, "null output");
     SVMI_TRY(check_terms(terms, n_terms, h->n));
-    return pauli_device(h, h->sv, nullptr, terms, n_terms, out);
+    return pauli_device(h, h->sv, terms, n_terms, out);
 }
 
 svmi_status svmi_expval_static(svmi_handle h, const svmi_pauli_term* terms, size_t n_terms, double* out)
@@ -1337,27 +1328,28 @@ svmi_status svmi_expval_static(svmi_handle h, const svmi_pauli_term* terms, size
     if (n_terms > kStaticMaxTerms)
         return fail(SVMI_ERR_ARG, "svmi_expval_static takes at most " + std::to_string(kStaticMaxTerms) +
                                       " Pauli terms (got " + std::to_string(n_terms) + "); use svmi_expval");
-    std::vector<PauliGroup> groups;
-    std::vector<PauliTerm> pt;
-    group_terms(terms, n_terms, groups, pt);
+    PauliPlan plan;
+    plan_pauli(terms, n_terms, h->n_int, pauli_tile_qubits(h->n_int), false, kMaxPauliPasses, plan);
     // scratch layout: groups | terms | block partials, each 256-B aligned
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-    const uint32_t grid = pauli_grid(h->dim);
-    const size_t og = 0, ot = up(groups.size() * sizeof(PauliGroup)), op = ot + up(pt.size() * sizeof(PauliTerm));
-    if (op + size_t(grid) * sizeof(double) > kStaticScratchBytes)
+    const size_t np = pauli_partials(h, plan);
+    const size_t og = 0, ot = up(plan.groups.size() * sizeof(PauliGroup)),
+                 op = ot + up(plan.terms.size() * sizeof(PauliTerm));
+    if (op + np * sizeof(double) > kStaticScratchBytes)
         return fail(SVMI_ERR_ARG, "svmi_expval_static: tables and partials exceed the static scratch");
     unsigned char* base = static_cast<unsigned char*>(h->static_scratch);
     PauliGroup* dg = reinterpret_cast<PauliGroup*>(base + og);
     PauliTerm* dt = reinterpret_cast<PauliTerm*>(base + ot);
     double* dp = reinterpret_cast<double*>(base + op);
-    if (!groups.empty()) {
-        SVMI_HIP(hipMemcpyAsync(dg, groups.data(), groups.size() * sizeof(PauliGroup), hipMemcpyHostToDevice,
+    if (!plan.groups.empty()) {
+        SVMI_HIP(hipMemcpyAsync(dg, plan.groups.data(), plan.groups.size() * sizeof(PauliGroup),
+                                hipMemcpyHostToDevice, h->stream));
+        SVMI_HIP(hipMemcpyAsync(dt, plan.terms.data(), plan.terms.size() * sizeof(PauliTerm), hipMemcpyHostToDevice,
                                 h->stream));
-        SVMI_HIP(hipMemcpyAsync(dt, pt.data(), pt.size() * sizeof(PauliTerm), hipMemcpyHostToDevice, h->stream));
     }
-    SVMI_HIP(launch_pauli(h->stream, h->sv, nullptr, h->dim, dg, uint32_t(groups.size()), dt, dp));
-    std::vector<double> part(grid);
-    SVMI_HIP(hipMemcpyAsync(part.data(), dp, grid * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    SVMI_TRY(pauli_launch(h, plan, dg, dt, h->sv, nullptr, nullptr, dp));
+    std::vector<double> part(np);
+    SVMI_HIP(hipMemcpyAsync(part.data(), dp, np * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     SVMI_HIP(hipStreamSynchronize(h->stream));
     double sum = 0.0;
     for (double v : part) sum += v;
@@ -1378,16 +1370,17 @@ svmi_status svmi_adjoint(svmi_handle h, const svmi_pauli_term* terms, size_t n_t
     SVMI_TRY(h->aux[0].ensure(h->dim * sizeof(c64)));
     SVMI_TRY(h->aux[1].ensure(h->dim * sizeof(c64)));
     // the observable's tables go up while the stream is idle
-    std::vector<PauliGroup> groups;
-    std::vector<PauliTerm> pt;
-    SVMI_TRY(pauli_upload(h, terms, n_terms, groups, pt));
+    PauliPlan plan;
+    SVMI_TRY(pauli_upload(h, terms, n_terms, true, plan));
     // forward
     SVMI_TRY(exec_program(h, h->prog, h->dprog, h->sv, nullptr, nullptr, nullptr, &h->jit));
     // phi = psi and lam = H psi in one pass, partials of E = <psi|lam>
     c64* phi = h->aux[0].as<c64>();
     c64* lam = h->aux[1].as<c64>();
-    uint32_t grid = 0;
-    SVMI_TRY(pauli_launch(h, h->sv, lam, phi, groups.size(), &grid));
+    const size_t np = pauli_partials(h, plan);
+    SVMI_TRY(h->scratch[2].ensure(np * sizeof(double)));
+    SVMI_TRY(pauli_launch(h, plan, h->scratch[0].as<PauliGroup>(), h->scratch[1].as<PauliTerm>(), h->sv, lam, phi,
+                          h->scratch[2].as<double>()));
     for (size_t p = 0; p < n_params; p++) grad_out[p] = 0.0;
     // backward (planned once per circuit and parameter map)
     const size_t n_slots = 3 * h->gates.size();
@@ -1406,11 +1399,11 @@ svmi_status svmi_adjoint(svmi_handle h, const svmi_pauli_term* terms, size_t n_t
     }
     const Program& bp = h->adj_prog;
     SVMI_TRY(exec_program(h, bp, h->adj_dprog, phi, lam, h->adj_gsum.as<double>()));
-    std::vector<double> g(bp.n_grad), part(grid);
+    std::vector<double> g(bp.n_grad), part(np);
     if (bp.n_grad)
         SVMI_HIP(hipMemcpyAsync(g.data(), h->adj_gsum.p, bp.n_grad * sizeof(double), hipMemcpyDeviceToHost,
                                 h->stream));
-    SVMI_HIP(hipMemcpyAsync(part.data(), h->scratch[2].p, grid * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    SVMI_HIP(hipMemcpyAsync(part.data(), h->scratch[2].p, np * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     SVMI_HIP(hipStreamSynchronize(h->stream));
     double E = 0.0;
     for (double v : part) E += v;
@@ -1815,26 +1808,37 @@ void host_program(Program& prog, std::vector<c64>& s0, std::vector<c64>& s1, std
 void host_pauli(int n, const std::vector<c64>& psi, std::vector<c64>* lam, const svmi_pauli_term* terms,
                 size_t n_terms, double* E)
 {
-    std::vector<PauliGroup> groups;
-    std::vector<PauliTerm> pt;
-    group_terms(terms, n_terms, groups, pt);
+    // small tiles, so that small states run several passes
+    PauliPlan plan;
+    plan_pauli(terms, n_terms, n, std::min(n, 6), lam != nullptr, kMaxPauliPasses, plan);
     const uint64_t dim = 1ull << n;
     double acc = 0.0;
-    for (uint64_t y = 0; y < dim; y++) {
-        c64 l{0.0, 0.0};
-        for (const PauliGroup& G : groups) {
-            const uint64_t x = y ^ G.xmask;
-            double fr = 0.0, fi = 0.0;
-            for (uint32_t t = G.begin; t < G.end; t++) {
-                const bool neg = __builtin_popcountll(x & pt[t].zmask) & 1;
-                fr += neg ? -pt[t].cre : pt[t].cre;
-                fi += neg ? -pt[t].cim : pt[t].cim;
+    std::vector<c64> out(dim, c64{0.0, 0.0});
+    for (const PauliPass& p : plan.passes)
+        for (uint64_t y = 0; y < dim; y++) {
+            uint32_t loc = 0;
+            for (uint32_t b = 0; b < p.k; b++) loc |= uint32_t((y >> p.pos[b]) & 1) << b;
+            const uint64_t base = y & p.extmask;
+            c64 l{0.0, 0.0};
+            for (uint32_t gi = p.begin; gi < p.end; gi++) {
+                const PauliGroup& G = plan.groups[gi];
+                uint64_t x = y ^ G.xmask;
+                if (gi < p.tile_end) {
+                    x = base;
+                    for (uint32_t b = 0; b < p.k; b++) x |= uint64_t(((loc ^ G.xmask) >> b) & 1) << p.pos[b];
+                }
+                double fr = 0.0, fi = 0.0;
+                for (uint32_t t = G.begin; t < G.end; t++) {
+                    const bool neg = __builtin_popcountll(y & plan.terms[t].zmask) & 1;
+                    fr += neg ? -plan.terms[t].cre : plan.terms[t].cre;
+                    fi += neg ? -plan.terms[t].cim : plan.terms[t].cim;
+                }
+                l = cmac(l, c64{fr, fi}, psi[x]);
             }
-            l = cmac(l, c64{fr, fi}, psi[x]);
+            out[y] = cadd(out[y], l);
+            acc += psi[y].re * l.re + psi[y].im * l.im;
         }
-        if (lam) (*lam)[y] = l;
-        acc += psi[y].re * l.re + psi[y].im * l.im;
-    }
+    if (lam) *lam = out;
     *E = acc;
 }
 
@@ -1949,7 +1953,7 @@ svmi_status svmi_debug_emulate_batch(const svmi_batch_item* items, size_t n_item
                         const uint64_t x = y ^ G.xmask;
                         double fr = 0.0, fi = 0.0;
                         for (uint32_t t = G.begin; t < G.end; t++) {
-                            const bool neg = __builtin_popcountll(x & bp.terms[t].zmask) & 1;
+                            const bool neg = __builtin_popcountll(y & bp.terms[t].zmask) & 1;
                             fr += neg ? -bp.terms[t].cre : bp.terms[t].cre;
                             fi += neg ? -bp.terms[t].cim : bp.terms[t].cim;
                         }

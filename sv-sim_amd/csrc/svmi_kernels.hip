@@ -440,65 +440,177 @@ k_batch_adj(SVMI_BATCH_TABLES, double* __restrict__ grad_partials, uint32_t s0, 
                          blockDim.x, smem, false);
 }
 
-// <H> step: lam = H phi on a chunk of kPauliChunk amplitudes and the chunk's
-// partial sum of Re <phi|lam>.
-__global__ void __launch_bounds__(kThreads)
+// ------------------------------------------------------------- Pauli sums
+//
+// The thread's M amplitudes of H psi at y = yb | col[j] (j < M): tile groups
+// read the tile in LDS (thread tid's register j is tile-local index
+// tid + nt j), the others read psi from memory.  A term's sign is
+// (-1)^{|yb & z|} per thread times a uniform sign per register (jsign), so a
+// term costs a few integer operations per thread and one add per amplitude
+// instead of a 64-bit population count per amplitude.
+//
+// Loads go in batches of up to 4, all issued before the first is used (left
+// to itself the compiler keeps two LDS reads in flight here, and a pass over
+// 28 qubits with 8 masks takes 2.84 ms instead of 1.0; all 29 masks of an
+// Ising sum there 16.5 -> 4.1 ms, in 3 passes that read 4.3 GB each).
+
+// l[j] += (cre + i cim) v[j - j0], j0 <= j < j0 + B
+template <int M, int B>
+__device__ __attribute__((always_inline)) inline void
+pauli_add(c64 (&l)[M], const c64 (&v)[B], int j0, double cre, double cim)
+{
+#pragma unroll
+    for (int j = 0; j < B; j++) {
+        l[j0 + j].re = SVMI_FMA(cre, v[j].re, l[j0 + j].re);
+        l[j0 + j].im = SVMI_FMA(cre, v[j].im, l[j0 + j].im);
+    }
+    if (cim != 0.0)   // uniform
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            l[j0 + j].re = SVMI_FMA(-cim, v[j].im, l[j0 + j].re);
+            l[j0 + j].im = SVMI_FMA(cim, v[j].re, l[j0 + j].im);
+        }
+}
+
+// the amplitudes of registers j0 .. j0 + B - 1 with the tile-local bits x flipped
+template <int B>
+__device__ __attribute__((always_inline)) inline void
+pauli_tile_read(c64 (&v)[B], const c64* t, int j0, uint32_t tid, uint32_t nt, uint32_t x)
+{
+    const uint32_t at = tid ^ x;   // x's thread bits, and its register bits above them
+    if (x < nt) {
+#pragma unroll
+        for (int j = 0; j < B; j++) v[j] = t[at + nt * (j0 + j)];
+    } else {
+#pragma unroll
+        for (int j = 0; j < B; j++) v[j] = t[at ^ (nt * (j0 + j))];
+    }
+}
+
+// kFull: the tile has all nt * M amplitudes (otherwise tsize, the rest unused).
+template <int M, bool kFull>
+__device__ __attribute__((always_inline)) inline void
+pauli_groups(c64 (&l)[M], const c64* t, const c64* __restrict__ psi, uint64_t yb, const uint64_t (&col)[M], uint32_t tid,
+             uint32_t nt, uint32_t tsize, const PauliGroup* __restrict__ groups,
+             const PauliTerm* __restrict__ terms, uint32_t g0, uint32_t gf, uint32_t gt, uint32_t g1)
+{
+    constexpr int B = M < 4 ? M : 4;
+#pragma unroll
+    for (int j = 0; j < M; j++) l[j] = c64{0.0, 0.0};
+    if (g0 < gf) {   // group records and terms are read one group ahead
+        const PauliTerm* __restrict__ ft = terms + groups[g0].begin;
+        uint32_t x = uint32_t(groups[g0].xmask);
+        double cre = ft[0].cre, cim = ft[0].cim;
+        for (uint32_t g = g0; g < gf; g++) {
+            const uint32_t nxt = g + 1 < gf ? g + 1 : g;
+            const uint32_t xn = uint32_t(groups[nxt].xmask);
+            const double cren = ft[nxt - g0].cre, cimn = ft[nxt - g0].cim;
+#pragma unroll
+            for (int j0 = 0; j0 < M; j0 += B) {
+                c64 v[B];
+                pauli_tile_read<B>(v, t, j0, tid, nt, x);
+                __builtin_amdgcn_sched_barrier(0);
+                pauli_add<M, B>(l, v, j0, cre, cim);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            x = xn, cre = cren, cim = cimn;
+        }
+    }
+    for (uint32_t g = gf; g < g1; g++) {
+        const PauliGroup G = groups[g];
+        const bool tile = g < gt;
+        for (uint32_t part = 0; part <= G.imag; part++) {   // real coefficients, then imaginary ones
+            double f[M];
+#pragma unroll
+            for (int j = 0; j < M; j++) f[j] = 0.0;
+            for (uint32_t e = G.begin; e < G.end; e++) {
+                const PauliTerm T = terms[e];
+                const double c0 = part ? T.cim : T.cre;
+                const double c = (__popcll(yb & T.zmask) & 1) ? -c0 : c0;
+#pragma unroll
+                for (int j = 0; j < M; j++)   // +-c as a scalar +-1.0 in one FMA
+                    f[j] = SVMI_FMA(__hiloint2double(int(0x3ff00000u | (T.jsign >> j) << 31), 0), c, f[j]);
+            }
+#pragma unroll
+            for (int j0 = 0; j0 < M; j0 += B) {
+                c64 v[B];
+                if (tile) {
+                    pauli_tile_read<B>(v, t, j0, tid, nt, uint32_t(G.xmask));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        if (kFull || tid + nt * (j0 + j) < tsize) v[j] = psi[(yb | col[j0 + j]) ^ G.xmask];
+                        else v[j] = c64{0.0, 0.0};
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (part) {
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        l[j0 + j].re = SVMI_FMA(-f[j0 + j], v[j].im, l[j0 + j].re);
+                        l[j0 + j].im = SVMI_FMA(f[j0 + j], v[j].re, l[j0 + j].im);
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        l[j0 + j].re = SVMI_FMA(f[j0 + j], v[j].re, l[j0 + j].re);
+                        l[j0 + j].im = SVMI_FMA(f[j0 + j], v[j].im, l[j0 + j].im);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// <H> step: lam = H phi on a tile of the low qubits (kPauliChunk amplitudes,
+// or the whole state where it is smaller) and the tile's partial sum of
+// Re <phi|lam>.  The tile is staged in LDS, so only X masks above it read
+// memory (from L2 mostly): 96 circuits of 10-20 qubits 2.09 -> 0.68 ms.
+__global__ void __launch_bounds__(kPauliThreads, 4)
 k_batch_pauli(BatchArgs a, uint32_t s0, uint32_t s1, uint64_t task0)
 {
-    __shared__ double red[kThreads];
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int M = kPauliRegs;
+    c64* tl = reinterpret_cast<c64*>(smem);
     const uint64_t t = task0 + blockIdx.x;
     const BatchStep st = a.steps[batch_step_of(a.steps, s0, s1, t)];
     const BatchCircuit& c = a.circuits[st.circuit];
     const uint64_t task = t - st.task_begin;
-    const uint64_t dim = 1ull << c.n;
+    const uint32_t tsize = c.n < uint32_t(kPauliTileQubits) ? 1u << c.n : kPauliChunk;
     const uint64_t y0 = task * kPauliChunk;
-    const uint64_t y1 = y0 + kPauliChunk < dim ? y0 + kPauliChunk : dim;
-    // the thread's kPauliPerThread amplitudes y0 + tid + 256 j in registers,
-    // groups and terms outermost: each term is read once per thread, not
-    // once per amplitude (same sums in the same order as one amplitude at a
-    // time)
-    constexpr int M = kPauliChunk / kThreads;
+    const uint32_t tid = threadIdx.x;
     c64 l[M];
+    uint64_t col[M];
 #pragma unroll
-    for (int j = 0; j < M; j++) l[j] = c64{0.0, 0.0};
-    for (uint32_t g = c.group_begin; g < c.group_end; g++) {
-        const PauliGroup G = a.groups[g];
-        double fr[M], fi[M];
-#pragma unroll
-        for (int j = 0; j < M; j++) fr[j] = fi[j] = 0.0;
-        for (uint32_t e = G.begin; e < G.end; e++) {
-            const PauliTerm T = a.terms[e];
-#pragma unroll
-            for (int j = 0; j < M; j++) {
-                const uint64_t x = (y0 + threadIdx.x + uint64_t(kThreads) * j) ^ G.xmask;
-                const bool neg = __popcll(x & T.zmask) & 1;
-                fr[j] += neg ? -T.cre : T.cre;
-                fi[j] += neg ? -T.cim : T.cim;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < M; j++) {
-            const uint64_t y = y0 + threadIdx.x + uint64_t(kThreads) * j;
-            if (y < y1) l[j] = cmac(l[j], c64{fr[j], fi[j]}, c.phi[y ^ G.xmask]);
-        }
-    }
+    for (int j = 0; j < M; j++) col[j] = uint64_t(kPauliThreads) * j;
+    const c64* phi = c.phi;
+    for (uint32_t x = tid; x < tsize; x += kPauliThreads) tl[x] = phi[y0 + x];
+    __syncthreads();
+    if (tsize == kPauliChunk)
+        pauli_groups<M, true>(l, tl, phi, y0 + tid, col, tid, kPauliThreads, tsize, a.groups, a.terms, c.group_begin,
+                              c.flat_end, c.tile_end, c.group_end);
+    else
+        pauli_groups<M, false>(l, tl, phi, y0 + tid, col, tid, kPauliThreads, tsize, a.groups, a.terms, c.group_begin,
+                               c.flat_end, c.tile_end, c.group_end);
     double acc = 0.0;
 #pragma unroll
     for (int j = 0; j < M; j++) {
-        const uint64_t y = y0 + threadIdx.x + uint64_t(kThreads) * j;
-        if (y < y1) {
-            c.lam[y] = l[j];
-            const c64 p = c.phi[y];
+        const uint32_t x = tid + kPauliThreads * j;
+        if (x < tsize) {
+            c.lam[y0 + x] = l[j];
+            const c64 p = tl[x];
             acc += p.re * l[j].re + p.im * l[j].im;
         }
     }
-    red[threadIdx.x] = acc;
+    __syncthreads();
+    double* red = reinterpret_cast<double*>(smem);
+    red[tid] = acc;
     __syncthreads();
     for (uint32_t k = blockDim.x / 2; k > 0; k >>= 1) {
-        if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+        if (tid < k) red[tid] += red[tid + k];
         __syncthreads();
     }
-    if (threadIdx.x == 0) a.e_partials[st.partial + task] = red[0];
+    if (tid == 0) a.e_partials[st.partial + task] = red[0];
 }
 
 size_t batch_launch_smem(uint32_t kind, uint32_t k, uint32_t max_grad, uint32_t max_xf)
@@ -508,7 +620,7 @@ size_t batch_launch_smem(uint32_t kind, uint32_t k, uint32_t max_grad, uint32_t 
         const size_t nwaves = (size_t(sweep_threads(k, 2)) + 63) / 64;
         return (size_t(32) << k) + size_t(16) * max_xf + size_t(8) * max_grad * nwaves;
     }
-    return 0;
+    return kind == BSTEP_PAULI ? size_t(16) * kPauliChunk : 0;
 }
 
 // The k_batch_fwd build of a forward launch.
@@ -531,7 +643,7 @@ hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L
     if (smem > g_max_smem) return hipErrorInvalidConfiguration;
     const uint32_t threads = L.kind == BSTEP_FWD ? sweep_threads(L.k, 1)
                              : L.kind == BSTEP_ADJ ? sweep_threads(L.k, 2)
-                                                   : kThreads;
+                                                   : kPauliThreads;
     const uint64_t max_grid = 1ull << 30;
     for (uint64_t t0 = 0; t0 < L.n_tasks; t0 += max_grid) {
         const uint32_t cnt = uint32_t(L.n_tasks - t0 < max_grid ? L.n_tasks - t0 : max_grid);
@@ -548,7 +660,7 @@ hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L
                                a.phases, a.ops, a.coef, a.hitab, a.grad_partials, L.step_begin, L.step_end, first);
             break;
         case BSTEP_PAULI:
-            hipLaunchKernelGGL(k_batch_pauli, dim3(cnt), dim3(threads), 0, st, a, L.step_begin, L.step_end, first);
+            hipLaunchKernelGGL(k_batch_pauli, dim3(cnt), dim3(threads), smem, st, a, L.step_begin, L.step_end, first);
             break;
         default:
             return hipErrorInvalidValue;
@@ -1188,79 +1300,75 @@ hipError_t launch_sample(hipStream_t st, const c64* s, uint32_t nthr, uint32_t c
     return hipGetLastError();
 }
 
-// ----------------------------------------------------------- Pauli sums
-//
-// lam[y] = sum_g sum_{t in g} c'_t (-1)^{|x & z_t|} psi[x], x = y ^ xmask_g,
-// c'_t = coeff_t * i^{|xmask & zmask_t|}.  Block partials of
-// Re(conj(psi[y]) lam[y]) give <psi|H|psi>.
+// ------------------------------------------------- Pauli sums of one state
 
-__global__ void __launch_bounds__(256)
-k_pauli(const c64* __restrict__ psi, c64* __restrict__ lam, uint64_t dim,
-        const PauliGroup* __restrict__ groups, uint32_t ngroups, const PauliTerm* __restrict__ terms,
-        double* __restrict__ partials, c64* __restrict__ copy)
+template <int M>
+__global__ void __launch_bounds__(kPauliThreads, 4)
+k_pauli(const c64* __restrict__ psi, c64* __restrict__ lam, uint64_t n_tiles, const PauliPass P, int accumulate,
+        const PauliGroup* __restrict__ groups, const PauliTerm* __restrict__ terms, double* __restrict__ partials,
+        c64* __restrict__ copy)
 {
-    __shared__ double red[256];
+    extern __shared__ __align__(16) unsigned char smem[];
+    c64* tl = reinterpret_cast<c64*>(smem);
+    const uint32_t tid = threadIdx.x, nt = blockDim.x;   // nt = 512, or 2^k < 512 with M = 1
+    uint64_t toff = 0;
+#pragma unroll
+    for (int b = 0; b < kPauliThreadBits; b++) toff |= uint64_t((tid >> b) & 1u) << P.pos[b];   // bits >= k of tid are 0
+    uint64_t col[M];
+#pragma unroll
+    for (int j = 0; j < M; j++) col[j] = P.col[j];
     double acc = 0.0;
-    // blocks of kPauliPerThread x 256 amplitudes, grid-strided; each thread
-    // keeps its kPauliPerThread amplitudes in registers with the groups and
-    // terms outermost, so each term is read once per block, not per amplitude
-    constexpr int M = kPauliPerThread;
-    for (uint64_t yb = uint64_t(blockIdx.x) * blockDim.x * M; yb < dim; yb += uint64_t(gridDim.x) * blockDim.x * M) {
-        c64 l[M];
-#pragma unroll
-        for (int j = 0; j < M; j++) l[j] = c64{0.0, 0.0};
-        for (uint32_t g = 0; g < ngroups; g++) {
-            const PauliGroup G = groups[g];
-            double fr[M], fi[M];
-#pragma unroll
-            for (int j = 0; j < M; j++) fr[j] = fi[j] = 0.0;
-            for (uint32_t t = G.begin; t < G.end; t++) {
-                const PauliTerm T = terms[t];
-#pragma unroll
-                for (int j = 0; j < M; j++) {
-                    const uint64_t x = (yb + threadIdx.x + uint64_t(blockDim.x) * j) ^ G.xmask;
-                    const bool neg = __popcll(x & T.zmask) & 1;
-                    fr[j] += neg ? -T.cre : T.cre;
-                    fi[j] += neg ? -T.cim : T.cim;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < M; j++) {
-                const uint64_t y = yb + threadIdx.x + uint64_t(blockDim.x) * j;
-                if (y < dim) l[j] = cmac(l[j], c64{fr[j], fi[j]}, psi[y ^ G.xmask]);
-            }
-        }
+    for (uint64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+        const uint64_t yb = deposit_bits(tile, P.extmask) | toff;
 #pragma unroll
         for (int j = 0; j < M; j++) {
-            const uint64_t y = yb + threadIdx.x + uint64_t(blockDim.x) * j;
-            if (y < dim) {
-                if (lam) lam[y] = l[j];
-                const c64 p = psi[y];
-                if (copy) copy[y] = p;
-                acc += p.re * l[j].re + p.im * l[j].im;
-            }
+            const c64 v = psi[yb | col[j]];
+            tl[tid + nt * j] = v;
+            if (copy) copy[yb | col[j]] = v;
         }
-    }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (uint32_t s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+        __syncthreads();
+        c64 l[M];
+        pauli_groups<M, true>(l, tl, psi, yb, col, tid, nt, nt * M, groups, terms, P.begin, P.flat_end, P.tile_end,
+                              P.end);
+#pragma unroll
+        for (int j = 0; j < M; j++) {
+            const c64 v = tl[tid + nt * j];
+            acc += v.re * l[j].re + v.im * l[j].im;
+        }
+        if (lam) {
+            if (accumulate)
+#pragma unroll
+                for (int j = 0; j < M; j++) l[j] = cadd(l[j], lam[yb | col[j]]);
+#pragma unroll
+            for (int j = 0; j < M; j++) lam[yb | col[j]] = l[j];
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
+    double* red = reinterpret_cast<double*>(smem);
+    red[tid] = acc;
+    __syncthreads();
+    for (uint32_t s = nt / 2; s > 0; s >>= 1) {
+        if (tid < s) red[tid] += red[tid + s];
+        __syncthreads();
+    }
+    if (tid == 0) partials[blockIdx.x] = red[0];
 }
 
-uint32_t pauli_grid(uint64_t dim)
+uint32_t pauli_grid(uint64_t dim, const PauliPass& pass)
 {
-    const uint64_t g = grid_for(dim, 256 * kPauliPerThread);
+    const uint64_t g = dim >> pass.k;
     return g > 2048 ? 2048 : uint32_t(g);
 }
 
-hipError_t launch_pauli(hipStream_t st, const c64* psi, c64* lam, uint64_t dim, const PauliGroup* groups,
-                        uint32_t ngroups, const PauliTerm* terms, double* partials, c64* copy)
+hipError_t launch_pauli(hipStream_t st, const c64* psi, c64* lam, uint64_t dim, const PauliPass& pass,
+                        bool accumulate, const PauliGroup* groups, const PauliTerm* terms, double* partials,
+                        c64* copy)
 {
-    hipLaunchKernelGGL(k_pauli, dim3(pauli_grid(dim)), dim3(256), 0, st, psi, lam, dim, groups, ngroups,
-                       terms, partials, copy);
+    auto* fn = pass.k == 12 ? &k_pauli<8> : pass.k == 10 ? &k_pauli<2> : pass.k <= 9 ? &k_pauli<1> : nullptr;
+    if (!fn) return hipErrorInvalidValue;
+    const uint32_t nt = pass.k < 9 ? 1u << pass.k : uint32_t(kPauliThreads);
+    hipLaunchKernelGGL(fn, dim3(pauli_grid(dim, pass)), dim3(nt), size_t(16) << pass.k, st, psi, lam, dim >> pass.k,
+                       pass, int(accumulate), groups, terms, partials, copy);
     return hipGetLastError();
 }
 

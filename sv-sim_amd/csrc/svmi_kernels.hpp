@@ -7,13 +7,37 @@
 
 namespace svmi {
 
+// Pauli sums (planned by plan_pauli, svmi_pauli.cpp).  A group holds the terms
+// of one X mask: (H psi)[y] = sum_groups f(y) psi[y ^ xmask] with
+// f(y) = sum_terms (-1)^{|y & zmask|} (cre + i cim).
 struct PauliGroup {
-    uint64_t xmask;
-    uint32_t begin, end;
+    uint64_t xmask;      // physical, or tile-local for a pass's tile groups
+    uint32_t begin, end; // terms
+    uint32_t imag;       // some term has cim != 0
+    uint32_t flat;       // one term with zmask 0: f is a constant
 };
 struct PauliTerm {
     uint64_t zmask;
-    double cre, cim;   // coeff * i^{|xmask & zmask|}
+    double cre, cim;     // coeff * i^{|x & z|} * (-1)^{|x & z|}
+    uint32_t jsign;      // bit j: parity of zmask on register j's offset (PauliPass::col[j])
+    uint32_t pad;
+};
+constexpr int kPauliTileQubits = 12;   // 2^12 amplitudes: 64 KiB of LDS, two workgroups per CU
+constexpr int kPauliThreadBits = 9;    // tile-local bits of the 512 threads, the rest are registers
+constexpr int kPauliThreads = 1 << kPauliThreadBits;
+constexpr int kPauliRegs = 1 << (kPauliTileQubits - kPauliThreadBits);
+constexpr int kPauliLow = 4;           // low qubits every tile keeps: 256-byte segments
+constexpr int kMaxPauliPasses = 6;
+// One pass over the state in tiles of the qubits pos[0..k): its groups
+// [begin, tile_end) flip tile qubits only and read the tile in LDS -- those of
+// [begin, flat_end) are flat and have consecutive terms -- and its groups
+// [tile_end, end) read psi[y ^ xmask] from memory.
+struct PauliPass {
+    uint64_t extmask;    // qubits outside the tile
+    uint64_t col[kPauliRegs];   // physical offset of register j
+    uint32_t pos[kPauliTileQubits];
+    uint32_t k;
+    uint32_t begin, flat_end, tile_end, end;
 };
 
 // ---- batched execution (one launch per dependency level) ----
@@ -34,7 +58,7 @@ struct BatchCircuit {
     c64* phi;             // state (forward result, then adjoint phi)
     c64* lam;             // H psi, then adjoint lambda
     uint32_t n;           // qubits of the device state
-    uint32_t group_begin, group_end;   // Pauli groups
+    uint32_t group_begin, flat_end, tile_end, group_end;   // Pauli groups, as a PauliPass has them
     uint32_t e_partial, n_e_partials;  // PAULI partials
     uint32_t slot_begin, n_slots;      // gradient accumulators (global numbering)
 };
@@ -53,10 +77,7 @@ struct BatchArgs {
     double* grad_partials;
 };
 
-constexpr uint32_t kPauliChunk = 4096;     // amplitudes per Pauli task
-static_assert(kPauliChunk % kThreads == 0, "a Pauli task is whole registers of its 256 threads");
-constexpr int kPauliPerThread = 4;         // amplitudes per thread per k_pauli block
-
+constexpr uint32_t kPauliChunk = 1u << kPauliTileQubits;   // amplitudes per Pauli task of a batch
 
 // One launch of a batch: the steps [step_begin, step_end) of one level,
 // all of one kind and (sweeps) one tile size k; their tasks are
@@ -97,10 +118,13 @@ hipError_t launch_block_totals(hipStream_t st, const c64* s, uint64_t nblocks, u
 hipError_t launch_sample(hipStream_t st, const c64* s, uint32_t nthr, uint32_t chunk,
                          const uint64_t* jobs, uint32_t njobs, const double* offsets,
                          const double* draws, uint64_t* out);
-uint32_t pauli_grid(uint64_t dim);
-// copy (optional): also copy[y] = psi[y]
-hipError_t launch_pauli(hipStream_t st, const c64* psi, c64* lam, uint64_t dim, const PauliGroup* groups,
-                        uint32_t ngroups, const PauliTerm* terms, double* partials, c64* copy = nullptr);
+// One pass of a Pauli sum: lam (optional) = or, with `accumulate`, += the pass's
+// groups applied to psi; copy (optional) = psi; pauli_grid partials of
+// Re <psi | the pass's part of H psi>.
+uint32_t pauli_grid(uint64_t dim, const PauliPass& pass);
+hipError_t launch_pauli(hipStream_t st, const c64* psi, c64* lam, uint64_t dim, const PauliPass& pass,
+                        bool accumulate, const PauliGroup* groups, const PauliTerm* terms, double* partials,
+                        c64* copy = nullptr);
 // dst[seg.dst] = sum of src[seg.src, seg.src + seg.len), per segment, in a
 // fixed order (one workgroup per segment).
 struct SumSegment {

@@ -1,0 +1,26 @@
+// svmi_pauli.hpp -- grouping and tiling of Pauli sums (host only).
+#pragma once
+
+#include <vector>
+
+#include "../../include/svmi.h"
+#include "svmi_kernels.hpp"
+
+namespace svmi {
+
+struct PauliPlan {
+    std::vector<PauliGroup> groups;   // in pass order
+    std::vector<PauliTerm> terms;
+    std::vector<PauliPass> passes;    // the first covers every amplitude of lam; at least one
+};
+
+// Plan for a state of n qubits with tiles of up to tile_qubits (<= kPauliTileQubits);
+// lam: H psi is written, not only summed.  max_passes 1: one pass whose tiles
+// are the lowest qubits.
+void plan_pauli(const svmi_pauli_term* terms, size_t n_terms, int n, int tile_qubits, bool lam, int max_passes,
+                PauliPlan& plan);
+
+// Tile size for a state of n qubits.
+int pauli_tile_qubits(int n);
+
+}  // namespace svmi
