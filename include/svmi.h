@@ -97,12 +97,14 @@ typedef struct svmi_stats {
 /* Engine options (svmi_set_option). */
 typedef enum svmi_option {
     SVMI_OPT_FUSION = 0,      /* 1 = tiled multi-gate sweeps (default), 0 = one pass per op */
-    SVMI_OPT_TILE_QUBITS = 1, /* qubits per LDS tile (4..13, default 12)                    */
-    SVMI_OPT_LOW_QUBITS = 2,  /* low qubits every tile keeps for coalescing (2..6, default 4) */
+    SVMI_OPT_TILE_QUBITS = 1, /* qubits per tile (4..13, two states up to 12; default by state size:
+                                 12, from 20 qubits on 13 (two states 11 and 12))             */
+    SVMI_OPT_LOW_QUBITS = 2,  /* low qubits every tile keeps for coalescing (0..8, default 4, from
+                                 20 qubits on 3 with the default tile)                        */
     SVMI_OPT_SWEEP_FLOPS = 3, /* per-amplitude FMA budget of one sweep (0 = unlimited)      */
     SVMI_OPT_PROFILE = 4,     /* 1 = time every launch with HIP events (svmi_stats)         */
-    SVMI_OPT_PIPELINE = 5,    /* 1 = persistent sweeps prefetching the next tile,
-                                 2 = the same with one 512-VGPR workgroup per CU, 0 = off (default) */
+    SVMI_OPT_PIPELINE = 5,    /* 0..64, no effect: every sweep holds its tile in registers and
+                                 leaves the overlap of tiles to the workgroups of a CU        */
     SVMI_OPT_OP_COST = 6,     /* fusion cost model: per-op cost in FMA per amplitude (default 2;
                                  0 for SVMI_OPT_SPECIALIZE unless set)                      */
     SVMI_OPT_COEF_BUDGET = 7, /* split a forward sweep whose op records and coefficients exceed
@@ -112,10 +114,10 @@ typedef enum svmi_option {
                                  per circuit); 0 = interpret the sweep programs (default)     */
     SVMI_OPT_MERGE_QUBITS = 9, /* widest dense block (1..4 register qubits) that fusion may
                                  form from a run of gates inside one phase (default 2)       */
-    SVMI_OPT_PREFETCH = 10,   /* 1 = one-state sweeps of 12-qubit tiles over large states run
-                                 persistent with two LDS tile buffers, the next tile streaming
-                                 in by LDS DMA during the current one's phases (one workgroup
-                                 per CU); 0 = one workgroup per tile, two per CU (default)   */
+    SVMI_OPT_PREFETCH = 10,   /* 1 = with SVMI_OPT_SPECIALIZE, compiled sweeps of 12-qubit tiles
+                                 over large states run persistent with two LDS tile buffers, the
+                                 next tile streaming in by LDS DMA during the current one's
+                                 phases; no effect on interpreted sweeps                      */
     SVMI_OPT_TILE_MAP = 11    /* 1 = CX and SWAP gates on two tile qubits that a phase does not
                                  hold in registers relabel the tile's LDS indices instead of
                                  needing a phase (default; not with SVMI_OPT_SPECIALIZE);

@@ -30,7 +30,7 @@ HIP_FLAGS = [
     "-mllvm", "-structurizecfg-skip-uniform-regions=true",
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
-ENGINE_SOURCES = ["svmi_api.hip", "svmi_kernels.hip", "svmi_lower.cpp", "svmi_plan.cpp", "svmi_pauli.cpp", "svmi_qir.cpp",
+ENGINE_SOURCES = ["svmi_api.hip", "svmi_kernels.hip", "svmi_lower.cpp", "svmi_plan.cpp", "svmi_layout.cpp", "svmi_pauli.cpp", "svmi_qir.cpp",
                   "svmi_qasm.cpp", "svmi_jit.cpp", "svmi_calib.hip"]
 # engine headers compiled into the library for the specialised sweep kernels
 # built at run time (svmi_jit.cpp)

@@ -50,42 +50,59 @@ bool gf2_insert(uint32_t (&basis)[32], uint32_t v)
     return false;
 }
 
-bool gf2_in_span(const uint32_t (&basis)[32], uint32_t v)
+// A sweep's register layouts address the tile as bijections: in every exchange
+// the (thread, register) columns of the writes and of the reads are
+// independent and below the exchange area's size, and the loads and stores
+// reach every tile qubit and no other.
+bool layout_valid(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, const uint64_t* lane_tab,
+                  const uint64_t* wave_tab, bool two)
 {
-    for (int b = 31; b >= 0 && v; b--)
-        if ((v >> b) & 1u) {
-            if (!basis[b]) return false;
-            v ^= basis[b];
-        }
-    return v == 0;
-}
-
-// A phase's LDS addressing stays inside its tile and is a bijection there:
-// the tile map's columns (scol at the tile register bits, gm at the group
-// bits) are independent and below 2^k, the gather columns span the same
-// register columns, gxor and sxor lie in that span, and a two-state phase's
-// state column is 2^k.
-bool phase_map_valid(const PhaseInfo& ph, uint32_t k, bool two)
-{
-    const int rb = two ? kRegBitsAdj : kRegBits;
-    if (k < uint32_t(rb) || k - rb > 10) return false;
-    const uint32_t lim = 1u << k;
-    uint32_t all[32] = {}, reg[32] = {}, gat[32] = {};
-    for (int s = 0; s < rb; s++) {
-        if (ph.scol[s] >= lim || !gf2_insert(all, ph.scol[s])) return false;
-        gf2_insert(reg, ph.scol[s]);
-    }
-    for (int i = 0; i < 10; i++) {
-        if (uint32_t(i) >= k - rb) {
-            if (ph.gm[i]) return false;
-        } else if (ph.gm[i] >= lim || !gf2_insert(all, ph.gm[i])) {
+    const uint32_t K = sw.k + (two ? 1u : 0u), t = K - kRegBits;
+    const uint32_t tl = std::min<uint32_t>(t, kLaneBits), tw = t - tl;
+    if (tw > uint32_t(kMaxWaveBits)) return false;
+    for (int side = 0; side < 2; side++) {
+        uint64_t basis[64] = {}, all = 0;
+        uint32_t rank = 0;
+        const auto add = [&](uint64_t v) {
+            all |= v;
+            for (int b = 63; b >= 0 && v; b--)
+                if ((v >> b) & 1) {
+                    if (!basis[b]) {
+                        basis[b] = v;
+                        rank++;
+                        return;
+                    }
+                    v ^= basis[b];
+                }
+        };
+        for (uint32_t i = 0; i < tl; i++) add(io.lane[side][i]);
+        for (uint32_t i = 0; i < tw; i++) add(io.wave[side][1u << i] ^ io.wave[side][0]);
+        for (int s = 0; s < (two ? kRegBitsAdj : kRegBits); s++) add(io.reg[side][1u << s]);
+        for (uint32_t v = 0; v < (1u << tw); v++) all |= io.wave[side][v];
+        for (int r = 0; r < (two ? kRegsAdj : kRegs); r++) all |= io.reg[side][r];
+        if (rank != sw.k || (all & 15) || ((all >> 4) & sw.extmask) ||
+            ((all >> 4) >> (sw.k + __builtin_popcountll(sw.extmask))))
             return false;
-        }
     }
-    for (int s = 0; s < rb; s++)
-        if (!gf2_in_span(reg, ph.gcol[s]) || !gf2_insert(gat, ph.gcol[s])) return false;
-    if (two && (ph.scol[kRegBits - 1] != lim || ph.gcol[kRegBits - 1] != lim)) return false;
-    return gf2_in_span(reg, ph.gxor) && gf2_in_span(reg, ph.sxor);
+    for (uint32_t p = io.ph_begin + 1; p < io.ph_end; p++) {
+        const uint64_t* lt = lane_tab + size_t(p) * kLaneEntries;
+        const uint64_t* wt = wave_tab + size_t(p) * kWaveEntries;
+        for (int rd = 0; rd < 2; rd++) {
+            uint32_t basis[32] = {};
+            const auto ok = [&](uint32_t v) { return !(v & 7u) && v < (8u << K) && gf2_insert(basis, v); };
+            for (uint32_t i = 0; i < tl; i++)
+                if (!ok(uint32_t(lt[1u << i] >> (16 * rd)) & 0xffffu)) return false;
+            for (uint32_t i = 0; i < tw; i++)
+                if (!ok(uint32_t((wt[1u << i] ^ wt[0]) >> (16 * rd)) & 0xffffu)) return false;
+            const uint32_t* reg = rd ? lph[p].rd : lph[p].w;
+            for (int s = 0; s < kRegBits; s++)
+                if (!ok(reg[1u << s])) return false;
+            for (int r = 0; r < kRegs; r++)
+                if (reg[r] >= (8u << K)) return false;
+        }
+        if ((uint32_t(wt[0]) >> 16) >= (8u << K)) return false;
+    }
+    return true;
 }
 
 #define SVMI_HIP(x)                                                                          \
@@ -157,42 +174,47 @@ struct DevBuf {
     T* as() const { return static_cast<T*>(p); }
 };
 
+// A program's tables in one device buffer, filled by one copy.
 struct DeviceProgram {
-    DevBuf phases, ops, coef, hitab;
+    DevBuf buf;
+    std::vector<unsigned char> host;   // the copy's source, until the upload's synchronisation
+    size_t o_ops = 0, o_coef = 0, o_lph = 0, o_lane = 0, o_wave = 0, o_io = 0, o_hitab = 0;
     template <class T>
-    static svmi_status put(DevBuf& b, const std::vector<T>& v, hipStream_t st)
+    size_t put(const std::vector<T>& v, size_t pad = 0)
     {
-        const size_t bytes = std::max<size_t>(v.size() * sizeof(T), 16);
-        SVMI_TRY(b.ensure(bytes));
-        if (!v.empty()) SVMI_HIP(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st));
-        return SVMI_OK;
+        const size_t at = (host.size() + 255) & ~size_t(255);
+        host.resize(at + v.size() * sizeof(T) + pad, 0);
+        if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
+        return at;
     }
-    // op arrays end with one NOP record: the sweep kernels read the header
-    // after each phase's last op
-    static svmi_status put_ops(DevBuf& b, const std::vector<DOp>& v, hipStream_t st)
+    // hitab: the tile-row tables, which only compiled sweeps read
+    svmi_status upload(const Program& p, hipStream_t st, bool hitab = false)
     {
-        static const DOp nop = {};
-        SVMI_TRY(b.ensure((v.size() + 1) * sizeof(DOp)));
-        if (!v.empty()) SVMI_HIP(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(DOp), hipMemcpyHostToDevice, st));
-        SVMI_HIP(hipMemcpyAsync(static_cast<DOp*>(b.p) + v.size(), &nop, sizeof(DOp), hipMemcpyHostToDevice, st));
-        return SVMI_OK;
-    }
-    svmi_status upload(const Program& p, hipStream_t st)
-    {
-        SVMI_TRY(put(phases, p.phases, st));
-        SVMI_TRY(put_ops(ops, p.ops, st));
-        SVMI_TRY(put(coef, p.coef, st));
-        SVMI_TRY(put(hitab, p.hitab, st));
+        host.clear();
+        // op arrays end with an unused record: the latency builds read the
+        // header after each phase's last op
+        o_ops = put(p.ops, sizeof(DOp));
+        o_coef = put(p.coef, 16);
+        o_lph = put(p.lphases, 16);
+        o_lane = put(p.lane_tab, 16);
+        o_wave = put(p.wave_tab, 16);
+        o_io = put(p.io, 16);
+        if (hitab) o_hitab = put(p.hitab, 16);
+        SVMI_TRY(buf.ensure(host.size()));
+        SVMI_HIP(hipMemcpyAsync(buf.p, host.data(), host.size(), hipMemcpyHostToDevice, st));
         SVMI_HIP(hipStreamSynchronize(st));
         return SVMI_OK;
     }
-    void release()
+    template <class T>
+    T* at(size_t off) const { return reinterpret_cast<T*>(static_cast<unsigned char*>(buf.p) + off); }
+    c64* coef() const { return at<c64>(o_coef); }
+    const SweepIO* io() const { return at<SweepIO>(o_io); }
+    uint64_t* hitab() const { return at<uint64_t>(o_hitab); }
+    SweepTables tables() const
     {
-        phases.release();
-        ops.release();
-        coef.release();
-        hitab.release();
+        return SweepTables{at<LayoutPhase>(o_lph), at<uint64_t>(o_lane), at<uint64_t>(o_wave), at<DOp>(o_ops), coef()};
     }
+    void release() { buf.release(); }
 };
 
 svmi_status check_gates(const svmi_gate* gates, size_t n_gates, int n)
@@ -331,10 +353,11 @@ void adjoint_entries(const svmi_gate* gates, size_t n_gates, const int32_t* para
 struct BatchPlan {
     std::vector<Program> fwd, adj;
     std::vector<SweepInfo> sweeps;
-    std::vector<PhaseInfo> phases;
+    std::vector<SweepIO> io;
+    std::vector<LayoutPhase> lphases;
+    std::vector<uint64_t> lane_tab, wave_tab;
     std::vector<DOp> ops;
     std::vector<c64> coef;
-    std::vector<uint64_t> hitab;
     std::vector<PauliGroup> groups;
     std::vector<PauliTerm> terms;
     std::vector<BatchCircuit> circs;     // phi/lam unset; state_off gives the layout
@@ -379,8 +402,7 @@ svmi_status verify_batch(const BatchPlan& bp)
             if (b.kind != L.kind || (sweep && bp.sweeps[b.sweep].k != L.k) || b.init_zero != L.init ||
                 (b.kind == BSTEP_ADJ && bp.sweeps[b.sweep].n_grad > L.max_grad) ||
                 (sweep && bp.sweeps[b.sweep].n_xf > L.max_xf) ||
-                (sweep && bp.sweeps[b.sweep].max_dense > L.max_dense) ||
-                (b.kind == BSTEP_FWD && bp.sweeps[b.sweep].mapped && !L.mapped))
+                (sweep && bp.sweeps[b.sweep].max_dense > L.max_dense))
                 return fail(SVMI_ERR_STATE, "batch plan: mixed launch");
             nt += b.n_tasks;
         }
@@ -400,47 +422,32 @@ svmi_status verify_batch(const BatchPlan& bp)
         if (b.kind == BSTEP_FWD || b.kind == BSTEP_ADJ) {
             if (b.sweep >= bp.sweeps.size()) return fail(SVMI_ERR_STATE, "batch plan: bad sweep index");
             const SweepInfo& sw = bp.sweeps[b.sweep];
-            if (sw.n_tiles != b.n_tasks || sw.k > uint32_t(b.kind == BSTEP_ADJ ? kMaxTileQubitsAdj : kMaxTileQubits) ||
-                sw.k < uint32_t(kRegBits) || sw.phase_end > bp.phases.size() || sw.phase_begin > sw.phase_end ||
-                sw.hitab + (1ull << (sw.k - sw.c)) > bp.hitab.size() || sw.n_grad > uint32_t(kMaxGradsPerSweep))
+            const SweepIO& io = bp.io[b.sweep];
+            const bool two = b.kind == BSTEP_ADJ;
+            if (sw.n_tiles != b.n_tasks || sw.k > uint32_t(two ? kMaxTileQubitsAdj : kMaxTileQubits) ||
+                sw.k < uint32_t(kRegBits) || io.ph_begin >= io.ph_end || io.ph_end > bp.lphases.size() ||
+                sw.n_grad > uint32_t(kMaxGradsPerSweep))
                 return fail(SVMI_ERR_STATE, "batch plan: bad sweep");
             if ((sw.k + uint32_t(__builtin_popcountll(sw.extmask))) != bp.circs[b.circuit].n)
                 return fail(SVMI_ERR_STATE, "batch plan: sweep does not match the circuit size");
-            if (b.kind == BSTEP_ADJ && b.partial + sw.n_tiles * sw.n_grad > bp.n_grad_partials)
+            if (two && b.partial + sw.n_tiles * sw.n_grad > bp.n_grad_partials)
                 return fail(SVMI_ERR_STATE, "batch plan: bad gradient partial range");
             if (sw.op_begin > sw.op_end || sw.op_end > bp.ops.size() || sw.n_xf > uint32_t(kMaxXfSlots) ||
                 16u * sw.n_lt > sw.n_xf || sw.lt_coef + 16ull * sw.n_lt > bp.coef.size())
                 return fail(SVMI_ERR_STATE, "batch plan: bad sweep op range");
-            if (sw.mapped) {   // the store's tile map: a bijection of the tile
-                uint32_t basis[32] = {};
-                bool ok = true;
-                for (uint32_t i = 0; i < 14 && ok; i++)
-                    ok = i < sw.k ? (sw.fcol[i] < (1u << sw.k) && gf2_insert(basis, sw.fcol[i])) : sw.fcol[i] == 0;
-                const uint32_t rb = uint32_t(b.kind == BSTEP_ADJ ? kRegBitsAdj : kRegBits);
-                for (uint32_t j = 0; j < 16 && ok; j++)
-                    ok = j < (1u << rb) ? sw.fj[j] == sweep_map(sw, j << (sw.k - rb)) : sw.fj[j] == 0;
-                if (!ok) return fail(SVMI_ERR_STATE, "batch plan: bad tile map");
-            }
             for (uint32_t o = sw.op_begin; o < sw.op_end; o++)
                 if ((has_tile_factor(bp.ops[o].h) && bp.ops[o].h.grad >= sw.n_xf) ||
                     (bp.ops[o].h.type == DOP_PHASETAB && bp.ops[o].h.gmask != kLaneTabGlobal &&
                      uint64_t(bp.ops[o].h.gmask) + 16ull * bp.ops[o].h.s0 > sw.n_xf))
                     return fail(SVMI_ERR_STATE, "batch plan: bad phase factor slot");
-            for (uint32_t p = sw.phase_begin; p < sw.phase_end; p++) {
-                const PhaseInfo& ph = bp.phases[p];
-                if (ph.op_end > bp.ops.size() || ph.op_begin > ph.op_end || ph.op_begin < sw.op_begin ||
-                    ph.op_end > sw.op_end)
+            if (!layout_valid(sw, io, bp.lphases.data(), bp.lane_tab.data(), bp.wave_tab.data(), two))
+                return fail(SVMI_ERR_STATE, "batch plan: bad register layout");
+            for (uint32_t p = io.ph_begin; p < io.ph_end; p++) {
+                const LayoutPhase& L = bp.lphases[p];
+                if (L.op_begin > L.op_end ||
+                    (L.op_begin < L.op_end && (L.op_begin < sw.op_begin || L.op_end > sw.op_end)))
                     return fail(SVMI_ERR_STATE, "batch plan: bad phase");
-                // adjoint phases: 3 tile bits, then k (lambda's half of the LDS)
-                const bool two = b.kind == BSTEP_ADJ;
-                for (int r = 0; r < kRegBits; r++) {
-                    const bool state_bit = two && r == kRegBits - 1;
-                    if (state_bit ? ph.r[r] != sw.k : ph.r[r] >= sw.k)
-                        return fail(SVMI_ERR_STATE, "batch plan: bad register bit");
-                }
-                if (!phase_map_valid(ph, sw.k, two) || (ph.mapped && !sw.mapped))
-                    return fail(SVMI_ERR_STATE, "batch plan: bad gather map");
-                for (uint32_t o = ph.op_begin; o < ph.op_end; o++)
+                for (uint32_t o = L.op_begin; o < L.op_end; o++)
                     if (bp.ops[o].h.coef > bp.coef.size()) return fail(SVMI_ERR_STATE, "batch plan: bad coef offset");
             }
         } else if (b.kind == BSTEP_PAULI) {
@@ -470,7 +477,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
         if (it.n_qubits < 1 || it.n_qubits > 30)
             return fail(SVMI_ERR_ARG, "batch item " + std::to_string(i) + ": n_qubits must be in [1, 30]");
         if ((it.fwd_tile && (it.fwd_tile < kRegBits || it.fwd_tile > kMaxTileQubits)) ||
-            (it.adj_tile && (it.adj_tile < kRegBits || it.adj_tile > kMaxTileQubitsAdj)) || it.op_cost > 33)
+            (it.adj_tile && (it.adj_tile < kRegBits || it.adj_tile > kMaxBatchAdjTile)) || it.op_cost > 33)
             return fail(SVMI_ERR_ARG, "batch item " + std::to_string(i) + ": fwd_tile must be in [4, 13], adj_tile in "
                                                                              "[4, 11], op_cost + 1 in [1, 33]");
         SVMI_TRY(check_gates(it.gates, it.n_gates, it.n_qubits));
@@ -496,12 +503,15 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 PlanOptions of;
                 of.tile_qubits = it.fwd_tile ? it.fwd_tile : tu.fwd_tile;
                 of.op_overhead = it.op_cost ? it.op_cost - 1 : tu.op_cost;
+                if (ni[i] >= 18) of.low_qubits = 3;   // as default_tile
                 plan_forward(it.gates, it.n_gates, ni[i], of, bp.fwd[i]);
                 std::vector<AdjEntry> entries;
                 adjoint_entries(it.gates, it.n_gates, it.param_slots, entries);
                 PlanOptions oa;
-                oa.tile_qubits = it.adj_tile ? it.adj_tile : tu.adj_tile;
+                // (16 circuits of 20-22 qubits with backward tiles of 11 / 12: 15.1 / 14.5 ms)
+                oa.tile_qubits = it.adj_tile ? it.adj_tile : ni[i] >= 18 ? kMaxTileQubitsAdj : tu.adj_tile;
                 oa.op_overhead = of.op_overhead;
+                oa.low_qubits = of.low_qubits;
                 build_adjoint_program(entries, ni[i], oa, bp.adj[i]);
                 plan_pauli(it.terms, it.n_terms, ni[i], kPauliTileQubits, true, 1, pauli[i]);
             }
@@ -521,29 +531,33 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                                     "for the 4 low qubits plus the op's qubits)");
     auto append_program = [&](const Program& pr) {
         const uint32_t op_base = uint32_t(bp.ops.size()), coef_base = uint32_t(bp.coef.size());
-        const uint32_t ph_base = uint32_t(bp.phases.size()), ht_base = uint32_t(bp.hitab.size());
+        const uint32_t lp_base = uint32_t(bp.lphases.size());
         const uint32_t sw_base = uint32_t(bp.sweeps.size());
         for (DOp d : pr.ops) {
             d.h.coef += coef_base;
             if (d.h.type == DOP_ROT && d.h.s0) d.h.grad += coef_base;   // its table
             bp.ops.push_back(d);
         }
-        for (PhaseInfo ph : pr.phases) {
-            ph.op_begin += op_base;
-            ph.op_end += op_base;
-            bp.phases.push_back(ph);
+        for (LayoutPhase L : pr.lphases) {
+            L.op_begin += op_base;
+            L.op_end += op_base;
+            L.coef_begin += coef_base;
+            bp.lphases.push_back(L);
+        }
+        for (SweepIO io : pr.io) {
+            io.ph_begin += lp_base;
+            io.ph_end += lp_base;
+            bp.io.push_back(io);
         }
         for (SweepInfo sw : pr.sweeps) {
-            sw.phase_begin += ph_base;
-            sw.phase_end += ph_base;
             sw.op_begin += op_base;
             sw.op_end += op_base;
-            sw.hitab += ht_base;
             sw.lt_coef += coef_base;
             bp.sweeps.push_back(sw);
         }
         bp.coef.insert(bp.coef.end(), pr.coef.begin(), pr.coef.end());
-        bp.hitab.insert(bp.hitab.end(), pr.hitab.begin(), pr.hitab.end());
+        bp.lane_tab.insert(bp.lane_tab.end(), pr.lane_tab.begin(), pr.lane_tab.end());
+        bp.wave_tab.insert(bp.wave_tab.end(), pr.wave_tab.begin(), pr.wave_tab.end());
         return sw_base;
     };
     bp.circs.resize(n_items);
@@ -654,7 +668,6 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
             const uint32_t ng = b.kind == BSTEP_ADJ ? bp.sweeps[b.sweep].n_grad : 0u;
             const uint32_t nx = (b.kind == BSTEP_FWD || b.kind == BSTEP_ADJ) ? bp.sweeps[b.sweep].n_xf : 0u;
             const uint32_t md = (b.kind == BSTEP_FWD || b.kind == BSTEP_ADJ) ? bp.sweeps[b.sweep].max_dense : 0u;
-            const uint32_t mp = b.kind == BSTEP_FWD ? bp.sweeps[b.sweep].mapped : 0u;
             if (!bp.launches.empty() && bp.launches.back().step_end == idx &&
                 bp.launches.back().step_begin >= bp.level_begin.back() && bp.launches.back().kind == b.kind &&
                 bp.launches.back().k == k && bp.launches.back().init == b.init_zero) {
@@ -664,7 +677,6 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 L.max_grad = std::max(L.max_grad, ng);
                 L.max_xf = std::max(L.max_xf, nx);
                 L.max_dense = std::max(L.max_dense, md);
-                L.mapped |= mp;
             } else {
                 BatchLaunch L;
                 std::memset(&L, 0, sizeof(L));
@@ -675,7 +687,6 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 L.max_grad = ng;
                 L.max_xf = nx;
                 L.max_dense = md;
-                L.mapped = mp;
                 L.init = b.init_zero;
                 L.task_begin = b.task_begin;
                 L.n_tasks = b.n_tasks;
@@ -718,11 +729,12 @@ struct svmi_sim {
     DeviceProgram dprog;
     JitSweeps jit;             // specialised kernels of prog's sweeps (SVMI_OPT_SPECIALIZE)
     bool specialize = false;
+    bool tile_set = false;     // SVMI_OPT_TILE_QUBITS given (else default_tile)
+    bool low_set = false;      // SVMI_OPT_LOW_QUBITS given
     bool op_cost_set = false;  // SVMI_OPT_OP_COST given (else specialised sweeps plan with op cost 0)
     std::string jit_error;     // why the last specialisation failed (the sweeps then interpret)
     PlanOptions opt;
     bool profile = false;
-    int pipeline = 0;
     bool prefetch = false;     // SVMI_OPT_PREFETCH
     std::vector<hipEvent_t> prof_events;
     std::vector<double> step_ms;   // with profiling: per-step times of the last program run
@@ -808,22 +820,20 @@ svmi_status exec_program(svmi_handle h, const Program& prog, DeviceProgram& dp, 
                 partials = h->scratch[5].as<double>();
             }
             if (jit && st.index < jit->fn.size() && jit->fn[st.index])
-                SVMI_HIP(jit_launch(h->stream, *jit, st.index, sw, s0, dp.coef.as<c64>(), dp.hitab.as<uint64_t>()));
+                SVMI_HIP(jit_launch(h->stream, *jit, st.index, sw, s0, dp.coef(), dp.hitab()));
             else
-                SVMI_HIP(launch_sweep(h->stream, prog.n_states, s0, s1, sw, dp.phases.as<PhaseInfo>(),
-                                      dp.ops.as<DOp>(), dp.coef.as<c64>(), dp.hitab.as<uint64_t>(), partials,
-                                      h->pipeline, h->prefetch));
+                SVMI_HIP(launch_sweep(h->stream, prog.n_states, s0, s1, sw, dp.io() + st.index, dp.tables(), partials));
             if (partials && !combined)
                 SVMI_HIP(launch_sum_rows(h->stream, partials, sw.n_grad, sw.n_tiles, grad_sums + sw.grad_base));
         } else if (st.kind == Step::MEASURE) {
             const MeasureStep& m = prog.measures[st.index];
             SVMI_TRY(h->scratch[4].ensure(measure_partials(int(m.n)) * sizeof(double)));
             SVMI_HIP(launch_measure(h->stream, s0, int(m.n), m.qubit, m.draw, h->scratch[4].as<double>(),
-                                    dp.coef.as<c64>() + m.coef, meas + st.index, int(m.dm_n)));
+                                    dp.coef() + m.coef, meas + st.index, int(m.dm_n)));
         } else {
             const StandaloneOp& so = prog.standalone[st.index];
-            SVMI_HIP(launch_standalone(h->stream, s0, h->n_int, so, dp.coef.as<c64>()));
-            if (prog.n_states == 2) SVMI_HIP(launch_standalone(h->stream, s1, h->n_int, so, dp.coef.as<c64>()));
+            SVMI_HIP(launch_standalone(h->stream, s0, h->n_int, so, dp.coef()));
+            if (prog.n_states == 2) SVMI_HIP(launch_standalone(h->stream, s1, h->n_int, so, dp.coef()));
         }
         if (prof) SVMI_HIP(hipEventRecord(h->prof_events[2 * si + 1], h->stream));
         h->stats.kernel_launches++;
@@ -1078,6 +1088,20 @@ svmi_status svmi_get_amplitudes(svmi_handle h, const uint64_t* idx, size_t count
     return SVMI_OK;
 }
 
+// Default tile and low qubits.  Tiles of 13 qubits (two states: 12) from 20
+// qubits on, where a state has at least 128 of them; on smaller states the
+// tiles of 12 (11) keep more CUs busy.  The large tiles keep 3 low qubits
+// (128-byte segments), which leaves one more for the circuit: at the copy
+// rate of 256-byte segments still, and fewer sweeps.  12 and 4 / 13 and 4 /
+// 13 and 3: u3 brick wall at 30 qubits 180 / 167 / 164 ms, QFT at 31 87.6 /
+// 93.6 / 81.8 ms, 20 random layers at 28 75.8 / 64.0 / 65.8 ms, at 18 361 /
+// 395 us.
+void default_tile(svmi_handle h, int n, bool two, PlanOptions& o)
+{
+    if (!h->tile_set) o.tile_qubits = n >= 20 ? (two ? 12 : 13) : (two ? 11 : 12);
+    if (!h->low_set && !h->tile_set && n >= 20) o.low_qubits = 3;
+}
+
 // Planner options of the forward program.  Specialised sweeps pay almost
 // nothing per op (no dispatch), so unless the caller set an op cost their
 // fusion model counts FMAs only: 20-layer u3 brick-wall at 30 qubits 300 ->
@@ -1085,6 +1109,7 @@ svmi_status svmi_get_amplitudes(svmi_handle h, const uint64_t* idx, size_t count
 PlanOptions forward_options(svmi_handle h)
 {
     PlanOptions o = h->opt;
+    if (!h->specialize) default_tile(h, h->n_int, false, o);
     if (h->specialize && !h->op_cost_set) o.op_overhead = 0;
     if (h->specialize) o.tile_map = false;   // the compiled sweeps address LDS without maps
     return o;
@@ -1093,7 +1118,8 @@ PlanOptions forward_options(svmi_handle h)
 // Device copy of h->prog and, with SVMI_OPT_SPECIALIZE, its compiled sweeps.
 svmi_status install_program(svmi_handle h)
 {
-    SVMI_TRY(h->dprog.upload(h->prog, h->stream));
+    if (h->specialize) build_row_tables(h->prog);
+    SVMI_TRY(h->dprog.upload(h->prog, h->stream, h->specialize));
     h->jit.release();
     h->jit_error.clear();
     h->stats.specialized_sweeps = 0;
@@ -1190,7 +1216,9 @@ svmi_status qir_run(svmi_handle h, int n_qubits, const svmi_qir_gate* gates, siz
         return fail(SVMI_ERR_ARG, dm ? "density matrix of n_qubits needs a handle of 2 * n_qubits qubits (has " +
                                            std::to_string(h->n) + ")"
                                      : "n_qubits must be in [1, " + std::to_string(h->n) + "] (the handle's qubits)");
-    SVMI_TRY(plan_qir(gates, n_gates, n_qubits, std::max(n_state, kRegBits), h->opt, h->qir_prog, dm));
+    PlanOptions opt = h->opt;
+    default_tile(h, n_state, false, opt);
+    SVMI_TRY(plan_qir(gates, n_gates, n_qubits, std::max(n_state, kRegBits), opt, h->qir_prog, dm));
     const Program& prog = h->qir_prog;
     SVMI_TRY(h->qir_dprog.upload(prog, h->stream));
     const size_t nm = prog.measures.size();
@@ -1390,7 +1418,9 @@ svmi_status svmi_adjoint(svmi_handle h, const svmi_pauli_term* terms, size_t n_t
         std::vector<AdjEntry> entries;
         adjoint_entries(h->gates.data(), h->gates.size(), param_slots, entries);
         h->adj_prog = Program();
-        build_adjoint_program(entries, h->n_int, h->opt, h->adj_prog);
+        PlanOptions o = h->opt;
+        default_tile(h, h->n_int, true, o);
+        build_adjoint_program(entries, h->n_int, o, h->adj_prog);
         SVMI_TRY(h->adj_dprog.upload(h->adj_prog, h->stream));
         SVMI_TRY(h->adj_gsum.ensure(std::max<size_t>(h->adj_prog.n_grad, 1) * sizeof(double)));
         h->adj_slots.assign(param_slots, param_slots + n_slots);
@@ -1471,11 +1501,11 @@ svmi_status svmi_batch_adjoint(int device, const svmi_batch_item* items, size_t 
         std::vector<size_t> idx;                  // original item indices
         std::vector<svmi_batch_item> items;
         BatchPlan bp;
-        DevBuf dsteps, dcircs, dsweeps, dphases, dops, dcoef, dhitab, dgroups, dterms, dpart, dsegs, dout;
+        DevBuf dsteps, dcircs, dsweeps, dio, dlph, dlane, dwave, dops, dcoef, dgroups, dterms, dpart, dsegs, dout;
         void release()
         {
-            for (DevBuf* b : {&dsteps, &dcircs, &dsweeps, &dphases, &dops, &dcoef, &dhitab, &dgroups, &dterms, &dpart,
-                              &dsegs, &dout})
+            for (DevBuf* b : {&dsteps, &dcircs, &dsweeps, &dio, &dlph, &dlane, &dwave, &dops, &dcoef, &dgroups, &dterms,
+                              &dpart, &dsegs, &dout})
                 b->release();
         }
     };
@@ -1511,11 +1541,12 @@ svmi_status svmi_batch_adjoint(int device, const svmi_batch_item* items, size_t 
         SVMI_TRY(put(k.dsteps, bp.steps.data(), bp.steps.size() * sizeof(BatchStep)));
         SVMI_TRY(put(k.dcircs, circs.data(), circs.size() * sizeof(BatchCircuit)));
         SVMI_TRY(put(k.dsweeps, bp.sweeps.data(), bp.sweeps.size() * sizeof(SweepInfo)));
-        SVMI_TRY(put(k.dphases, bp.phases.data(), bp.phases.size() * sizeof(PhaseInfo)));
-        bp.ops.push_back(DOp{});   // a NOP past the end: the kernels read one header ahead
+        SVMI_TRY(put(k.dio, bp.io.data(), bp.io.size() * sizeof(SweepIO)));
+        SVMI_TRY(put(k.dlph, bp.lphases.data(), bp.lphases.size() * sizeof(LayoutPhase)));
+        SVMI_TRY(put(k.dlane, bp.lane_tab.data(), bp.lane_tab.size() * sizeof(uint64_t)));
+        SVMI_TRY(put(k.dwave, bp.wave_tab.data(), bp.wave_tab.size() * sizeof(uint64_t)));
         SVMI_TRY(put(k.dops, bp.ops.data(), bp.ops.size() * sizeof(DOp)));
         SVMI_TRY(put(k.dcoef, bp.coef.data(), bp.coef.size() * sizeof(c64)));
-        SVMI_TRY(put(k.dhitab, bp.hitab.data(), bp.hitab.size() * sizeof(uint64_t)));
         SVMI_TRY(put(k.dgroups, bp.groups.data(), bp.groups.size() * sizeof(PauliGroup)));
         SVMI_TRY(put(k.dterms, bp.terms.data(), bp.terms.size() * sizeof(PauliTerm)));
         SVMI_TRY(k.dpart.ensure(std::max<size_t>((bp.n_grad_partials + bp.n_e_partials) * sizeof(double), 16)));
@@ -1525,10 +1556,9 @@ svmi_status svmi_batch_adjoint(int device, const svmi_batch_item* items, size_t 
         a.steps = k.dsteps.as<BatchStep>();
         a.circuits = k.dcircs.as<BatchCircuit>();
         a.sweeps = k.dsweeps.as<SweepInfo>();
-        a.phases = k.dphases.as<PhaseInfo>();
-        a.ops = k.dops.as<DOp>();
-        a.coef = k.dcoef.as<c64>();
-        a.hitab = k.dhitab.as<uint64_t>();
+        a.io = k.dio.as<SweepIO>();
+        a.t = SweepTables{k.dlph.as<LayoutPhase>(), k.dlane.as<uint64_t>(), k.dwave.as<uint64_t>(), k.dops.as<DOp>(),
+                          k.dcoef.as<c64>()};
         a.groups = k.dgroups.as<PauliGroup>();
         a.terms = k.dterms.as<PauliTerm>();
         a.grad_partials = k.dpart.as<double>();
@@ -1593,10 +1623,12 @@ svmi_status svmi_set_option(svmi_handle h, int option, int64_t value)
     case SVMI_OPT_TILE_QUBITS:
         if (value < kRegBits || value > kMaxTileQubits) return fail(SVMI_ERR_ARG, "tile qubits must be in [4, 13]");
         h->opt.tile_qubits = int(value);
+        h->tile_set = true;
         break;
     case SVMI_OPT_LOW_QUBITS:
         if (value < 0 || value > 8) return fail(SVMI_ERR_ARG, "low qubits must be in [0, 8]");
         h->opt.low_qubits = int(value);
+        h->low_set = true;
         break;
     case SVMI_OPT_SWEEP_FLOPS:
         if (value < 0) return fail(SVMI_ERR_ARG, "sweep budget must be >= 0");
@@ -1614,7 +1646,6 @@ svmi_status svmi_set_option(svmi_handle h, int option, int64_t value)
     case SVMI_OPT_PROFILE: h->profile = value != 0; return SVMI_OK;
     case SVMI_OPT_PIPELINE:
         if (value < 0 || value > 64) return fail(SVMI_ERR_ARG, "pipeline must be in [0, 64]");
-        h->pipeline = int(value);
         return SVMI_OK;
     case SVMI_OPT_PREFETCH: h->prefetch = value != 0; return SVMI_OK;
     case SVMI_OPT_SPECIALIZE: h->specialize = value != 0; break;
@@ -1695,18 +1726,16 @@ void host_standalone(std::vector<c64>& s, int n, const StandaloneOp& so, const s
     }
 }
 
-// One tile of one sweep on the host (the kernels' sweep_tile without LDS).
-// gsum_tile receives the tile's gradient accumulators (ns == 2).
-void host_tile(const SweepInfo& sw, const PhaseInfo* phases, const DOp* ops, const c64* coef, const uint64_t* hitab,
-               int ns, c64* s0, c64* s1, uint64_t tile, bool init_zero, double* gsum_tile)
+// One tile of one sweep on the host, as the kernels' sweep_tile runs it: every
+// thread's register group, and exchanges through an array of slots (a slot
+// holds the real parts, then the imaginary ones).  An exchange without
+// LPH_CROSS that reads another wave's slot, a slot written twice or never
+// throws.  gsum_tile receives the tile's gradient accumulators (ns == 2).
+void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, const uint64_t* lane_tab,
+               const uint64_t* wave_tab, const DOp* ops, const c64* coef, int ns, c64* s0, c64* s1, uint64_t tile,
+               bool init_zero, double* gsum_tile)
 {
-    // as the kernels: one LDS-like array, lambda's half at [2^k, 2^(k+1));
-    // a group is 16 amplitudes (two states: 8 of phi then 8 of lambda, the
-    // phase's last register bit being k)
-    const uint32_t tsize = 1u << sw.k, ngroups = sweep_threads(sw.k, ns);
-    const uint32_t cmask = (1u << sw.c) - 1u;
-    std::vector<c64> t(size_t(tsize) * ns);
-    std::vector<uint64_t> gidx(tsize);
+    const uint32_t nt = sweep_threads(sw.k, ns);
     for (uint32_t i = 0; i < sw.n_grad; i++) gsum_tile[i] = 0.0;
     const uint64_t base = tile_base(sw, tile);
     std::vector<c64> xf(std::max<uint32_t>(sw.n_xf, 1));
@@ -1714,44 +1743,85 @@ void host_tile(const SweepInfo& sw, const PhaseInfo* phases, const DOp* ops, con
     for (uint32_t i = 0; i < 16u * sw.n_lt; i++) xf[sw.n_xf - 16u * sw.n_lt + i] = coef[sw.lt_coef + i];
     for (uint32_t o = sw.op_begin; o < sw.op_end; o++)
         if (has_tile_factor(ops[o].h)) xf[ops[o].h.grad] = tile_factor(ops[o].h, coef, base, xbits);
-    for (uint32_t l = 0; l < tsize; l++) {
-        gidx[l] = base | hitab[sw.hitab + (l >> sw.c)] | (l & cmask);
-        t[l] = init_zero ? c64{gidx[l] == 0 ? 1.0 : 0.0, 0.0} : s0[gidx[l]];
-        if (ns == 2) t[tsize + l] = s1[gidx[l]];
-    }
-    // two-state sweeps always address LDS through their tile maps (the
-    // identity where nothing was folded), one-state sweeps when mapped
-    const bool mp = ns == 2 || sw.mapped;
-    for (uint32_t p = sw.phase_begin; p < sw.phase_end; p++) {
-        const PhaseInfo& ph = phases[p];
-        uint32_t off[kRegs], goffs[kRegs];
-        phase_offsets(ph, off);
-        phase_gather_offsets(ph, goffs);
-        uint32_t soffs[kRegs];
-        phase_scatter_offsets(ph, soffs);
-        for (uint32_t g = 0; g < ngroups; g++) {
-            const uint32_t goff = group_offset(ph, g);
-            const uint32_t gphys = mp ? mapped_group_offset(ph, g) : goff;
-            c64 a[kRegs];
-            for (int r = 0; r < kRegs; r++) a[r] = t[gphys ^ goffs[r]];
-            for (uint32_t o = ph.op_begin; o < ph.op_end; o++) {
+    struct Group {
+        c64 a[kRegs];
+    };
+    std::vector<Group> g(nt), h(nt);
+    uint64_t runs = 0;
+    for (uint32_t i = 0; i < io.n_runs; i++) runs |= ((tile << io.run[i].shl) >> io.run[i].shr) & io.run[i].mask;
+    const uint32_t vhi = uint32_t(tile >> io.vhi_shift);
+    if (runs != base || vhi != uint32_t(extract_bits(base, sw.exthi))) throw std::logic_error("layout: tile base");
+    const auto amp = [&](int side, uint32_t t, int r) {
+        uint64_t u = (base << 4) ^ io.wave[side][t >> kLaneBits];
+        for (int i = 0; i < kLaneBits; i++)
+            if ((t >> i) & 1u) u ^= io.lane[side][i];
+        const uint64_t ro = io.reg[side][ns == 2 ? r % kRegsAdj : r];
+        if (((io.additive >> side) & 1u) && (u & ro)) throw std::logic_error("layout: offsets do not add");
+        return (u ^ ro) >> 4;
+    };
+    for (uint32_t t = 0; t < nt; t++)
+        for (int r = 0; r < kRegs; r++) {
+            const uint64_t x = amp(0, t, r);
+            g[t].a[r] = init_zero ? c64{x == 0 ? 1.0 : 0.0, 0.0} : (ns == 2 && r >= kRegsAdj ? s1 : s0)[x];
+        }
+    const uint32_t slots = (1u << sw.k) * uint32_t(ns);
+    std::vector<uint32_t> by(slots);   // writer (thread * 16 + register) of a slot
+    for (uint32_t p = io.ph_begin; p < io.ph_end; p++) {
+        const LayoutPhase& L = lph[p];
+        const auto entry = [&](uint32_t t) {
+            return lane_tab[size_t(p) * kLaneEntries + (t & 63u)] ^ wave_tab[size_t(p) * kWaveEntries + (t >> 6)];
+        };
+        const auto slot = [&](uint32_t b, const uint32_t (&reg)[kRegs], int r) {
+            b ^= reg[r];
+            if ((b & 7u) || (b >> 3) >= slots) throw std::logic_error("layout: slot out of range");
+            return b >> 3;
+        };
+        if (p != io.ph_begin) {
+            std::fill(by.begin(), by.end(), ~0u);
+            for (uint32_t t = 0; t < nt; t++)
+                for (int r = 0; r < kRegs; r++) {
+                    uint32_t& b = by[slot(uint32_t(entry(t)) & 0xffffu, L.w, r)];
+                    if (b != ~0u) throw std::logic_error("layout: slot written twice");
+                    b = t * kRegs + uint32_t(r);
+                }
+            for (uint32_t t = 0; t < nt; t++)
+                for (int r = 0; r < kRegs; r++) {
+                    uint32_t& b = by[slot(uint32_t(entry(t)) >> 16, L.rd, r)];
+                    if (b == ~0u) throw std::logic_error("layout: slot read twice or never written");
+                    if (!(L.flags & LPH_CROSS) && (b / kRegs) >> 6 != t >> 6)
+                        throw std::logic_error("layout: an exchange inside the waves leaves a wave");
+                    h[t].a[r] = g[b / kRegs].a[b % kRegs];
+                    b = ~0u;
+                }
+            g.swap(h);
+        }
+        const RegOffsets off{L.rcol};
+        for (uint32_t t = 0; t < nt; t++) {
+            const uint32_t goff = uint32_t(entry(t) >> 32) & 0xffffu, grp = uint32_t(entry(t) >> 48);
+            for (uint32_t o = L.op_begin; o < L.op_end; o++) {
                 const DOp& op = ops[o];
                 if (op.h.type == DOP_GRAD_DENSE || op.h.type == DOP_GRAD_DIAG)
-                    gsum_tile[op.h.grad] += exec_grad_op<kRegBits, kRegsAdj>(op.h, &op, a, coef, goff, off, base);
+                    gsum_tile[op.h.grad] += exec_grad_op<kRegBits, kRegsAdj>(op.h, &op, g[t].a, coef, goff, off, base);
                 else
-                    exec_state_op(op.h, &op, a, coef, goff, g, off, base, xf.data(), sw.exthi,
-                                  uint32_t(extract_bits(base, sw.exthi)));
+                    exec_state_op(op.h, &op, g[t].a, coef, goff, grp, off, base, xf.data(), sw.exthi, vhi);
             }
-            for (int r = 0; r < kRegs; r++) t[mp ? (gphys ^ soffs[r]) : ((goff | off[r]) ^ ph.sxor)] = a[r];
         }
     }
-    const uint32_t tbits = sw.k - uint32_t(ns == 2 ? kRegBitsAdj : kRegBits);   // log2 of the tile's threads
-    for (uint32_t l = 0; l < tsize; l++) {
-        // as the kernels' store: M(tid) ^ M(nt j) with l = tid + nt j
-        const uint32_t m = sw.mapped ? sweep_map_thread(sw, l & ((1u << tbits) - 1u)) ^ sw.fj[l >> tbits] : l;
-        s0[gidx[l]] = t[m];
-        if (ns == 2) s1[gidx[l]] = t[tsize + m];
+    bool met = io.store_guard != 0;   // the waves met between the loads and the stores
+    for (uint32_t p = io.ph_begin + 1; p < io.ph_end; p++) met = met || (lph[p].flags & LPH_CROSS);
+    if (!met) {
+        std::vector<std::pair<uint64_t, uint32_t>> from, to;   // (amplitude, wave)
+        for (uint32_t t = 0; t < nt; t++)
+            for (int r = 0; r < kRegs; r++) {
+                from.push_back({amp(0, t, r), t >> 6});
+                to.push_back({amp(1, t, r), t >> 6});
+            }
+        std::sort(from.begin(), from.end());
+        std::sort(to.begin(), to.end());
+        if (from != to) throw std::logic_error("layout: a wave stores over another wave's loads");
     }
+    for (uint32_t t = 0; t < nt; t++)
+        for (int r = 0; r < kRegs; r++) (ns == 2 && r >= kRegsAdj ? s1 : s0)[amp(1, t, r)] = g[t].a[r];
 }
 
 // A measurement step on the host: P(1) over the first 2^m.n amplitudes, the
@@ -1798,8 +1868,9 @@ void host_program(Program& prog, std::vector<c64>& s0, std::vector<c64>& s1, std
         const SweepInfo& sw = prog.sweeps[st.index];
         std::vector<double> g(sw.n_grad);
         for (uint64_t tile = 0; tile < sw.n_tiles; tile++) {
-            host_tile(sw, prog.phases.data(), prog.ops.data(), prog.coef.data(), prog.hitab.data(), ns, s0.data(),
-                      ns == 2 ? s1.data() : nullptr, tile, false, g.data());
+            host_tile(sw, prog.io[st.index], prog.lphases.data(), prog.lane_tab.data(), prog.wave_tab.data(),
+                      prog.ops.data(), prog.coef.data(), ns, s0.data(), ns == 2 ? s1.data() : nullptr, tile, false,
+                      g.data());
             for (uint32_t i = 0; i < sw.n_grad; i++) gsum[sw.grad_base + i] += g[i];
         }
     }
@@ -1938,9 +2009,9 @@ svmi_status svmi_debug_emulate_batch(const svmi_batch_item* items, size_t n_item
             if (st.kind == BSTEP_FWD || st.kind == BSTEP_ADJ) {
                 const SweepInfo& sw = bp.sweeps[st.sweep];
                 std::vector<double> g(sw.n_grad);
-                host_tile(sw, bp.phases.data(), bp.ops.data(), bp.coef.data(), bp.hitab.data(),
-                          st.kind == BSTEP_ADJ ? 2 : 1, ph, st.kind == BSTEP_ADJ ? lm : nullptr, task,
-                          L.init != 0, g.data());
+                host_tile(sw, bp.io[st.sweep], bp.lphases.data(), bp.lane_tab.data(), bp.wave_tab.data(),
+                          bp.ops.data(), bp.coef.data(), st.kind == BSTEP_ADJ ? 2 : 1, ph,
+                          st.kind == BSTEP_ADJ ? lm : nullptr, task, L.init != 0, g.data());
                 for (uint32_t i = 0; i < sw.n_grad; i++) g_part[st.partial + i * sw.n_tiles + task] = g[i];
             } else {
                 const uint64_t dim = 1ull << c.n;
@@ -2012,6 +2083,7 @@ svmi_status svmi_debug_jit(int n, const svmi_gate* gates, size_t n_gates, int ti
     PlanOptions o = debug_options(1, tile_qubits, low_qubits, 0);
     o.tile_map = false;   // as SVMI_OPT_SPECIALIZE plans
     plan_forward(gates, n_gates, std::max(n, kRegBits), o, prog);
+    build_row_tables(prog);
     std::vector<char> covered;
     const uint64_t dma_grid = compile == 2 ? 256 : 0;   // double-buffered kernels for a 256-CU device
     const std::string src = jit_source(prog, covered, dma_grid);

@@ -12,8 +12,13 @@ namespace svmi {
 // which would push the whole register group to scratch memory.
 #if defined(__HIP_DEVICE_COMPILE__)
 #define SVMI_FENCE(N) asm volatile("; svmi case %0" ::"i"(N))
+// a per-thread value that an op derives others from: the copy keeps what is
+// derived inside the op's case, or the compiler computes it for every phase
+// (and keeps it in registers) whether such an op comes or not
+#define SVMI_LOCAL(v) asm volatile("" : "+v"(v))
 #else
 #define SVMI_FENCE(N) ((void)0)
+#define SVMI_LOCAL(v) ((void)0)
 #endif
 #define SVMI_CASE_ID(LABEL, ID, STMT) \
     case LABEL:                         \
@@ -135,7 +140,7 @@ SVMI_HD inline void dispatch_cdense(const DOpHdr& h, c64 (&a)[N], const c64* __r
 {
     if ((base & h.emask) != h.emask) return;
     if ((goff & h.gmask) != h.gmask) return;
-    const c64* M = coef + h.coef;
+    const c64* M = coef_at(coef, h.coef);
     switch (h.s0) {
         SVMI_CASE_ID(0, 200, (apply_cdense<0, N>(a, M, h.rsel)))
         SVMI_CASE_ID(1, 201, (apply_cdense<1, N>(a, M, h.rsel)))
@@ -208,17 +213,26 @@ SVMI_HD inline void apply_cphase(const DOpHdr& op, c64 (&a)[N], const c64* __res
     apply_rsel<N>(a, coef[op.coef], op.rsel);
 }
 
-template <int N>
-SVMI_HD inline void apply_diag(const DOp& op, c64 (&a)[N], const c64* __restrict__ coef, uint32_t goff,
-                               const uint32_t (&off)[kRegs], uint64_t base)
+// (off: an array or RegOffsets; table entries in batches of 4, so that the
+// op does not need 64 registers beside the group)
+template <int N, class Off>
+SVMI_HD inline void apply_diag(const DOpHdr& h, const DOp& op, c64 (&a)[N], const c64* __restrict__ coef,
+                               uint32_t goff, const Off& off, uint64_t base)
 {
+    SVMI_LOCAL(goff);
     const uint32_t e = diag_ext_index(op, base);
-    const c64* tab = coef + op.h.coef;
-    c64 f[kRegs];
+    const c64* tab = coef_at(coef, h.coef);
 #pragma unroll
-    for (int r = 0; r < kRegs; r++) f[r] = tab[diag_index(op, goff | off[r], e)];
+    for (int r0 = 0; r0 < kRegs; r0 += 4) {
+        c64 f[4];
 #pragma unroll
-    for (int r = 0; r < N; r++) cmul_to(a[r], f[r & (kRegs - 1)]);
+        for (int r = 0; r < 4; r++) f[r] = tab[diag_index(op, goff | off[r0 + r], e)];
+#pragma unroll
+        for (int h = 0; h < N; h += kRegs)
+#pragma unroll
+            for (int r = 0; r < 4; r++) cmul_to(a[h + r0 + r], f[r]);
+        SVMI_FENCE(500);
+    }
 }
 
 // Apply one non-gradient op to one state's register group.
@@ -229,7 +243,7 @@ template <int N>
 SVMI_HD inline void apply_phaseset(const DOpHdr& h, c64 (&a)[N], const c64* __restrict__ coef, uint32_t goff,
                                    uint64_t base, const c64* xf)
 {
-    const PhaseEntry* pe = reinterpret_cast<const PhaseEntry*>(coef + h.coef);
+    const PhaseEntry* pe = reinterpret_cast<const PhaseEntry*>(coef_at(coef, h.coef));
     double pr = 1.0, pi = 0.0;
     if (h.s1) {   // the tile's product of the entries without lane condition
         const c64 f = xf[h.grad];
@@ -257,6 +271,7 @@ template <int N>
 SVMI_HD inline void apply_phasetab(const DOpHdr& h, c64 (&a)[N], const c64* __restrict__ coef, uint32_t grp,
                                    const c64* xf)
 {
+    SVMI_LOCAL(grp);
     c64 ph = c64{1.0, 0.0};
     if (h.s1) ph = xf[h.grad];
     // two loops, so the LDS tables are read as LDS (a pointer that may be
@@ -327,8 +342,8 @@ SVMI_HD inline c64 tile_factor(const DOpHdr& h, const c64* __restrict__ coef, ui
 template <int N>
 SVMI_HD inline void apply_rot(const DOpHdr& h, c64 (&a)[N], const c64* __restrict__ coef, uint32_t v)
 {
-    if (h.s0) apply_rtab<N>(a, coef + h.grad + 16u * v);
-    const c64* L = coef + h.coef;
+    if (h.s0) apply_rtab<N>(a, coef_at(coef, h.grad + 16u * v));
+    const c64* L = coef_at(coef, h.coef);
     const c64 f0 = L[0], f1 = L[1], f2 = L[2], f3 = L[3];
 #define SVMI_ROT_SLOT(S, F)                                              \
     if ((h.smask >> S) & 1u) {                                           \
@@ -354,10 +369,10 @@ SVMI_HD inline void apply_rot(const DOpHdr& h, c64 (&a)[N], const c64* __restric
 // vmask / vhi: the sweep's variant qubits (SweepInfo::exthi) and the tile
 // base's bits there, so a table over all of them finds its variant with one
 // compare (otherwise the bits of its own mask are extracted).
-template <int kMaxQ = kRegBits, int N = kRegs>
+template <int kMaxQ = kRegBits, int N = kRegs, class Off>
 SVMI_HD inline void exec_state_op(const DOpHdr& h, const DOp* __restrict__ op, c64 (&a)[N],
                                   const c64* __restrict__ coef, uint32_t goff, uint32_t grp,
-                                  const uint32_t (&off)[kRegs], uint64_t base, const c64* xf,
+                                  const Off& off, uint64_t base, const c64* xf,
                                   uint64_t vmask = 0, uint32_t vhi = 0)
 {
     const auto variant = [&](uint64_t emask) {
@@ -379,7 +394,7 @@ SVMI_HD inline void exec_state_op(const DOpHdr& h, const DOp* __restrict__ op, c
     }
     if (h.type == DOP_RTAB) {
         SVMI_FENCE(DOP_RTAB + 100);
-        apply_rtab<N>(a, coef + h.coef + 16u * variant(h.emask));
+        apply_rtab<N>(a, coef_at(coef, h.coef + 16u * variant(h.emask)));
         SVMI_FENCE(DOP_RTAB + 100);
         return;
     }
@@ -396,13 +411,13 @@ SVMI_HD inline void exec_state_op(const DOpHdr& h, const DOp* __restrict__ op, c
         return;
     }
     switch (h.type) {
-        SVMI_CASE_ID(DOP_DENSE, DOP_DENSE + 100, (dispatch_dense<kMaxQ, N>(h.smask, a, coef + h.coef)))
+        SVMI_CASE_ID(DOP_DENSE, DOP_DENSE + 100, (dispatch_dense<kMaxQ, N>(h.smask, a, coef_at(coef, h.coef))))
         SVMI_CASE_ID(DOP_X, DOP_X + 100, dispatch_x<N>(h.s0, a))
         SVMI_CASE_ID(DOP_CX, DOP_CX + 100, dispatch_cx<N>(h.s0, h.s1, a))
         SVMI_CASE_ID(DOP_SWAP, DOP_SWAP + 100, dispatch_swap<N>(h.s0, h.s1, a))
         SVMI_CASE_ID(DOP_SRN, DOP_SRN + 100, dispatch_srn<N>(h.s0, a))
         SVMI_CASE_ID(DOP_CPHASE, DOP_CPHASE + 100, apply_cphase<N>(h, a, coef, goff, base))
-        SVMI_CASE_ID(DOP_DIAG, DOP_DIAG + 100, apply_diag<N>(*op, a, coef, goff, off, base))
+        SVMI_CASE_ID(DOP_DIAG, DOP_DIAG + 100, apply_diag<N>(h, *op, a, coef, goff, off, base))
         SVMI_CASE_ID(DOP_PHASESET, DOP_PHASESET + 100, apply_phaseset<N>(h, a, coef, goff, base, xf))
         SVMI_CASE_ID(DOP_CDENSE, DOP_CDENSE + 100, dispatch_cdense<N>(h, a, coef, goff, base))
     default: break;
@@ -411,12 +426,12 @@ SVMI_HD inline void exec_state_op(const DOpHdr& h, const DOp* __restrict__ op, c
 
 // Gradient op: Re sum conj(lam) K phi over this group;
 // pl = phi's H amplitudes of the group then lambda's.
-template <int kMaxQ, int H>
+template <int kMaxQ, int H, class Off>
 SVMI_HD inline double exec_grad_op(const DOpHdr& h, const DOp* __restrict__ op, const c64 (&pl)[2 * H],
-                                   const c64* __restrict__ coef, uint32_t goff, const uint32_t (&off)[kRegs],
+                                   const c64* __restrict__ coef, uint32_t goff, const Off& off,
                                    uint64_t base)
 {
-    if (h.type == DOP_GRAD_DENSE) return dispatch_grad_dense<kMaxQ, H>(h.smask, pl, coef + h.coef, h.s0);
+    if (h.type == DOP_GRAD_DENSE) return dispatch_grad_dense<kMaxQ, H>(h.smask, pl, coef_at(coef, h.coef), h.s0);
     // DOP_GRAD_DIAG
     const uint32_t e = diag_ext_index(*op, base);
     const c64* tab = coef + h.coef;
@@ -454,52 +469,6 @@ SVMI_HD inline void phase_gather_offsets(const PhaseInfo& ph, uint32_t (&off)[kR
             if ((r >> s) & 1) o ^= ph.gcol[s];
         off[r] = o;
     }
-}
-
-// Scatter offsets of a mapped phase: register rho is written to LDS offset
-// sxor ^ (XOR of scol[s] over the set bits s of rho) within the group.
-SVMI_HD inline void phase_scatter_offsets(const PhaseInfo& ph, uint32_t (&off)[kRegs])
-{
-#pragma unroll
-    for (int r = 0; r < kRegs; r++) {
-        uint32_t o = ph.sxor;
-#pragma unroll
-        for (int s = 0; s < kRegBits; s++)
-            if ((r >> s) & 1) o ^= ph.scol[s];
-        off[r] = o;
-    }
-}
-
-// LDS index of group g's base under a phase's tile map: XOR of gm[i] over the
-// set bits i of g (the group's register bits being zero).
-SVMI_HD inline uint32_t mapped_group_offset(const PhaseInfo& ph, uint32_t g)
-{
-    uint32_t o = 0;
-#pragma unroll
-    for (int i = 0; i < 10; i++)
-        if ((g >> i) & 1u) o ^= ph.gm[i];
-    return o;
-}
-
-// LDS index of tile-local index l under a sweep's final tile map.
-SVMI_HD inline uint32_t sweep_map(const SweepInfo& sw, uint32_t l)
-{
-    uint32_t o = 0;
-#pragma unroll
-    for (int b = 0; b < 14; b++)
-        if ((l >> b) & 1u) o ^= sw.fcol[b];
-    return o;
-}
-
-// The thread part of the store's map: M(tid) for tid below the tile's
-// thread count (at most 2^10 threads).
-SVMI_HD inline uint32_t sweep_map_thread(const SweepInfo& sw, uint32_t tid)
-{
-    uint32_t o = 0;
-#pragma unroll
-    for (int b = 0; b < 10; b++)
-        if ((tid >> b) & 1u) o ^= sw.fcol[b];
-    return o;
 }
 
 // Tile-local base index of group g: insert zero bits at the 4 register bits.

@@ -8,11 +8,12 @@
 // diagonal or SRN on <= 5 qubits) and scheduled (svmi_plan.cpp) into sweeps.
 // A sweep is one read+write pass over the state: the state is cut into tiles
 // of 2^k amplitudes that share all bits outside the sweep's tile qubit set T;
-// every tile is staged in LDS and a sequence of phases is applied to it.  A
-// phase picks 4 tile bits as "register bits" R: each thread holds the 16
-// amplitudes of one group (fixed non-R bits) in registers, applies every op of
-// the phase, and writes the group back to LDS.  Non-diagonal ops of a phase
-// act on R only; diagonal ops may act on any qubit (tile bit or not).
+// every tile is held by one workgroup, 16 amplitudes per thread, and a
+// sequence of phases is applied to it.  A phase picks 4 tile bits as
+// "register bits" R: each thread holds the 16 amplitudes of one group (fixed
+// non-R bits) in registers and applies every op of the phase; between two
+// phases the groups change through LDS (svmi_layout.cpp).  Non-diagonal ops
+// of a phase act on R only; diagonal ops may act on any qubit (tile bit or not).
 #pragma once
 
 #if defined(__HIPCC_RTC__)   // runtime compilation: its runtime header has the integer types
@@ -72,13 +73,22 @@ SVMI_HD inline c64 cmac(c64 acc, c64 m, c64 v)
     acc.im = SVMI_FMA(m.im, v.re, acc.im);
     return acc;
 }
+// acc += m * v in place
+SVMI_HD inline void cmac_to(c64& acc, c64 m, c64 v)
+{
+    acc.re = SVMI_FMA(m.re, v.re, acc.re);
+    acc.im = SVMI_FMA(m.re, v.im, acc.im);
+    acc.re = SVMI_FMA(-m.im, v.im, acc.re);
+    acc.im = SVMI_FMA(m.im, v.re, acc.im);
+}
 // conj(a) * b
 SVMI_HD inline c64 cconjmul(c64 a, c64 b) { return c64{a.re * b.re + a.im * b.im, a.re * b.im - a.im * b.re}; }
 
 constexpr int kRegBits = 4;                 // register bits per phase
 constexpr int kRegs = 1 << kRegBits;        // amplitudes per thread per group
-constexpr int kMaxTileQubits = 13;          // LDS tile: 2^13 * 16 B = 128 KiB
-constexpr int kMaxTileQubitsAdj = 11;       // two states (phi, lambda): 2 * 32 KiB
+constexpr int kMaxTileQubits = 13;          // 512 threads, 64 KiB of exchange area: two tiles per CU
+constexpr int kMaxTileQubitsAdj = 12;       // two states (phi, lambda): the same threads and LDS
+constexpr int kMaxBatchAdjTile = 11;        // largest svmi_batch_item::adj_tile
 // Two-state phases have 3 register bits; their fourth register "bit" is k,
 // the bit above the tile, which selects lambda's half of the LDS (phi at
 // [0, 2^k), lambda at [2^k, 2^(k+1))).  A thread's 16-amplitude group is then
@@ -103,7 +113,8 @@ constexpr int kMaxGradsPerSweep = 256;      // adjoint accumulators per sweep (L
 // Device op types.
 enum DOpType : uint16_t {
     DOP_NOP = 0,
-    DOP_DENSE = 1,   // dense 2^q x 2^q on register slots `smask`; coef = matrix
+    DOP_DENSE = 1,   // dense 2^q x 2^q on register slots `smask`; coef = matrix (q >= 3) or its
+                     // factors (q <= 2, apply_dense)
     DOP_X = 2,       // bit flip on slot s0
     DOP_CX = 3,      // control slot s0, target slot s1
     DOP_SWAP = 4,    // slots s0, s1
@@ -241,8 +252,8 @@ struct PhaseInfo {
     uint32_t scol[4];
     uint16_t gm[10];
     uint32_t mapped;     // M differs from the identity
+    uint32_t coef_begin, coef_end;   // the coefficients its ops read
 };
-static_assert(sizeof(PhaseInfo) == 88, "PhaseInfo layout");
 
 struct SweepInfo {
     uint32_t phase_begin, phase_end;
@@ -269,6 +280,84 @@ struct SweepInfo {
     uint32_t mapped;     // some phase or the tile's store addresses LDS through a tile map M
     uint16_t fcol[14];   // M after the last phase: fcol[b] = M(1 << b)
     uint16_t fj[16];     // M(j nt) (nt = the tile's threads): the store's per-register part
+    uint32_t stage;      // largest coefficient count of a phase
+};
+constexpr uint32_t kMaxStage = 2048;   // coefficients of a phase that the latency builds stage in LDS
+
+// ----------------------------------------------------------------------------
+// Register layouts (svmi_layout.cpp): how a sweep runs on the device.  The
+// tile lives in registers, 16 amplitudes per thread: the first phase's groups
+// are loaded from memory, the last one's stored, and between two phases the
+// tile changes hands through LDS, the real parts first and then the imaginary
+// ones, so an exchange needs 8 bytes of LDS per amplitude.  Every address is
+// linear over GF(2) in the thread and register bits: a thread's part comes
+// from a table by lane XOR one by wave, a register's part is the XOR of the
+// columns of its set bits.
+// ----------------------------------------------------------------------------
+constexpr int kLaneBits = 6;
+constexpr int kMaxWaveBits = 4;
+constexpr int kLaneEntries = 1 << kLaneBits;
+constexpr int kWaveEntries = 1 << kMaxWaveBits;
+
+// The thread part of a phase's addresses, as four 16-bit fields: LDS byte
+// offset written (by the previous phase's layout) and read in the exchange
+// before the phase, the group's tile-local index bits, the group's number.
+SVMI_HD inline uint64_t thread_entry(uint32_t w, uint32_t r, uint32_t goff, uint32_t grp)
+{
+    return uint64_t(w) | uint64_t(r) << 16 | uint64_t(goff) << 32 | uint64_t(grp) << 48;
+}
+
+enum : uint32_t {
+    LPH_CROSS = 1,     // the exchange moves amplitudes between waves
+    LPH_GUARD = 2,     // other waves may still read this wave's part of LDS
+};
+// (What is uniform is stored ready for use: the sweeps are bound by the rate
+// at which a SIMD issues instructions, scalar ones included.)
+struct LayoutPhase {
+    uint32_t w[kRegs], rd[kRegs];   // exchange before the phase: LDS byte offset of each register
+    uint32_t op_begin, op_end;
+    uint32_t flags;                 // LPH_*
+    uint32_t coef_n;                // the phase's coefficients: [coef_begin, coef_begin + coef_n)
+    uint32_t rcol[4];               // 1 << register bit (tile-local; two states: the last is 1 << k)
+    uint32_t coef_begin;
+    uint32_t pad[3];
+};
+static_assert(sizeof(LayoutPhase) == 176, "LayoutPhase layout");
+
+// A run of tile id bits that are consecutive qubits: base bits
+// ((tile << shl) >> shr) & mask.
+struct TileRun {
+    uint64_t mask;
+    uint32_t shl, shr;
+};
+constexpr int kMaxTileRuns = 40;
+constexpr uint32_t kIoAdditive = 1;   // (<< side) register and thread offsets share no bits: they add
+
+// A sweep's layout phases, and the byte offsets of its loads ([0]) and stores
+// ([1]) from a tile's first amplitude: the XOR of the set lane bits' columns,
+// the wave's entry and the register's.
+struct SweepIO {
+    uint64_t lane[2][kLaneBits];
+    uint64_t wave[2][kWaveEntries];
+    uint64_t reg[2][kRegs];      // two states: the first 8, for either state
+    uint32_t ph_begin, ph_end;   // into the layout phases; lane and wave tables run parallel to them
+    uint32_t store_guard;        // a wave stores where another one loads, and no exchange between the
+                                 // waves lies in between: the workgroup meets before the stores
+    uint32_t additive;
+    uint32_t n_runs;             // of the tile id
+    uint32_t vhi_shift;          // tile >> vhi_shift: the variant qubits (SweepInfo::exthi)
+    uint64_t pad;
+    TileRun run[kMaxTileRuns];
+};
+
+// Registers' tile-local offsets without an array of 16 (the ops index it with
+// constants after unrolling).
+struct RegOffsets {
+    const uint32_t (&c)[4];
+    SVMI_HD uint32_t operator[](int r) const
+    {
+        return ((r & 1) ? c[0] : 0u) | ((r & 2) ? c[1] : 0u) | ((r & 4) ? c[2] : 0u) | ((r & 8) ? c[3] : 0u);
+    }
 };
 
 // A standalone op (run by its own kernel on the whole state, outside sweeps).
@@ -325,7 +414,19 @@ struct SlotMask {
     }
 };
 
+// coef + i as base and 32-bit byte offset (one scalar shift instead of a
+// 64-bit shift and add per access).
+SVMI_HD inline const c64* coef_at(const c64* coef, uint32_t i)
+{
+    return reinterpret_cast<const c64*>(reinterpret_cast<const char*>(coef) + uint32_t(i * 16u));
+}
+
 // Dense 2^q x 2^q (row-major, matrix bit i <-> i-th set slot of S).
+// Up to two qubits M holds factors of the matrix (matrix = Lo . Up, Up with a
+// unit diagonal; Up above the diagonal, Lo on and below it): both triangles
+// run in place -- the same FMAs as the product, and no second copy of the
+// amplitudes, with which the sweep kernels would not fit 128 registers (284
+// spilled, 29 with this form).
 template <int S, int N = kRegs>
 SVMI_HD inline void apply_dense(c64 (&a)[N], const c64* __restrict__ M)
 {
@@ -335,15 +436,34 @@ SVMI_HD inline void apply_dense(c64 (&a)[N], const c64* __restrict__ M)
     for (int h = 0; h < N; h += kRegs)
 #pragma unroll
         for (int o = 0; o < (kRegs >> q); o++) {
-            c64 v[D];
+            const auto v = [&](int j) -> c64& {
+                return a[h | SlotMask<S>::spread_out(o) | SlotMask<S>::spread(j)];
+            };
+            if constexpr (q <= 2) {
 #pragma unroll
-            for (int j = 0; j < D; j++) v[j] = a[h | SlotMask<S>::spread_out(o) | SlotMask<S>::spread(j)];
+                for (int i = 0; i < D; i++)
 #pragma unroll
-            for (int i = 0; i < D; i++) {
-                c64 acc = c64{0.0, 0.0};
+                    for (int j = i + 1; j < D; j++) cmac_to(v(i), M[i * D + j], v(j));
 #pragma unroll
-                for (int j = 0; j < D; j++) acc = cmac(acc, M[i * D + j], v[j]);
-                a[h | SlotMask<S>::spread_out(o) | SlotMask<S>::spread(i)] = acc;
+                for (int i = D - 1; i >= 0; i--) {
+                    cmul_to(v(i), M[i * D + i]);
+#pragma unroll
+                    for (int j = 0; j < i; j++) cmac_to(v(i), M[i * D + j], v(j));
+                }
+            } else {
+                c64 w[D];
+#pragma unroll
+                for (int j = 0; j < D; j++) w[j] = v(j);
+#pragma unroll
+                for (int i = 0; i < D; i++) {
+                    c64 acc = c64{0.0, 0.0};
+#pragma unroll
+                    for (int j = 0; j < D; j++) acc = cmac(acc, M[i * D + j], w[j]);
+                    v(i) = acc;
+#if defined(__HIP_DEVICE_COMPILE__)
+                    __builtin_amdgcn_sched_barrier(0);   // rows one by one: fewer registers
+#endif
+                }
             }
         }
 }

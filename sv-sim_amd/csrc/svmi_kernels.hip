@@ -1,13 +1,12 @@
 // svmi_kernels.hip -- CDNA4 (gfx950) kernels of the state-vector engine.
 //
-// k_sweep<NS>: one tiled sweep (the hot kernel).  One workgroup per tile of
-//   2^k amplitudes, 2^(k-4) threads; the tile is staged in LDS (swizzled),
-//   each phase gathers one 16-amplitude register group per thread, runs the
-//   phase's ops in registers and writes the group back; after the last phase
-//   the tile goes back to HBM.  Loads/stores are 16-byte per lane and the
-//   low c physical qubits of every tile are contiguous, so each group of
-//   2^c lanes reads one 2^c*16-byte segment.  NS = 2 runs the adjoint sweep
-//   over (phi, lambda) and accumulates gradient partial sums per tile.
+// k_sweep1 / k_sweep2: one tiled sweep (the hot kernels).  One workgroup per
+//   tile of 2^k amplitudes (per state), 16 amplitudes per thread in registers;
+//   each phase runs its ops on them and the tile changes hands through LDS in
+//   between.  Loads and stores are 16 bytes per lane and the low c physical
+//   qubits of every tile are contiguous, so each group of 2^c lanes reads one
+//   2^c*16-byte segment.  k_sweep2 runs the adjoint sweep over (phi, lambda)
+//   and accumulates gradient partial sums per tile.
 // Standalone ops (5-qubit dense, per-op mode), sampling, Pauli sums and
 //   state fills are simple grid-stride kernels.
 #include <hip/hip_runtime.h>
@@ -18,66 +17,6 @@
 namespace svmi {
 
 // ------------------------------------------------------------------ sweeps
-
-// Tile staging.  A tile is 2^k amplitudes; thread tid owns tile-local
-// indices l = tid + nt*j (j < J: 16 for one state, 8 per state for two);
-// global index = base | row(l >> c) | (l & cmask).  LDS holds the tile
-// XOR-swizzled (lds_slot) at LDS index lo + l: lo = 0, or 2^k for lambda's
-// half of a two-state tile.
-
-// HBM (or |0..0> when init_zero) -> registers r[j] for the tile at `base`.
-template <int J>
-__device__ __attribute__((always_inline)) inline void
-tile_fetch(c64 (&r)[J], const c64* __restrict__ s, const SweepInfo& sw, const uint64_t* __restrict__ ht,
-           uint64_t base, uint32_t tid, uint32_t nt, bool init_zero)
-{
-    const uint32_t cmask = (1u << sw.c) - 1u;
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const uint32_t l = tid + nt * j;
-        const uint64_t g = base | ht[l >> sw.c] | (l & cmask);
-        r[j] = init_zero ? c64{g == 0 ? 1.0 : 0.0, 0.0} : s[g];
-    }
-}
-
-template <int J>
-__device__ __attribute__((always_inline)) inline void
-tile_put(const c64 (&r)[J], c64* t, uint32_t lo, uint32_t tid, uint32_t nt)
-{
-#pragma unroll
-    for (int j = 0; j < J; j++) t[lds_slot(lo + tid + nt * j)] = r[j];
-}
-
-// LDS -> HBM for the tile at `base` when the sweep ends with a tile map:
-// tile-local index l = tid + nt j sits at LDS index M(tid) ^ M(nt j), the
-// second part precomputed per sweep (SweepInfo::fj).
-template <int J>
-__device__ __attribute__((always_inline)) inline void
-tile_store_mapped(const c64* t, uint32_t lo, c64* __restrict__ s, const SweepInfo& sw,
-                  const uint64_t* __restrict__ ht, uint64_t base, uint32_t tid, uint32_t nt)
-{
-    const uint32_t cmask = (1u << sw.c) - 1u;
-    const uint32_t mt = sweep_map_thread(sw, tid);
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const uint32_t l = tid + nt * j;
-        s[base | ht[l >> sw.c] | (l & cmask)] = t[lds_slot(lo + (mt ^ sw.fj[j]))];
-    }
-}
-
-// LDS -> HBM for the tile at `base`.
-template <int J>
-__device__ __attribute__((always_inline)) inline void
-tile_store(const c64* t, uint32_t lo, c64* __restrict__ s, const SweepInfo& sw, const uint64_t* __restrict__ ht,
-           uint64_t base, uint32_t tid, uint32_t nt)
-{
-    const uint32_t cmask = (1u << sw.c) - 1u;
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const uint32_t l = tid + nt * j;
-        s[base | ht[l >> sw.c] | (l & cmask)] = t[lds_slot(lo + l)];
-    }
-}
 
 // v of a lane moved by one DPP pattern (both halves of the double from the
 // same source lane); lanes without a source, or outside row_mask, get 0.
@@ -104,80 +43,6 @@ __device__ __attribute__((always_inline)) inline double wave_sum_lane63(double v
     return v;
 }
 
-// The phases of one sweep on the tile in LDS (t0; for NS = 2 phi then lambda).
-// Threads tid < nt own one register group per phase; with kIdle (batched
-// kernel: blockDim >= nt) the others only join the barriers.  Without kIdle
-// every thread is active, which keeps the phase body free of divergence
-// (and its register groups out of scratch).  Ends with a barrier.
-// kMap: the phases address LDS through their tile maps (every two-state
-// sweep; one-state sweeps whose SweepInfo::mapped is set).
-template <int NS, bool kIdle, int kMaxQ, bool kMap = (NS == 2)>
-__device__ __attribute__((always_inline)) inline void
-tile_phases(c64* t0, double* gacc, const c64* xf, const SweepInfo& sw,
-            const PhaseInfo* __restrict__ phases, const DOp* __restrict__ ops, const c64* __restrict__ coef,
-            uint64_t base, uint32_t tid, uint32_t nt)
-{
-    const bool active = !kIdle || tid < nt;
-    const uint32_t nwaves = (nt + 63) / 64;
-    const uint32_t vhi = uint32_t(extract_bits(base, sw.exthi));
-    for (uint32_t p = sw.phase_begin; p < sw.phase_end; p++) {
-        if (active) {
-            const PhaseInfo ph = phases[p];
-            uint32_t off[kRegs], goffs[kRegs];
-            phase_offsets(ph, off);
-            phase_gather_offsets(ph, goffs);
-            const uint32_t goff = group_offset(ph, tid);
-            // NS = 2: the phase's last register bit is k, so a[0..7] are
-            // phi's amplitudes and a[8..15] lambda's (t1 = t0 + 2^k) and every
-            // op, dispatched once, acts on both.  The group's amplitudes sit
-            // at LDS indices under the tile map (gphys, gather and scatter
-            // offsets); the ops see the plain tile-local indices (goff, off).
-            uint32_t gphys = goff;
-            if constexpr (kMap) gphys = mapped_group_offset(ph, tid);
-            c64 a[kRegs];
-#pragma unroll
-            for (int r = 0; r < kRegs; r++) a[r] = t0[lds_slot(kMap ? (gphys ^ goffs[r]) : (goff | goffs[r]))];
-            // op headers are fetched one op ahead so the scalar-load latency
-            // of the next op overlaps the arithmetic of the current one (every
-            // op array ends with a NOP, so the read past a phase's last op
-            // stays inside it)
-            const DOp* __restrict__ op = ops + ph.op_begin;
-            DOpHdr nxt = op->h;
-            for (uint32_t o = ph.op_begin; o < ph.op_end; o++, op++) {
-                const DOpHdr h = nxt;
-                nxt = op[1].h;
-                if constexpr (NS == 2) {
-                    if (h.type == DOP_GRAD_DENSE || h.type == DOP_GRAD_DIAG) {
-                        // every gradient op of a sweep has its own slot and each
-                        // wave runs it once: a plain store, no read
-                        double v = exec_grad_op<kMaxDenseQubitsAdj, kRegsAdj>(h, op, a, coef, goff, off, base);
-                        if (nt >= 64) {
-                            v = wave_sum_lane63(v);
-                            if ((tid & 63u) == 63u) gacc[h.grad * nwaves + (tid >> 6)] = v;
-                        } else {
-                            const int width = int(nt);
-                            for (int d = width >> 1; d > 0; d >>= 1) v += __shfl_xor(v, d, width);
-                            if (tid == 0) gacc[h.grad * nwaves] = v;
-                        }
-                        continue;
-                    }
-                }
-                exec_state_op<kMaxQ>(h, op, a, coef, goff, tid, off, base, xf, sw.exthi, vhi);
-            }
-            if constexpr (kMap) {
-                uint32_t soffs[kRegs];
-                phase_scatter_offsets(ph, soffs);
-#pragma unroll
-                for (int r = 0; r < kRegs; r++) t0[lds_slot(gphys ^ soffs[r])] = a[r];
-            } else {
-#pragma unroll
-                for (int r = 0; r < kRegs; r++) t0[lds_slot((goff | off[r]) ^ ph.sxor)] = a[r];
-            }
-        }
-        __syncthreads();
-    }
-}
-
 // The tile's phase factors (one per factor slot of the sweep) into LDS; the
 // caller's next barrier publishes them.
 __device__ __attribute__((always_inline)) inline void
@@ -195,55 +60,236 @@ tile_factors(c64* xf, const SweepInfo& sw, const DOp* __restrict__ ops, const c6
     }
 }
 
-// LDS of a tile: t0 (NS = 2: phi's 2^k then lambda's) | phase factors |
-// gradient accumulators.
+// LDS of a tile: exchange area (8 bytes per amplitude of every state) | phase
+// factors | gradient accumulators.
+size_t sweep_smem_bytes(const SweepInfo& sw, int ns)
+{
+    const size_t nwaves = (size_t(sweep_threads(sw.k, ns)) + 63) / 64;
+    return (size_t(8) << sw.k) * ns + size_t(16) * sw.n_xf + size_t(8) * sw.n_grad * nwaves;
+}
+
+// The program's read-only tables, as restrict arguments of the kernels: from a
+// struct of pointers the op records and coefficients would be read with
+// vector loads instead of through the scalar cache.
+#define SVMI_TABLES                                                                                 \
+    const LayoutPhase *__restrict__ lph, const uint64_t *__restrict__ ltab,                         \
+        const uint64_t *__restrict__ wtab, const DOp *__restrict__ ops, const c64 *__restrict__ coef
+#define SVMI_TABLE_ARGS lph, ltab, wtab, ops, coef
+#define SVMI_TABLES_OF(t) (t).lphases, (t).lane_tab, (t).wave_tab, (t).ops, (t).coef
+
+__device__ __attribute__((always_inline)) inline double& lds_at(unsigned char* smem, uint32_t byte)
+{
+    return *reinterpret_cast<double*>(smem + byte);
+}
+
 // One tile of one sweep: load, phases, store (and for NS = 2 the tile's
 // gradient partials).  init_zero: the tile is generated as |0..0>.
-template <int NS, bool kIdle, int kMaxQ = (NS == 2 ? kMaxDenseQubitsAdj : kRegBits), bool kMap = (NS == 2)>
+//
+// The tile stays in registers: a[0..15] per thread (NS = 2: phi's 8
+// amplitudes, then lambda's), 64 VGPRs, which with the op templates fit the
+// 128 that leave four waves per SIMD.  Between two phases the amplitudes
+// change threads through LDS, real parts first: 8 bytes per amplitude, so two
+// 13-qubit tiles share a CU (tiles held in LDS: one, or two of 12 qubits at
+// two waves per SIMD).  u3 brick wall at 30 qubits, 23 sweeps of 9.18 ms ->
+// 19 of 8.65 ms (12-qubit tiles: 23 of 7.83); a two-state sweep at 25 qubits
+// 641 -> 490 us.
+//
+// What bounds it: HBM (6.4 ms of the 8.65 at the copy rate), then the issue
+// slots of a SIMD, which scalar instructions and branches share with the
+// FMAs; hence the tables of ready offsets (LayoutPhase, SweepIO), 32-bit
+// coefficient offsets and no loads ahead: 4070 -> 3490 instructions per wave,
+// 1600 of them FMAs, u3 176 -> 167 ms.
+//
+// kLat: the build for sweeps of few tiles, which leave the chip idle and are
+// bound by latency: a cold scalar load takes a microsecond, a register table
+// four of them in a row.  Every phase's coefficients are staged in LDS during
+// the phase before it and the next op's header is loaded during an op.
+template <int NS, int kMaxQ, bool kLat = false>
 __device__ __attribute__((always_inline)) inline void
-sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw,
-           const PhaseInfo* __restrict__ phases, const DOp* __restrict__ ops,
-           const c64* __restrict__ coef, const uint64_t* __restrict__ hitab,
-           double* __restrict__ grad_partials, uint64_t tile, uint32_t nt, unsigned char* smem,
-           bool init_zero)
+sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, const SweepIO* __restrict__ io, SVMI_TABLES,
+           double* __restrict__ grad_partials, uint64_t tile, unsigned char* smem, bool init_zero)
 {
-    const uint32_t tsize = 1u << sw.k;
-    c64* t0 = reinterpret_cast<c64*>(smem);
-    c64* xf = t0 + tsize * NS;
-    double* gacc = reinterpret_cast<double*>(xf + sw.n_xf);
-    const uint32_t tid = threadIdx.x;
-    const bool active = !kIdle || tid < nt;
+    const uint32_t tid = threadIdx.x, nt = blockDim.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nwaves = (nt + 63) / 64;
-    const uint64_t* ht = hitab + sw.hitab;
-    const uint64_t base = tile_base(sw, tile);
-
-    constexpr int J = NS == 2 ? kRegsAdj : kRegs;   // amplitudes per thread per state
-    if (active) {
-        // both states' loads are issued before either waits
-        c64 r[J], r1[J];
-        tile_fetch(r, s0, sw, ht, base, tid, nt, init_zero);
-        if constexpr (NS == 2) tile_fetch(r1, s1, sw, ht, base, tid, nt, false);
-        tile_put(r, t0, 0u, tid, nt);
-        if constexpr (NS == 2) tile_put(r1, t0, tsize, tid, nt);
+    c64* xf = reinterpret_cast<c64*>(smem + (size_t(8 * NS) << sw.k));
+    double* gacc = reinterpret_cast<double*>(xf + sw.n_xf);
+    uint64_t base = 0;
+    for (uint32_t i = 0; i < io->n_runs; i++) {
+        const TileRun r = io->run[i];
+        base |= ((tile << r.shl) >> r.shr) & r.mask;
     }
-    if (NS == 2)
-        for (uint32_t i = tid; i < sw.n_grad * nwaves; i += blockDim.x) gacc[i] = 0.0;
+    // the thread's byte offset of a load (0) or store (1)
+    const auto thread_off = [&](int side) {
+        uint64_t u = (base << 4) ^ io->wave[side][wave];
+#pragma unroll
+        for (int i = 0; i < kLaneBits; i++) u ^= ((lane >> i) & 1u) ? io->lane[side][i] : uint64_t(0);
+        return u;
+    };
+    const auto amp = [](c64* s, uint64_t off) { return reinterpret_cast<c64*>(reinterpret_cast<char*>(s) + off); };
+    // the tile's factors before its loads: their tables take 64 registers
     tile_factors(xf, sw, ops, coef, base, tid);
-    __syncthreads();
-    tile_phases<NS, kIdle, kMaxQ, kMap>(t0, gacc, xf, sw, phases, ops, coef, base, tid, nt);
-    if (active) {
-        if (kMap && sw.mapped) {
-            tile_store_mapped<J>(t0, 0u, s0, sw, ht, base, tid, nt);
-            if constexpr (NS == 2) tile_store_mapped<J>(t0, tsize, s1, sw, ht, base, tid, nt);
+    c64 a[kRegs];
+    {
+        // in batches of four, so that addresses do not hold registers long
+        const uint64_t g = thread_off(0);
+        if (init_zero) {
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) a[r] = c64{(g ^ io->reg[0][r]) == 0 ? 1.0 : 0.0, 0.0};
+        } else if (io->additive & kIoAdditive) {
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                const bool second = NS == 2 && r >= kRegsAdj;
+                a[r] = *amp(amp(second ? s1 : s0, g), io->reg[0][second ? r - kRegsAdj : r]);
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
         } else {
-            tile_store<J>(t0, 0u, s0, sw, ht, base, tid, nt);
-            if constexpr (NS == 2) tile_store<J>(t0, tsize, s1, sw, ht, base, tid, nt);
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                const bool second = NS == 2 && r >= kRegsAdj;
+                a[r] = *amp(second ? s1 : s0, g ^ io->reg[0][second ? r - kRegsAdj : r]);
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    const uint32_t vhi = uint32_t(tile >> io->vhi_shift);
+    // a phase's thread entry is loaded during the phase before it
+    const uint32_t ph_begin = io->ph_begin, ph_end = io->ph_end;
+    c64* const stage = reinterpret_cast<c64*>(gacc + sw.n_grad * nwaves + (sw.n_grad * nwaves & 1u));
+    if constexpr (kLat) {
+        const uint32_t n = lph[ph_begin].coef_n, c0 = lph[ph_begin].coef_begin;
+        for (uint32_t i = tid; i < n; i += nt) stage[i] = coef[c0 + i];
+    }
+    if (kLat || sw.n_xf) __syncthreads();
+    uint64_t le = ltab[ph_begin * uint32_t(kLaneEntries) + lane];
+    for (uint32_t p = ph_begin; p < ph_end; p++) {
+        const LayoutPhase& L = lph[p];
+        const uint64_t te = le ^ wtab[p * uint32_t(kWaveEntries) + wave];
+        const uint32_t pn = p + 1 < ph_end ? p + 1 : p;
+        le = ltab[pn * uint32_t(kLaneEntries) + lane];
+        if (p != ph_begin) {
+            uint32_t w = uint32_t(te) & 0xffffu, rd = uint32_t(te) >> 16;
+            const uint32_t flags = L.flags;
+            const bool cross = flags & LPH_CROSS;
+            // a wave's LDS operations complete in order: inside the waves the
+            // order of the instructions is enough
+            const auto meet = [&]() {
+                if (cross) __syncthreads();
+                else asm volatile("" ::: "memory");
+            };
+            if (flags & LPH_GUARD) __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                lds_at(smem, w ^ L.w[r]) = a[r].re;
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            meet();
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                a[r].re = lds_at(smem, rd ^ L.rd[r]);
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            // fresh copies, or 32 addresses would stay in registers from the first half
+            asm volatile("" : "+v"(w), "+v"(rd));
+            meet();
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                lds_at(smem, w ^ L.w[r]) = a[r].im;
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            meet();
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                a[r].im = lds_at(smem, rd ^ L.rd[r]);
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        const uint32_t goff = uint32_t(te >> 32) & 0xffffu, grp = uint32_t(te >> 48);
+        const RegOffsets off{L.rcol};
+        const uint32_t op_end = L.op_end;
+        const DOp* __restrict__ op = ops + L.op_begin;
+        // kLat: this phase's coefficients in one half of the stage; the next
+        // one's are on their way, up to kPre per thread in registers
+        constexpr uint32_t kPre = 4;
+        const c64* __restrict__ cf = coef;
+        c64 pre[kLat ? kPre : 1];
+        uint32_t pre_n = 0, pre_c = 0;
+        DOpHdr nxt;
+        if constexpr (kLat) {
+            cf = stage + ((p - ph_begin) & 1u) * sw.stage;
+            if (p + 1 < ph_end) {
+                pre_n = lph[p + 1].coef_n;
+                pre_c = lph[p + 1].coef_begin;
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kPre; i++)
+                pre[i] = coef[tid + nt * i < pre_n ? pre_c + tid + nt * i : 0u];
+            nxt = op->h;
+        }
+        for (uint32_t o = L.op_begin; o < op_end; o++, op++) {
+            DOpHdr h;
+            if constexpr (kLat) {   // (op arrays end with an unused record)
+                h = nxt;
+                nxt = op[1].h;
+                if (h.type == DOP_ROT && h.s0) h.grad -= L.coef_begin;   // its table
+                h.coef -= L.coef_begin;
+            } else {
+                h = op->h;
+            }
+            if constexpr (NS == 2) {
+                if (h.type == DOP_GRAD_DENSE || h.type == DOP_GRAD_DIAG) {
+                    // every gradient op of a sweep has its own slot and each
+                    // wave runs it once: a plain store, no read
+                    double v = exec_grad_op<kMaxDenseQubitsAdj, kRegsAdj>(h, op, a, cf, goff, off, base);
+                    if (nt >= 64) {
+                        v = wave_sum_lane63(v);
+                        if (lane == 63u) gacc[h.grad * nwaves + wave] = v;
+                    } else {
+                        const int width = int(nt);
+                        for (int d = width >> 1; d > 0; d >>= 1) v += __shfl_xor(v, d, width);
+                        if (tid == 0) gacc[h.grad * nwaves] = v;
+                    }
+                    continue;
+                }
+            }
+            exec_state_op<kMaxQ>(h, op, a, cf, goff, grp, off, base, xf, sw.exthi, vhi);
+        }
+        if constexpr (kLat) {
+            c64* const to = stage + ((p + 1 - ph_begin) & 1u) * sw.stage;
+#pragma unroll
+            for (uint32_t i = 0; i < kPre; i++)
+                if (tid + nt * i < pre_n) to[tid + nt * i] = c64{pre[i].re, pre[i].im};   // (by value: see k_pauli)
+            for (uint32_t i = tid + nt * kPre; i < pre_n; i += nt) to[i] = coef[pre_c + i];
+            __syncthreads();
+        }
+    }
+    if (io->store_guard) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's loads are done
+        __syncthreads();
+    }
+    {
+        const uint64_t g = thread_off(1);
+        if (io->additive & (kIoAdditive << 1)) {
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                const bool second = NS == 2 && r >= kRegsAdj;
+                *amp(amp(second ? s1 : s0, g), io->reg[1][second ? r - kRegsAdj : r]) = a[r];
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < kRegs; r++) {
+                const bool second = NS == 2 && r >= kRegsAdj;
+                *amp(second ? s1 : s0, g ^ io->reg[1][second ? r - kRegsAdj : r]) = a[r];
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
         }
     }
     // gradient partials are stored grad-major ([i][tile]) so the sum over
     // tiles of one gradient reads one contiguous segment
-    if (NS == 2) {
-        for (uint32_t i = tid; i < sw.n_grad; i += blockDim.x) {
+    if constexpr (NS == 2) {
+        if (sw.n_grad) __syncthreads();
+        for (uint32_t i = tid; i < sw.n_grad; i += nt) {
             double v = 0.0;
             for (uint32_t w = 0; w < nwaves; w++) v += gacc[i * nwaves + w];
             grad_partials[i * sw.n_tiles + tile] = v;
@@ -251,137 +297,35 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw,
     }
 }
 
-// One state, one tile per workgroup: up to 8 waves per CU (one 2^13 tile of
-// 512 threads, or two 2^12 tiles of 256), so 256 VGPRs per thread.
-// stagger_lo..stagger_hi: workgroups of the first resident wave that start
-// later (by `stagger` sleeps of 127*64 cycles), so that the co-resident
-// workgroups of a CU alternate loading and computing.
+// Waves per SIMD of the sweep kernels: dense blocks of three and four register
+// qubits need up to 64 registers for their results.
+template <int kMaxQ>
+constexpr int kSweepWaves = kMaxQ <= 2 ? 4 : 2;
+
+// One state, one tile per workgroup.
 // kMaxQ: widest dense block compiled in (sweeps with blocks of at most two
 // register qubits run the kMaxQ = 2 build, which holds fewer registers).
-// kMap: the build for sweeps with tile maps (SweepInfo::mapped).
-template <int kMaxQ, bool kMap>
-__global__ void __launch_bounds__(kMaxTileThreads, 1)
-k_sweep1(c64* __restrict__ s0, const SweepInfo sw, const PhaseInfo* __restrict__ phases,
-         const DOp* __restrict__ ops, const c64* __restrict__ coef, const uint64_t* __restrict__ hitab,
-         uint64_t tile_offset, uint32_t stagger_lo, uint32_t stagger_hi, uint32_t stagger)
+// kLat: see sweep_tile.
+template <int kMaxQ, bool kLat>
+__global__ void __launch_bounds__(kMaxTileThreads, kLat ? 2 : kSweepWaves<kMaxQ>)
+k_sweep1(c64* __restrict__ s0, const SweepInfo sw, const SweepIO* __restrict__ io, SVMI_TABLES, uint64_t tile_offset)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    if (blockIdx.x >= stagger_lo && blockIdx.x < stagger_hi)
-        for (uint32_t i = 0; i < stagger; i++) __builtin_amdgcn_s_sleep(127);
-    sweep_tile<1, false, kMaxQ, kMap>(s0, nullptr, sw, phases, ops, coef, hitab, nullptr, tile_offset + blockIdx.x, blockDim.x,
-                         smem, false);
+    sweep_tile<1, kMaxQ, kLat>(s0, nullptr, sw, io, SVMI_TABLE_ARGS, nullptr, tile_offset + blockIdx.x, smem, false);
 }
 
-// One state, persistent and software-pipelined: workgroup w handles tiles
-// w, w + gridDim.x, ...  While the phases of tile t run out of LDS, the
-// loads of the next tile are already in flight into registers, so HBM
-// traffic overlaps the arithmetic inside each workgroup (co-resident
-// workgroups start in step and would otherwise load and compute together).
-// kWide: 256-thread workgroups with the full 512-VGPR budget (one per CU);
-// otherwise up to 512 threads and 256 VGPRs.
-template <bool kWide>
-__global__ void __launch_bounds__(kWide ? 256 : kMaxTileThreads, 1)
-k_sweep1p(c64* __restrict__ s0, const SweepInfo sw, const PhaseInfo* __restrict__ phases,
-          const DOp* __restrict__ ops, const c64* __restrict__ coef, const uint64_t* __restrict__ hitab,
-          uint64_t tile_offset, uint64_t n_tiles)
-{
-    extern __shared__ __align__(16) unsigned char smem[];
-    c64* t0 = reinterpret_cast<c64*>(smem);
-    c64* xf = t0 + (size_t(1) << sw.k);
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    const uint64_t* ht = hitab + sw.hitab;
-    uint64_t t = blockIdx.x;
-    c64 nx[kRegs];
-    tile_fetch(nx, s0, sw, ht, tile_base(sw, tile_offset + t), tid, nt, false);
-    for (;;) {
-        const uint64_t base = tile_base(sw, tile_offset + t);
-        tile_put(nx, t0, 0u, tid, nt);
-        tile_factors(xf, sw, ops, coef, base, tid);
-        __syncthreads();
-        const uint64_t tn = t + gridDim.x;
-        const bool more = tn < n_tiles;
-        if (more) tile_fetch(nx, s0, sw, ht, tile_base(sw, tile_offset + tn), tid, nt, false);
-        tile_phases<1, false, kRegBits>(t0, nullptr, xf, sw, phases, ops, coef, base, tid, nt);
-        tile_store<kRegs>(t0, 0u, s0, sw, ht, base, tid, nt);
-        if (!more) break;
-        __syncthreads();  // the store's LDS reads finish before the next put
-        t = tn;
-    }
-}
-
-// ---------------------------------------------- double-buffered sweeps
-//
-// LDS DMA helpers (lds_dma16, tile_dma): svmi_exec.hpp.
-
-size_t dma_sweep_smem_bytes(const SweepInfo& sw)
-{
-    return (size_t(32) << kDmaTileQubits) + (size_t(8) << (kDmaTileQubits - sw.c)) + size_t(16) * sw.n_xf;
-}
-
-// One state, persistent, two tile buffers of 2^12 amplitudes: while the
-// phases of tile t run in one buffer, tile t + gridDim.x streams into the
-// other, so HBM traffic overlaps the arithmetic inside every workgroup (one
-// per CU).  LDS: two tiles | the sweep's row table | phase factors.  Per
-// tile: wait for its DMA (all but the previous tile's kRegs stores, the
-// youngest memory operations), barrier, the tile's factors, the next tile's
-// DMA, barrier, phases, stores.
-template <int kMaxQ>
-__global__ void __launch_bounds__(kDmaThreads, 1)
-k_sweep1d(c64* __restrict__ s0, const SweepInfo sw, const PhaseInfo* __restrict__ phases,
-          const DOp* __restrict__ ops, const c64* __restrict__ coef, const uint64_t* __restrict__ hitab)
-{
-    extern __shared__ __align__(16) unsigned char smem[];
-    constexpr uint32_t kT = 1u << kDmaTileQubits;
-    c64* buf = reinterpret_cast<c64*>(smem);
-    uint64_t* ht = reinterpret_cast<uint64_t*>(buf + 2 * kT);
-    c64* xf = reinterpret_cast<c64*>(ht + (kT >> sw.c));
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-    for (uint32_t i = tid; i < (kT >> sw.c); i += kDmaThreads) ht[i] = hitab[sw.hitab + i];
-    __syncthreads();
-    const uint32_t lds0 = lds_address(buf);
-    uint64_t t = blockIdx.x;
-    tile_dma(s0, ht, sw.c, tile_base(sw, t), lds0, wave, lane);
-    uint32_t cur = 0;
-    bool first = true;
-    for (;;) {
-        // tile_store<kRegs> below issues kRegs = 16 stores per thread, so
-        // vmcnt(16) leaves only those outstanding and this tile's DMA done
-        if (first) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        __syncthreads();
-        const uint64_t base = tile_base(sw, t);
-        const uint64_t tn = t + gridDim.x;
-        const bool more = tn < sw.n_tiles;
-        // factors first: their global loads would otherwise wait for the
-        // DMA; the explicit vmcnt(0) tells the compiler's wait analysis that
-        // no load of theirs is still in flight (a pending one whose register
-        // a later LDS read reuses would make it wait for everything)
-        tile_factors(xf, sw, ops, coef, base, tid);
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), expcnt/lgkmcnt unconstrained
-        if (more) tile_dma(s0, ht, sw.c, tile_base(sw, tn), lds0 + (cur ^ 1u) * kT * 16u, wave, lane);
-        if (sw.n_xf) __syncthreads();
-        c64* t0 = buf + cur * kT;
-        tile_phases<1, false, kMaxQ>(t0, nullptr, xf, sw, phases, ops, coef, base, tid, kDmaThreads);
-        tile_store<kRegs>(t0, 0u, s0, sw, ht, base, tid, kDmaThreads);
-        if (!more) break;
-        t = tn;
-        cur ^= 1u;
-        first = false;
-    }
-}
-
-// Two states (adjoint): two register groups per thread (one wave per SIMD),
-// dense ops of at most 2 qubits.
-__global__ void __launch_bounds__(kThreads, 1)
-k_sweep2(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo sw, const PhaseInfo* __restrict__ phases,
-         const DOp* __restrict__ ops, const c64* __restrict__ coef, const uint64_t* __restrict__ hitab,
+// Two states (adjoint), dense ops of at most 2 qubits.
+template <bool kLat>
+__global__ void __launch_bounds__(kMaxTileThreads, kLat ? 2 : 4)
+k_sweep2(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo sw, const SweepIO* __restrict__ io, SVMI_TABLES,
          double* __restrict__ grad_partials, uint64_t tile_offset)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    sweep_tile<2, false>(s0, s1, sw, phases, ops, coef, hitab, grad_partials, tile_offset + blockIdx.x, blockDim.x,
-                         smem, false);
+    sweep_tile<2, kMaxDenseQubitsAdj, kLat>(s0, s1, sw, io, SVMI_TABLE_ARGS, grad_partials, tile_offset + blockIdx.x,
+                                            smem, false);
 }
 
+constexpr uint64_t kLatTiles = 256;   // sweeps of at most this many tiles run the latency builds
 static size_t g_max_smem = 64 * 1024;  // dynamic LDS the sweep kernels may use
 
 // --------------------------------------------------------------- batching
@@ -407,37 +351,36 @@ __device__ inline uint32_t batch_step_of(const BatchStep* __restrict__ steps, ui
     return lo;
 }
 
-// Read-only program tables of a batch, as restrict kernel arguments so the
-// tile code reads op headers through the scalar path as k_sweep does.
-#define SVMI_BATCH_TABLES                                                                            \
-    const BatchStep* __restrict__ steps, const BatchCircuit* __restrict__ circuits,                  \
-        const SweepInfo* __restrict__ sweeps, const PhaseInfo* __restrict__ phases,                 \
-        const DOp* __restrict__ ops, const c64* __restrict__ coef, const uint64_t* __restrict__ hitab
+#define SVMI_BATCH_TABLES                                                                           \
+    const BatchStep *__restrict__ steps, const BatchCircuit *__restrict__ circuits,                 \
+        const SweepInfo *__restrict__ sweeps, const SweepIO *__restrict__ ios
 
 // kInit: the steps are first forward sweeps (tiles generated as |0..0>).
-// kMap: some of the launch's sweeps have tile maps.
-template <bool kInit, int kMaxQ, bool kMap>
-__global__ void __launch_bounds__(kMaxTileThreads, 1)
-k_batch_fwd(SVMI_BATCH_TABLES, uint32_t s0, uint32_t s1, uint64_t task0)
+template <bool kInit, int kMaxQ>
+__global__ void __launch_bounds__(kMaxTileThreads, kSweepWaves<kMaxQ>)
+k_batch_fwd(SVMI_BATCH_TABLES, SVMI_TABLES, uint32_t s0, uint32_t s1, uint64_t task0)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint64_t t = task0 + blockIdx.x;
     const BatchStep st = steps[batch_step_of(steps, s0, s1, t)];
     const SweepInfo sw = sweeps[st.sweep];
-    sweep_tile<1, false, kMaxQ, kMap>(circuits[st.circuit].phi, nullptr, sw, phases, ops, coef, hitab, nullptr,
-                         t - st.task_begin, blockDim.x, smem, kInit);
+    const SweepIO* __restrict__ io = ios + st.sweep;
+    sweep_tile<1, kMaxQ>(circuits[st.circuit].phi, nullptr, sw, io, SVMI_TABLE_ARGS, nullptr, t - st.task_begin, smem,
+                         kInit);
 }
 
-__global__ void __launch_bounds__(kThreads, 1)
-k_batch_adj(SVMI_BATCH_TABLES, double* __restrict__ grad_partials, uint32_t s0, uint32_t s1, uint64_t task0)
+__global__ void __launch_bounds__(kMaxTileThreads, 4)
+k_batch_adj(SVMI_BATCH_TABLES, SVMI_TABLES, double* __restrict__ grad_partials, uint32_t s0, uint32_t s1,
+            uint64_t task0)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint64_t t = task0 + blockIdx.x;
     const BatchStep st = steps[batch_step_of(steps, s0, s1, t)];
     const SweepInfo sw = sweeps[st.sweep];
+    const SweepIO* __restrict__ io = ios + st.sweep;
     const BatchCircuit& c = circuits[st.circuit];
-    sweep_tile<2, false>(c.phi, c.lam, sw, phases, ops, coef, hitab, grad_partials + st.partial, t - st.task_begin,
-                         blockDim.x, smem, false);
+    sweep_tile<2, kMaxDenseQubitsAdj>(c.phi, c.lam, sw, io, SVMI_TABLE_ARGS, grad_partials + st.partial,
+                                      t - st.task_begin, smem, false);
 }
 
 // ------------------------------------------------------------- Pauli sums
@@ -615,26 +558,20 @@ k_batch_pauli(BatchArgs a, uint32_t s0, uint32_t s1, uint64_t task0)
 
 size_t batch_launch_smem(uint32_t kind, uint32_t k, uint32_t max_grad, uint32_t max_xf)
 {
-    if (kind == BSTEP_FWD) return (size_t(16) << k) + size_t(16) * max_xf;
-    if (kind == BSTEP_ADJ) {
-        const size_t nwaves = (size_t(sweep_threads(k, 2)) + 63) / 64;
-        return (size_t(32) << k) + size_t(16) * max_xf + size_t(8) * max_grad * nwaves;
-    }
-    return kind == BSTEP_PAULI ? size_t(16) * kPauliChunk : 0;
+    if (kind != BSTEP_FWD && kind != BSTEP_ADJ) return size_t(16) * kPauliChunk;
+    SweepInfo sw;   // the largest of the launch's sweeps
+    sw.k = k;
+    sw.n_xf = max_xf;
+    sw.n_grad = kind == BSTEP_ADJ ? max_grad : 0;
+    return sweep_smem_bytes(sw, kind == BSTEP_ADJ ? 2 : 1);
 }
 
 // The k_batch_fwd build of a forward launch.
-using BatchFwdFn = void (*)(const BatchStep*, const BatchCircuit*, const SweepInfo*, const PhaseInfo*, const DOp*,
-                            const c64*, const uint64_t*, uint32_t, uint32_t, uint64_t);
-template <bool kInit, bool kMap>
-BatchFwdFn batch_fwd_kernel_of(const BatchLaunch& L)
-{
-    return L.max_dense <= 2 ? &k_batch_fwd<kInit, 2, kMap> : &k_batch_fwd<kInit, kRegBits, kMap>;
-}
+using BatchFwdFn = void (*)(SVMI_BATCH_TABLES, SVMI_TABLES, uint32_t, uint32_t, uint64_t);
 BatchFwdFn batch_fwd_kernel(const BatchLaunch& L)
 {
-    if (L.init) return L.mapped ? batch_fwd_kernel_of<true, true>(L) : batch_fwd_kernel_of<true, false>(L);
-    return L.mapped ? batch_fwd_kernel_of<false, true>(L) : batch_fwd_kernel_of<false, false>(L);
+    if (L.init) return L.max_dense <= 2 ? &k_batch_fwd<true, 2> : &k_batch_fwd<true, kRegBits>;
+    return L.max_dense <= 2 ? &k_batch_fwd<false, 2> : &k_batch_fwd<false, kRegBits>;
 }
 
 hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L)
@@ -651,13 +588,13 @@ hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L
         switch (L.kind) {
         case BSTEP_FWD: {
             auto* fn = batch_fwd_kernel(L);
-            hipLaunchKernelGGL(fn, dim3(cnt), dim3(threads), smem, st, a.steps, a.circuits, a.sweeps, a.phases,
-                               a.ops, a.coef, a.hitab, L.step_begin, L.step_end, first);
+            hipLaunchKernelGGL(fn, dim3(cnt), dim3(threads), smem, st, a.steps, a.circuits, a.sweeps, a.io,
+                               SVMI_TABLES_OF(a.t), L.step_begin, L.step_end, first);
             break;
         }
         case BSTEP_ADJ:
-            hipLaunchKernelGGL(k_batch_adj, dim3(cnt), dim3(threads), smem, st, a.steps, a.circuits, a.sweeps,
-                               a.phases, a.ops, a.coef, a.hitab, a.grad_partials, L.step_begin, L.step_end, first);
+            hipLaunchKernelGGL(k_batch_adj, dim3(cnt), dim3(threads), smem, st, a.steps, a.circuits, a.sweeps, a.io,
+                               SVMI_TABLES_OF(a.t), a.grad_partials, L.step_begin, L.step_end, first);
             break;
         case BSTEP_PAULI:
             hipLaunchKernelGGL(k_batch_pauli, dim3(cnt), dim3(threads), smem, st, a, L.step_begin, L.step_end, first);
@@ -669,100 +606,27 @@ hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L
     return hipGetLastError();
 }
 
-size_t sweep_smem_bytes(const SweepInfo& sw, int ns)
-{
-    const size_t nt = sweep_threads(sw.k, ns);
-    const size_t nwaves = (nt + 63) / 64;
-    return (size_t(16) << sw.k) * ns + size_t(16) * sw.n_xf + size_t(8) * sw.n_grad * nwaves;
-}
-
-// Workgroups of k_sweep1p resident at once for tile size k (occupancy x CUs).
-template <bool kWide>
-static uint64_t pipeline_grid(uint32_t k)
-{
-    static uint64_t cache[kMaxTileQubits + 1] = {};
-    if (cache[k]) return cache[k];
-    int dev = 0, cus = 0, per = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-        cus = 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(&k_sweep1p<kWide>),
-                                                     1 << (k - kRegBits), size_t(16) << k) != hipSuccess ||
-        per < 1)
-        per = 1;
-    (void)hipGetLastError();
-    cache[k] = uint64_t(cus) * uint64_t(per);
-    return cache[k];
-}
-
-// Workgroups of k_sweep1d resident at once (CUs x occupancy at the largest
-// LDS it may use; 0 if it cannot run).
-static uint64_t dma_grid()
-{
-    static uint64_t cache = ~0ull;
-    if (cache != ~0ull) return cache;
-    int dev = 0, cus = 0, per = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1 ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(&k_sweep1d<kRegBits>),
-                                                     int(kDmaThreads), g_max_smem) != hipSuccess)
-        per = 0;
-    (void)hipGetLastError();
-    cache = per > 0 ? uint64_t(cus) * uint64_t(per) : 0;
-    return cache;
-}
-
-hipError_t launch_sweep(hipStream_t st, int ns, c64* s0, c64* s1, const SweepInfo& sw,
-                        const PhaseInfo* phases, const DOp* ops, const c64* coef,
-                        const uint64_t* hitab, double* grad_partials, int pipeline, bool prefetch)
+hipError_t launch_sweep(hipStream_t st, int ns, c64* s0, c64* s1, const SweepInfo& sw, const SweepIO* io,
+                        const SweepTables& t, double* grad_partials)
 {
     const uint32_t nt = sweep_threads(sw.k, ns);
-    const size_t smem = sweep_smem_bytes(sw, ns);
-    if (smem > g_max_smem) return hipErrorInvalidConfiguration;
-    // sweeps with tile maps run on k_sweep1's mapped build only
-    if (ns == 1 && sw.mapped) pipeline = 0, prefetch = false;
-    if (ns == 1 && prefetch && pipeline == 0 && sw.k == kDmaTileQubits && nt == kDmaThreads &&
-        dma_sweep_smem_bytes(sw) <= g_max_smem) {
-        const uint64_t grid = dma_grid();
-        if (grid && sw.n_tiles >= 2 * grid) {
-            hipLaunchKernelGGL(sw.max_dense <= 2 ? k_sweep1d<2> : k_sweep1d<kRegBits>, dim3(uint32_t(grid)),
-                               dim3(kDmaThreads), dma_sweep_smem_bytes(sw), st, s0, sw, phases, ops, coef, hitab);
-            return hipGetLastError();
-        }
-    }
-    if (ns == 1 && (pipeline == 1 || pipeline == 2)) {
-        const bool wide = pipeline == 2 && nt <= 256;
-        const uint64_t resident = wide ? pipeline_grid<true>(sw.k) : pipeline_grid<false>(sw.k);
-        if (sw.n_tiles > resident) {
-            if (wide)
-                hipLaunchKernelGGL(k_sweep1p<true>, dim3(uint32_t(resident)), dim3(nt), smem, st, s0, sw, phases, ops,
-                                   coef, hitab, uint64_t(0), sw.n_tiles);
-            else
-                hipLaunchKernelGGL(k_sweep1p<false>, dim3(uint32_t(resident)), dim3(nt), smem, st, s0, sw, phases,
-                                   ops, coef, hitab, uint64_t(0), sw.n_tiles);
-            return hipGetLastError();
-        }
-    }
+    size_t smem = sweep_smem_bytes(sw, ns);
+    // at most one tile per CU (256): the latency build, if the phases'
+    // coefficients fit its stage (blocks of three and four register qubits
+    // from LDS would not fit its registers)
+    const bool lat = sw.max_dense <= 2 && sw.n_tiles <= kLatTiles && sw.stage <= kMaxStage && smem + 8 + 32 * sw.stage <= g_max_smem;
+    if (lat) smem += 8 + 32 * sw.stage;
+    if (smem > g_max_smem || nt > uint32_t(kMaxTileThreads)) return hipErrorInvalidConfiguration;
     const uint64_t max_grid = 1ull << 30;
     for (uint64_t t0 = 0; t0 < sw.n_tiles; t0 += max_grid) {
         const uint64_t cnt = sw.n_tiles - t0 < max_grid ? sw.n_tiles - t0 : max_grid;
         if (ns == 1) {
-            // pipeline 3: stagger the second workgroup slot of every CU
-            uint32_t lo = 0, hi = 0, sl = 0;
-            if (pipeline >= 3) {
-                const uint64_t res = pipeline_grid<false>(sw.k);
-                lo = uint32_t(res / 2);
-                hi = uint32_t(res);
-                sl = uint32_t(pipeline - 2);
-            }
-            auto* fn = sw.mapped ? (sw.max_dense <= 2 ? &k_sweep1<2, true> : &k_sweep1<kRegBits, true>)
-                                 : (sw.max_dense <= 2 ? &k_sweep1<2, false> : &k_sweep1<kRegBits, false>);
-            hipLaunchKernelGGL(fn, dim3(uint32_t(cnt)), dim3(nt), smem, st, s0, sw, phases, ops, coef, hitab, t0, lo,
-                               hi, sl);
+            auto* fn = lat ? &k_sweep1<2, true> : sw.max_dense <= 2 ? &k_sweep1<2, false> : &k_sweep1<kRegBits, false>;
+            hipLaunchKernelGGL(fn, dim3(uint32_t(cnt)), dim3(nt), smem, st, s0, sw, io, SVMI_TABLES_OF(t), t0);
+        } else {
+            hipLaunchKernelGGL(lat ? &k_sweep2<true> : &k_sweep2<false>, dim3(uint32_t(cnt)), dim3(nt), smem, st, s0,
+                               s1, sw, io, SVMI_TABLES_OF(t), grad_partials, t0);
         }
-        else
-            hipLaunchKernelGGL(k_sweep2, dim3(uint32_t(cnt)), dim3(nt), smem, st, s0, s1, sw, phases, ops,
-                               coef, hitab, grad_partials, t0);
     }
     return hipGetLastError();
 }
@@ -781,51 +645,19 @@ hipError_t init_sweep_kernels()
         optin = 64 * 1024;
     size_t want = size_t(optin);
     if (want > 160 * 1024) want = 160 * 1024;
-    if (want > 64 * 1024) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1<kRegBits, false>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1<2, false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1<kRegBits, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1<2, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1p<false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1p<true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1d<kRegBits>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep1d<2>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep2),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(want));
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            want = 64 * 1024;
-        }
-    }
-    auto raise = [&](const void* fn) {
+    const auto raise = [&](const void* fn) {
         return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(want)) == hipSuccess;
     };
     if (want > 64 * 1024 &&
-        !(raise(reinterpret_cast<const void*>(&k_batch_fwd<true, kRegBits, false>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, kRegBits, false>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, 2, false>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, 2, false>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, kRegBits, true>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, kRegBits, true>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, 2, true>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, 2, true>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_adj)))) {
+        !(raise(reinterpret_cast<const void*>(&k_sweep1<2, false>)) &&
+          raise(reinterpret_cast<const void*>(&k_sweep1<kRegBits, false>)) &&
+          raise(reinterpret_cast<const void*>(&k_sweep1<2, true>)) &&
+          raise(reinterpret_cast<const void*>(&k_sweep2<false>)) &&
+          raise(reinterpret_cast<const void*>(&k_sweep2<true>)) && raise(reinterpret_cast<const void*>(&k_batch_adj)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, 2>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, 2>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, kRegBits>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, kRegBits>)))) {
         (void)hipGetLastError();
         want = 64 * 1024;
     }

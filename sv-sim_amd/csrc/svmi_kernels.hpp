@@ -63,14 +63,21 @@ struct BatchCircuit {
     uint32_t slot_begin, n_slots;      // gradient accumulators (global numbering)
 };
 
+// Device tables of a program's sweeps.
+struct SweepTables {
+    const LayoutPhase* lphases;
+    const uint64_t* lane_tab;
+    const uint64_t* wave_tab;
+    const DOp* ops;
+    const c64* coef;
+};
+
 struct BatchArgs {
     const BatchStep* steps;
     const BatchCircuit* circuits;
     const SweepInfo* sweeps;
-    const PhaseInfo* phases;
-    const DOp* ops;
-    const c64* coef;
-    const uint64_t* hitab;
+    const SweepIO* io;
+    SweepTables t;
     const PauliGroup* groups;
     const PauliTerm* terms;
     double* e_partials;
@@ -89,7 +96,6 @@ struct BatchLaunch {
     uint32_t init;          // FWD: first sweeps (tiles start as |0..0>)
     uint32_t max_xf;        // largest n_xf of the group's sweeps
     uint32_t max_dense;     // FWD: widest dense block of the group's sweeps
-    uint32_t mapped;        // FWD: some of the group's sweeps have tile maps
     uint64_t task_begin, n_tasks;
 };
 size_t batch_launch_smem(uint32_t kind, uint32_t k, uint32_t max_grad, uint32_t max_xf);
@@ -99,13 +105,8 @@ hipError_t init_sweep_kernels();
 hipError_t init_sample_kernels();   // after init_sweep_kernels
 size_t sweep_smem_limit();
 size_t sweep_smem_bytes(const SweepInfo& sw, int ns);
-// pipeline != 0: one-state sweeps larger than one resident grid run
-// persistent and prefetch the next tile (k_sweep1p); 2 = 512-VGPR variant.
-// prefetch (with pipeline 0): one-state sweeps of 12-qubit tiles over at
-// least two resident grids run k_sweep1d (double-buffered LDS DMA).
-hipError_t launch_sweep(hipStream_t st, int ns, c64* s0, c64* s1, const SweepInfo& sw,
-                        const PhaseInfo* phases, const DOp* ops, const c64* coef,
-                        const uint64_t* hitab, double* grad_partials, int pipeline, bool prefetch);
+hipError_t launch_sweep(hipStream_t st, int ns, c64* s0, c64* s1, const SweepInfo& sw, const SweepIO* io /* device */,
+                        const SweepTables& t, double* grad_partials);
 hipError_t launch_standalone(hipStream_t st, c64* s, int n, const StandaloneOp& so, const c64* coef);
 hipError_t launch_fill_basis(hipStream_t st, c64* s, uint64_t dim);
 hipError_t launch_gather(hipStream_t st, const c64* s, uint64_t dim, const uint64_t* idx, uint64_t cnt, c64* out);

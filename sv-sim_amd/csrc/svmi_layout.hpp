@@ -1,0 +1,11 @@
+// svmi_layout.hpp -- register layouts of planned sweeps (host only).
+#pragma once
+
+#include "svmi_plan.hpp"
+
+namespace svmi {
+
+// Fills prog.io, lphases, lane_tab and wave_tab for every sweep of prog.
+void build_layouts(Program& prog);
+
+}  // namespace svmi

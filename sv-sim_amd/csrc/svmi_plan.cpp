@@ -10,6 +10,7 @@
 //   bits R instead of T.
 // Every sweep is one read and one write of the whole state.
 #include "svmi_plan.hpp"
+#include "svmi_layout.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -317,6 +318,75 @@ struct Encoder {
 
     // Encode op for a phase: tloc[p] = tile-local bit of physical qubit p (or -1),
     // slot_of[l] = register slot of local bit l (or -1).
+    // M (2^k x 2^k, k <= 2) -> its factors as apply_dense takes them.  Columns
+    // are exchanged where a diagonal entry is less than half of its row's
+    // largest, and the exchange -- every permutation of two or four
+    // amplitudes is a product of CX, SWAP and X -- is emitted before the op.
+    void factor_dense(std::vector<c64>& M, int k, uint32_t smask)
+    {
+        const int D = 1 << k;
+        int perm[4] = {0, 1, 2, 3};
+        for (int i = 0; i < D; i++) {
+            const auto size = [&](int c) { return std::hypot(M[i * D + c].re, M[i * D + c].im); };
+            int p = i;
+            for (int c = i + 1; c < D; c++)
+                if (size(c) > size(p)) p = c;
+            if (p != i && size(i) < 0.5 * size(p)) {
+                for (int r = 0; r < D; r++) std::swap(M[r * D + i], M[r * D + p]);
+                std::swap(perm[i], perm[p]);
+            }
+            const c64 d = M[i * D + i];
+            const double n2 = d.re * d.re + d.im * d.im;
+            for (int c = i + 1; c < D; c++) {
+                c64& u = M[i * D + c];
+                if (n2 == 0.0) {   // the whole row is zero
+                    u = c64{0.0, 0.0};
+                    continue;
+                }
+                const c64 t = cmul(u, c64{d.re, -d.im});
+                u = c64{t.re / n2, t.im / n2};
+                for (int r = i + 1; r < D; r++) {
+                    const c64 w = cmul(M[r * D + i], u);
+                    M[r * D + c] = c64{M[r * D + c].re - w.re, M[r * D + c].im - w.im};
+                }
+            }
+        }
+        const uint32_t s0 = uint32_t(__builtin_ctz(smask)), s1 = k == 2 ? uint32_t(31 - __builtin_clz(smask)) : s0;
+        DOp d;
+        std::memset(&d, 0, sizeof(d));
+        d.targets = prog.n_states == 2 ? DOP_TO_BOTH : DOP_TO_PSI;
+        const auto put = [&](uint32_t type, uint32_t a, uint32_t b) {
+            d.h.type = type;
+            d.h.s0 = a;
+            d.h.s1 = b;
+            prog.ops.push_back(d);
+        };
+        // up to two of CX(0, 1), CX(1, 0), SWAP, then X on either bit
+        for (int seq = 0; seq < (k == 2 ? 16 : 1); seq++)
+            for (int x = 0; x < D; x++) {
+                int v[4] = {0, 1, 2, 3};
+                const auto run = [&](int kind) {
+                    if (kind == 1) std::swap(v[1], v[3]);
+                    if (kind == 2) std::swap(v[2], v[3]);
+                    if (kind == 3) std::swap(v[1], v[2]);
+                };
+                run(seq & 3);
+                run(seq >> 2);
+                bool same = true;
+                for (int r = 0; r < D; r++) same = same && v[r ^ x] == perm[r];
+                if (!same) continue;
+                for (int kind : {seq & 3, seq >> 2}) {
+                    if (kind == 1) put(DOP_CX, s0, s1);
+                    if (kind == 2) put(DOP_CX, s1, s0);
+                    if (kind == 3) put(DOP_SWAP, s0, s1);
+                }
+                if (x & 1) put(DOP_X, s0, 0);
+                if (x & 2) put(DOP_X, s1, 0);
+                return;
+            }
+        throw std::logic_error("dense op: column order");
+    }
+
     void encode(const SOp& s, const int* tloc, const int* slot_of, uint32_t grad_slot)
     {
         const LOp& op = *s.op;
@@ -436,6 +506,7 @@ struct Encoder {
         d.h.type = s.grad ? DOP_GRAD_DENSE : DOP_DENSE;
         d.h.smask = 0;
         for (int i = 0; i < op.k; i++) d.h.smask |= 1u << slots[i];
+        if (!s.grad && op.k <= 2) factor_dense(M, op.k, d.h.smask);
         d.h.coef = s.grad ? push_grad_coef(M) : push_coef(M);
         if (s.grad) d.h.s0 = nonzero_mask(d.h.coef, uint32_t(D * D));
         prog.ops.push_back(d);
@@ -1210,7 +1281,6 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
     sw.c = uint32_t(c);
     sw.phase_begin = uint32_t(prog.phases.size());
     sw.op_begin = uint32_t(prog.ops.size());
-    sw.hitab = uint32_t(prog.hitab.size());
     sw.n_ext = 0;
     sw.extmask = 0;
     for (int p = 0; p < n; p++)
@@ -1219,12 +1289,6 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
             sw.n_ext++;
         }
     sw.n_tiles = uint64_t(1) << (n - k);
-    for (uint64_t h = 0; h < (uint64_t(1) << (k - c)); h++) {
-        uint64_t off = 0;
-        for (int j = 0; j < k - c; j++)
-            if ((h >> j) & 1) off |= uint64_t(1) << tpos[c + j];
-        prog.hitab.push_back(off);
-    }
     sw.grad_base = prog.n_grad;
 
     // phase scheduling: pick the register bits R of each phase by a small
@@ -1393,6 +1457,7 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
             rm.flush();
         }
         pi.op_begin = uint32_t(prog.ops.size());
+        pi.coef_begin = uint32_t(prog.coef.size());
         if (opt.rotations) {
             const bool two = prog.n_states == 2;
             std::vector<const SOp*> merged_rot;
@@ -1466,6 +1531,7 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
             enc.encode(*s, tloc, slot_of, gslot);
         }
         pi.op_end = uint32_t(prog.ops.size());
+        pi.coef_end = uint32_t(prog.coef.size());
         const uint32_t ops0 = pi.op_begin;
         fold_leading_permutations(prog, pi);
         if (fold_map && pi.op_begin == pi.op_end && pi.gxor == 0 && pi.sxor == 0) {
@@ -1707,6 +1773,7 @@ void build_forward_program(const std::vector<LOp>& ops, int n, const PlanOptions
     sops.reserve(ops.size());
     for (const LOp& op : ops) sops.push_back(make_sop(&op, false, -1));
     schedule(sops, n, opt, prog);
+    build_layouts(prog);
 }
 
 void build_segmented_program(const std::vector<std::vector<LOp>>& segments, const std::vector<MeasureStep>& measures,
@@ -1729,6 +1796,7 @@ void build_segmented_program(const std::vector<std::vector<LOp>>& segments, cons
     }
     for (const MeasureStep& m : prog.measures)
         if (m.coef == UINT32_MAX) throw std::logic_error("measurement without a collapse op");
+    build_layouts(prog);
 }
 
 void build_adjoint_program(const std::vector<AdjEntry>& entries, int n, const PlanOptions& opt,
@@ -1742,6 +1810,17 @@ void build_adjoint_program(const std::vector<AdjEntry>& entries, int n, const Pl
     PlanOptions o = opt;
     o.fusion = true;  // adjoint always runs as tiled sweeps
     schedule(sops, n, o, prog);
+    build_layouts(prog);
+}
+
+void build_row_tables(Program& prog)
+{
+    prog.hitab.clear();
+    for (SweepInfo& sw : prog.sweeps) {
+        sw.hitab = uint32_t(prog.hitab.size());
+        const uint64_t tile = ((uint64_t(1) << prog.n) - 1) & ~sw.extmask & ~((uint64_t(1) << sw.c) - 1);
+        for (uint64_t h = 0; h < (uint64_t(1) << (sw.k - sw.c)); h++) prog.hitab.push_back(deposit_bits(h, tile));
+    }
 }
 
 // FP64 multiply-adds per amplitude the program's state ops execute (a
