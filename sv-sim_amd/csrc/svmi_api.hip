@@ -178,7 +178,7 @@ struct DevBuf {
 struct DeviceProgram {
     DevBuf buf;
     std::vector<unsigned char> host;   // the copy's source, until the upload's synchronisation
-    size_t o_ops = 0, o_coef = 0, o_lph = 0, o_lane = 0, o_wave = 0, o_io = 0, o_hitab = 0;
+    size_t o_ops = 0, o_coef = 0, o_lph = 0, o_lane = 0, o_wave = 0, o_io = 0;
     template <class T>
     size_t put(const std::vector<T>& v, size_t pad = 0)
     {
@@ -187,8 +187,7 @@ struct DeviceProgram {
         if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
         return at;
     }
-    // hitab: the tile-row tables, which only compiled sweeps read
-    svmi_status upload(const Program& p, hipStream_t st, bool hitab = false)
+    svmi_status upload(const Program& p, hipStream_t st)
     {
         host.clear();
         // op arrays end with an unused record: the latency builds read the
@@ -199,7 +198,6 @@ struct DeviceProgram {
         o_lane = put(p.lane_tab, 16);
         o_wave = put(p.wave_tab, 16);
         o_io = put(p.io, 16);
-        if (hitab) o_hitab = put(p.hitab, 16);
         SVMI_TRY(buf.ensure(host.size()));
         SVMI_HIP(hipMemcpyAsync(buf.p, host.data(), host.size(), hipMemcpyHostToDevice, st));
         SVMI_HIP(hipStreamSynchronize(st));
@@ -209,7 +207,6 @@ struct DeviceProgram {
     T* at(size_t off) const { return reinterpret_cast<T*>(static_cast<unsigned char*>(buf.p) + off); }
     c64* coef() const { return at<c64>(o_coef); }
     const SweepIO* io() const { return at<SweepIO>(o_io); }
-    uint64_t* hitab() const { return at<uint64_t>(o_hitab); }
     SweepTables tables() const
     {
         return SweepTables{at<LayoutPhase>(o_lph), at<uint64_t>(o_lane), at<uint64_t>(o_wave), at<DOp>(o_ops), coef()};
@@ -735,7 +732,6 @@ struct svmi_sim {
     std::string jit_error;     // why the last specialisation failed (the sweeps then interpret)
     PlanOptions opt;
     bool profile = false;
-    bool prefetch = false;     // SVMI_OPT_PREFETCH
     hipEvent_t io_ev[4] = {};      // set_state / get_state: a worker's copy is done
     std::vector<hipEvent_t> prof_events;
     std::vector<double> step_ms;   // with profiling: per-step times of the last program run
@@ -821,7 +817,7 @@ svmi_status exec_program(svmi_handle h, const Program& prog, DeviceProgram& dp, 
                 partials = h->scratch[5].as<double>();
             }
             if (jit && st.index < jit->fn.size() && jit->fn[st.index])
-                SVMI_HIP(jit_launch(h->stream, *jit, st.index, sw, s0, dp.coef(), dp.hitab()));
+                SVMI_HIP(jit_launch(h->stream, *jit, st.index, sw, s0, dp.tables()));
             else
                 SVMI_HIP(launch_sweep(h->stream, prog.n_states, s0, s1, sw, dp.io() + st.index, dp.tables(), partials));
             if (partials && !combined)
@@ -1181,34 +1177,42 @@ void default_tile(svmi_handle h, int n, bool two, PlanOptions& o)
 
 // Planner options of the forward program.  Specialised sweeps pay almost
 // nothing per op (no dispatch), so unless the caller set an op cost their
-// fusion model counts FMAs only: 20-layer u3 brick-wall at 30 qubits 300 ->
-// 258 ms per circuit; the interpreted sweeps are fastest at the default 2.
+// fusion model counts FMAs only (the u3 brickwall and the random layers of 27
+// qubits take the same 15.8 and 32.6 ms with the interpreted sweeps' 2).
+//
+// Compiled sweeps keep tiles of 12 qubits, and from 20 qubits on 3 low ones
+// where the tile is the default (QFT of 27 qubits 4.38 -> 4.16 ms, u3
+// brickwall of 27, 20 layers, 17.1 -> 16.0 ms).  They use tile maps only below
+// 20 qubits: there a phase less shows (QFT of 16 qubits 25.4 -> 21.7 us), while
+// a sweep of a large state is bound by its pass over memory (QFT of 27 qubits
+// 4.16 ms without, 4.26 ms with maps).
+constexpr int kJitLargeQubits = 20;
+
 PlanOptions forward_options(svmi_handle h)
 {
     PlanOptions o = h->opt;
-    if (!h->specialize) default_tile(h, h->n_int, false, o);
-    if (h->specialize && !h->op_cost_set) o.op_overhead = 0;
-    if (h->specialize) o.tile_map = false;   // the compiled sweeps address LDS without maps
+    if (!h->specialize) {
+        default_tile(h, h->n_int, false, o);
+        return o;
+    }
+    if (!h->op_cost_set) o.op_overhead = 0;
+    if (h->n_int >= kJitLargeQubits) {
+        if (!h->low_set && !h->tile_set) o.low_qubits = 3;
+        o.tile_map = false;
+    }
     return o;
 }
 
 // Device copy of h->prog and, with SVMI_OPT_SPECIALIZE, its compiled sweeps.
 svmi_status install_program(svmi_handle h)
 {
-    if (h->specialize) build_row_tables(h->prog);
-    SVMI_TRY(h->dprog.upload(h->prog, h->stream, h->specialize));
+    SVMI_TRY(h->dprog.upload(h->prog, h->stream));
     h->jit.release();
     h->jit_error.clear();
     h->stats.specialized_sweeps = 0;
     h->stats.compile_ms = 0.0;
     if (!h->specialize) return SVMI_OK;
-    uint64_t dma_grid = 0;   // SVMI_OPT_PREFETCH: double-buffered kernels, one workgroup per CU
-    if (h->prefetch) {
-        int cus = 0;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) == hipSuccess && cus > 0)
-            dma_grid = uint64_t(cus);
-    }
-    if (!jit_build(h->prog, device_arch().c_str(), h->jit, h->jit_error, dma_grid)) {
+    if (!jit_build(h->prog, device_arch().c_str(), h->jit, h->jit_error)) {
         h->jit.release();
         // the sweeps are interpreted; the reason stays readable
         if (!h->jit_error.empty()) g_err = "specialisation: " + h->jit_error;
@@ -1724,7 +1728,7 @@ svmi_status svmi_set_option(svmi_handle h, int option, int64_t value)
     case SVMI_OPT_PIPELINE:
         if (value < 0 || value > 64) return fail(SVMI_ERR_ARG, "pipeline must be in [0, 64]");
         return SVMI_OK;
-    case SVMI_OPT_PREFETCH: h->prefetch = value != 0; return SVMI_OK;
+    case SVMI_OPT_PREFETCH: return SVMI_OK;   // no effect
     case SVMI_OPT_SPECIALIZE: h->specialize = value != 0; break;
     case SVMI_OPT_MERGE_QUBITS:
         if (value < 1 || value > kRegBits) return fail(SVMI_ERR_ARG, "merge qubits must be in [1, 4]");
@@ -2158,12 +2162,10 @@ svmi_status svmi_debug_jit(int n, const svmi_gate* gates, size_t n_gates, int ti
     SVMI_TRY(check_gates(gates, n_gates, n));
     Program prog;
     PlanOptions o = debug_options(1, tile_qubits, low_qubits, 0);
-    o.tile_map = false;   // as SVMI_OPT_SPECIALIZE plans
+    o.tile_map = n < kJitLargeQubits;   // as SVMI_OPT_SPECIALIZE plans
     plan_forward(gates, n_gates, std::max(n, kRegBits), o, prog);
-    build_row_tables(prog);
     std::vector<char> covered;
-    const uint64_t dma_grid = compile == 2 ? 256 : 0;   // double-buffered kernels for a 256-CU device
-    const std::string src = jit_source(prog, covered, dma_grid);
+    const std::string src = jit_source(prog, covered);
     if (buf && buflen) {
         const size_t m = std::min(buflen - 1, src.size());
         std::memcpy(buf, src.data(), m);
@@ -2172,7 +2174,7 @@ svmi_status svmi_debug_jit(int n, const svmi_gate* gates, size_t n_gates, int ti
     if (compile) {
         std::string err;
         double ms = 0.0;
-        const size_t bytes = jit_compile_only(prog, "gfx950", &ms, err, dma_grid);
+        const size_t bytes = jit_compile_only(prog, "gfx950", &ms, err);
         if (!bytes) return fail(SVMI_ERR_UNSUPPORTED, "jit: " + err);
         if (compile_ms) *compile_ms = ms;
         if (code_bytes) *code_bytes = bytes;

@@ -18,13 +18,7 @@ extern const int kJitHeaderCount;
 
 namespace {
 
-constexpr uint32_t kJitMaxTileQubits = 12;   // static LDS of one tile: 64 KiB
-
-void emit_hdr(std::ostringstream& o, const DOpHdr& h)
-{
-    o << "{" << h.type << "u, " << h.smask << "u, " << h.s0 << "u, " << h.s1 << "u, " << h.coef << "u, " << h.grad
-      << "u, " << h.rsel << "u, " << h.gmask << "u, " << h.emask << "ull}";
-}
+constexpr uint32_t kJitMaxTileQubits = 12;   // wider tiles are interpreted
 
 // Registers r (0..15) whose register bits satisfy `rsel`, as a list.
 std::vector<int> selected(uint32_t rsel)
@@ -36,17 +30,24 @@ std::vector<int> selected(uint32_t rsel)
 }
 
 // Tile-local offset of register r in phase ph (the register bits' part).
-uint32_t reg_offset(const PhaseInfo& ph, int r)
+uint32_t reg_offset(const LayoutPhase& ph, int r)
 {
     uint32_t o = 0;
     for (int b = 0; b < kRegBits; b++)
-        if ((r >> b) & 1) o |= 1u << ph.r[b];
+        if ((r >> b) & 1) o |= ph.rcol[b];
     return o;
+}
+
+// The variant of a register table over the qubits `emask` outside the tile.
+std::string variant(uint64_t emask, const SweepInfo& sw)
+{
+    if (!emask) return "0u";
+    return emask == sw.exthi ? "vhi" : "rtab_variant(" + std::to_string(emask) + "ull, base)";
 }
 
 // One op as direct code: the templates of svmi_exec.hpp / svmi_internal.hpp
 // with every slot, mask and offset a literal, so no dispatch is compiled.
-void emit_state_op(std::ostringstream& o, const DOp& d, const PhaseInfo& ph)
+void emit_state_op(std::ostringstream& o, const DOp& d, const LayoutPhase& ph, const SweepInfo& sw)
 {
     const DOpHdr& h = d.h;
     const std::string cond = "(base & " + std::to_string(h.emask) + "ull) == " + std::to_string(h.emask) +
@@ -63,11 +64,11 @@ void emit_state_op(std::ostringstream& o, const DOp& d, const PhaseInfo& ph)
           << h.coef << "].re, coef[" << h.coef << "].im);\n";
         return;
     case DOP_RTAB:
-        o << "        apply_rtab(a, coef + " << h.coef << "u + 16u * rtab_variant(" << h.emask << "ull, base));\n";
+        o << "        apply_rtab(a, coef + " << h.coef << "u + 16u * " << variant(h.emask, sw) << ");\n";
         return;
     case DOP_ROT:
         if (h.s0)
-            o << "        apply_rtab(a, coef + " << h.grad << "u + 16u * rtab_variant(" << h.emask << "ull, base));\n";
+            o << "        apply_rtab(a, coef + " << h.grad << "u + 16u * " << variant(h.emask, sw) << ");\n";
         for (int sl = 0; sl < kRegBits; sl++)
             if ((h.smask >> sl) & 1u)
                 o << "        apply_lift<" << sl << ", " << (((h.s1 >> sl) & 1u) ? "true" : "false") << ">(a, coef["
@@ -91,7 +92,7 @@ void emit_state_op(std::ostringstream& o, const DOp& d, const PhaseInfo& ph)
             if (d.qloc[i] < 0) o << " | (uint32_t((base >> " << d.qphys[i] << ") & 1u) << " << i << ")";
             else {
                 bool reg = false;
-                for (int b = 0; b < kRegBits; b++) reg = reg || int(ph.r[b]) == d.qloc[i];
+                for (int b = 0; b < kRegBits; b++) reg = reg || ph.rcol[b] == 1u << d.qloc[i];
                 if (!reg) o << " | (((goff >> " << d.qloc[i] << ") & 1u) << " << i << ")";
             }
         }
@@ -126,8 +127,10 @@ void emit_state_op(std::ostringstream& o, const DOp& d, const PhaseInfo& ph)
     case DOP_PHASETAB: {
         o << "        {\n            c64 ph = " << (h.s1 ? "xf[" + std::to_string(h.grad) + "]" : "c64{1.0, 0.0}")
           << ";\n";
+        const bool global = h.gmask == kLaneTabGlobal;   // the lane tables, else in xf
         for (uint32_t j = 0; j < h.s0; j++)
-            o << "            ph = cmul(ph, coef[" << (h.coef + 16u * j) << "u + ((tid >> " << 4 * j << ") & 15u)]);\n";
+            o << "            ph = cmul(ph, " << (global ? "coef[" : "xf[") << ((global ? h.coef : h.gmask) + 16u * j)
+              << "u + ((grp >> " << 4 * j << ") & 15u)]);\n";
         for (int r : selected(h.rsel)) o << "            a[" << r << "] = cmul(a[" << r << "], ph);\n";
         o << "        }\n";
         return;
@@ -136,150 +139,129 @@ void emit_state_op(std::ostringstream& o, const DOp& d, const PhaseInfo& ph)
     }
 }
 
-// `var` = the tile base of tile id `tile` (the id's bits deposited on the
-// qubits outside the tile).
-void emit_base(std::ostringstream& o, const SweepInfo& sw, const char* var, const char* tile, const char* ind)
+// `var` = thread address `thread` XOR the literal `reg`.  `span` holds every bit
+// a thread address can have: what the literal shares with it is XORed (a value
+// that many registers have in common), the rest added, so that it can become
+// the instruction's immediate offset.
+std::string address(const char* thread, uint64_t reg, uint64_t span, const char* suffix)
 {
-    o << ind << "uint64_t " << var << " = 0;\n";
-    int j = 0;
-    for (const uint64_t m : {sw.extmask & ~sw.exthi, sw.exthi})
-        for (int p = 0; p < 64; p++)
-            if ((m >> p) & 1) o << ind << var << " |= ((" << tile << " >> " << j++ << ") & 1ull) << " << p << ";\n";
+    std::string e = thread;
+    if (reg & span) e = "(" + e + " ^ " + std::to_string(reg & span) + suffix + ")";
+    if (reg & ~span) e += " + " + std::to_string(reg & ~span) + suffix;
+    return e;
 }
 
-// The tile's phase factors into xf (uses `base`, `tid`).
-void emit_factors(std::ostringstream& o, const Program& prog, const SweepInfo& sw, uint32_t nt, const char* ind)
+// The thread's byte offset of the sweep's loads (side 0) or stores (1), and
+// one line per register.
+void emit_io(std::ostringstream& o, const SweepIO& io, int side, uint32_t threads)
 {
-    if (sw.n_xf) {
-        o << ind << "uint64_t xbits = 0;\n";
-        int jx = 0;
-        for (int p = 0; p < 64; p++)
-            if ((sw.extmask >> p) & 1) o << ind << "xbits |= ((base >> " << p << ") & 1ull) << " << jx++ << ";\n";
+    uint64_t span = 0;
+    const uint32_t lanes = threads < uint32_t(kLaneEntries) ? threads : uint32_t(kLaneEntries);
+    o << "    {\n        uint64_t g = base << 4;\n";
+    for (int i = 0; i < kLaneBits && (1u << i) < lanes; i++) {
+        span |= io.lane[side][i];
+        o << "        g ^= (lane & " << (1u << i) << "u) ? " << io.lane[side][i] << "ull : 0ull;\n";
     }
-    for (uint32_t op = sw.op_begin; op < sw.op_end; op++) {
-        const DOpHdr& h = prog.ops[op].h;
-        if (has_tile_factor(h)) {
-            o << ind << "if (tid == " << (h.grad % nt) << "u) {\n" << ind << "    constexpr DOpHdr H = ";
-            emit_hdr(o, h);
-            o << ";\n" << ind << "    xf[" << h.grad << "] = tile_factor(H, coef, base, xbits);\n" << ind << "}\n";
-        }
+    span |= io.wave[side][0];
+    if (io.wave[side][0]) o << "        g ^= " << io.wave[side][0] << "ull;\n";
+    for (uint32_t v = 1; v < threads / lanes; v *= 2) {   // XOR-linear in the wave's bits
+        const uint64_t col = io.wave[side][v] ^ io.wave[side][0];
+        span |= col;
+        o << "        g ^= (wave & " << v << "u) ? " << col << "ull : 0ull;\n";
     }
+    for (int r = 0; r < kRegs; r++) {
+        const std::string at = "AMP(" + address("g", io.reg[side][r], span, "ull") + ")";
+        if (side) o << "        " << at << " = a[" << r << "];\n";
+        else o << "        { const c64 v = " << at << "; a[" << r << "] = c64{v.re, v.im}; }\n";
+        if (r % 4 == 3) o << "        SCHED();\n";
+    }
+    o << "    }\n";
 }
 
-// The sweep's phases on the tile at t0 (each ends with a barrier).
-void emit_phases(std::ostringstream& o, const Program& prog, const SweepInfo& sw)
+// One phase: the exchange that leads into it (the real parts, then the
+// imaginary parts), its ops.
+void emit_phase(std::ostringstream& o, const Program& prog, const SweepInfo& sw, uint32_t p, bool first,
+                uint32_t threads)
 {
-    for (uint32_t p = sw.phase_begin; p < sw.phase_end; p++) {
-        const PhaseInfo& ph = prog.phases[p];
-        o << "    {\n        constexpr PhaseInfo P = {{" << ph.r[0] << "u, " << ph.r[1] << "u, " << ph.r[2] << "u, "
-          << ph.r[3] << "u}, 0u, 0u, {" << ph.gcol[0] << "u, " << ph.gcol[1] << "u, " << ph.gcol[2] << "u, "
-          << ph.gcol[3] << "u}, " << ph.gxor << "u, " << ph.sxor << "u};\n"
-          << "        uint32_t off[kRegs], goffs[kRegs];\n        phase_offsets(P, off);\n"
-          << "        phase_gather_offsets(P, goffs);\n"
-          << "        const uint32_t goff = group_offset(P, tid);\n        c64 a[kRegs];\n"
-          << "#pragma unroll\n        for (int r = 0; r < kRegs; r++) a[r] = t0[lds_slot(goff | off[r])];\n";
-        // the phase's leading register permutations, which the interpreter
-        // folds into its gather map, run here as the ops they were (ops are
-        // stored contiguously phase after phase, so they sit between the
-        // previous phase's end and this phase's first op): measured faster
-        // than a gather through permuted literal offsets in the QFT's
-        // permutation-only sweeps
-        const uint32_t op0 = p ? prog.phases[p - 1].op_end : 0u;
-        bool unfold = op0 <= ph.op_begin;
-        for (uint32_t op = op0; unfold && op < ph.op_begin; op++) {
-            const uint32_t t = prog.ops[op].h.type;
-            unfold = t == DOP_X || t == DOP_CX || t == DOP_SWAP;
+    const LayoutPhase& L = prog.lphases[p];
+    const uint64_t* lt = &prog.lane_tab[size_t(p) * kLaneEntries];
+    const uint64_t* wt = &prog.wave_tab[size_t(p) * kWaveEntries];
+    o << "    {\n        const uint64_t te = ltab[" << uint64_t(p) * kLaneEntries << "u + lane] ^ wtab["
+      << uint64_t(p) * kWaveEntries << "u + wave];\n";
+    if (!first) {
+        uint64_t span = 0;
+        const uint32_t lanes = threads < uint32_t(kLaneEntries) ? threads : uint32_t(kLaneEntries);
+        for (uint32_t i = 0; i < lanes; i++) span |= lt[i];
+        for (uint32_t i = 0; i < threads / lanes; i++) span |= wt[i];
+        o << "        const uint32_t w = uint32_t(te) & 0xffffu, rd = uint32_t(te) >> 16;\n";
+        const char* meet = (L.flags & LPH_CROSS) ? "        __syncthreads();\n" : "        ORDER();\n";
+        if (L.flags & LPH_GUARD) o << "        __syncthreads();\n";
+        for (const char* part : {"re", "im"}) {
+            for (int r = 0; r < kRegs; r++)
+                o << "        LDS(" << address("w", L.w[r], span & 0xffffu, "u") << ") = a[" << r << "]." << part
+                  << ";\n";
+            o << meet;
+            for (int r = 0; r < kRegs; r++)
+                o << "        a[" << r << "]." << part << " = LDS("
+                  << address("rd", L.rd[r], (span >> 16) & 0xffffu, "u") << ");\n";
+            if (part[0] == 'r') o << meet;
         }
-        uint32_t gcol[kRegBits], gxor = 0;
-        for (int b = 0; b < kRegBits; b++) gcol[b] = 1u << ph.r[b];
-        for (uint32_t op = op0; unfold && op < ph.op_begin; op++) {   // must rebuild this phase's map
-            const DOpHdr& h = prog.ops[op].h;
-            if (h.type == DOP_X) gxor ^= gcol[h.s0];
-            else if (h.type == DOP_CX) gcol[h.s0] ^= gcol[h.s1];
-            else std::swap(gcol[h.s0], gcol[h.s1]);
-        }
-        for (int b = 0; b < kRegBits; b++) unfold = unfold && gcol[b] == ph.gcol[b];
-        unfold = unfold && gxor == ph.gxor;
-        if (!unfold) throw std::logic_error("jit: a phase's gather map is not its leading permutations");
-        for (uint32_t op = op0; op < ph.op_begin; op++) emit_state_op(o, prog.ops[op], ph);
-        for (uint32_t op = ph.op_begin; op < ph.op_end; op++) emit_state_op(o, prog.ops[op], ph);
-        o << "#pragma unroll\n        for (int r = 0; r < kRegs; r++) t0[lds_slot((goff | off[r]) ^ " << ph.sxor
-          << "u)] = a[r];\n"
-          << "    }\n    __syncthreads();\n";
     }
+    o << "        const uint32_t goff = uint32_t(te >> 32) & 0xffffu, grp = uint32_t(te >> 48);\n"
+      << "        (void)goff;\n        (void)grp;\n";
+    for (uint32_t op = L.op_begin; op < L.op_end; op++) {
+        emit_state_op(o, prog.ops[op], L, sw);
+        o << "        SCHED();\n";
+    }
+    o << "    }\n";
 }
 
+// The steps of sweep_tile (svmi_kernels.hip) for one sweep, with every
+// offset, flag and op a literal: the tile in registers, four waves per SIMD,
+// no dispatch and no address arithmetic per register, so that a sweep of a
+// QFT runs at the copy rate.  Compiled kernels with the tile in LDS before /
+// now: QFT of 27 qubits 5.00 / 4.17 ms (5 sweeps of 4.3 GB: 5.1 TB/s),
+// u3 brickwall of 27, 20 layers, 18.3 / 15.8 ms, 20 random layers of 27 35.7 /
+// 32.6 ms, QFT of 16 23.9 / 21.4 us.  (Double-buffered persistent kernels that
+// fetched the next tile by LDS DMA took 6.2, 22.2 and 39.8 ms.)
 void emit_sweep(std::ostringstream& o, const Program& prog, uint32_t i)
 {
     const SweepInfo& sw = prog.sweeps[i];
+    const SweepIO& io = prog.io[i];
     const uint32_t nt = 1u << (sw.k - kRegBits);
-    // second bound: at least two waves per SIMD, i.e. at most 256 VGPRs
-    o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ", 2)\n"
-      << "svmi_jit_" << i << "(c64* __restrict__ s, const c64* __restrict__ coef, const uint64_t* __restrict__ ht, "
-         "uint64_t tile0)\n{\n"
-      << "    __shared__ __align__(16) c64 t0[" << (1u << sw.k) << "];\n"
+    bool wide = false;   // dense blocks of 3 or 4 qubits need registers for their results
+    for (uint32_t op = sw.op_begin; op < sw.op_end; op++)
+        wide = wide || (prog.ops[op].h.type == DOP_DENSE && __builtin_popcount(prog.ops[op].h.smask) > 2);
+    // second bound: waves per SIMD
+    o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ", " << (wide ? 2 : 4) << ")\n"
+      << "svmi_jit_" << i << "(c64* __restrict__ s, const c64* __restrict__ coef, const DOp* __restrict__ ops, "
+         "const uint64_t* __restrict__ ltab, const uint64_t* __restrict__ wtab, uint64_t tile0)\n{\n"
+      << "    __shared__ __align__(16) unsigned char ex[" << (8u << sw.k) << "];\n"
       << "    __shared__ __align__(16) c64 xf[" << (sw.n_xf ? sw.n_xf : 1u) << "];\n"
-      << "    const uint32_t tid = threadIdx.x;\n"
-      << "    const uint64_t tile = tile0 + blockIdx.x;\n";
-    emit_base(o, sw, "base", "tile", "    ");
-    const uint32_t cmask = (1u << sw.c) - 1u;
-    o << "#pragma unroll\n    for (int j = 0; j < " << kRegs << "; j++) {\n"
-      << "        const uint32_t l = tid + " << nt << "u * j;\n"
-      << "        t0[lds_slot(l)] = s[base | ht[" << sw.hitab << "u + (l >> " << sw.c << ")] | (l & " << cmask
-      << "u)];\n    }\n";
-    emit_factors(o, prog, sw, nt, "    ");
-    o << "    __syncthreads();\n";
-    emit_phases(o, prog, sw);
-    o << "#pragma unroll\n    for (int j = 0; j < " << kRegs << "; j++) {\n"
-      << "        const uint32_t l = tid + " << nt << "u * j;\n"
-      << "        s[base | ht[" << sw.hitab << "u + (l >> " << sw.c << ")] | (l & " << cmask
-      << "u)] = t0[lds_slot(l)];\n    }\n}\n\n";
-}
-
-// Sweeps of 12-qubit tiles as persistent double-buffered kernels (one
-// workgroup of 256 threads per CU): while the phases of tile t run in one LDS
-// buffer, tile t + gridDim.x streams into the other by LDS DMA (tile_dma);
-// the wait for a tile's DMA leaves only the previous tile's 16 stores per
-// thread outstanding (vmcnt(16); the first tile waits for everything).
-bool dma_eligible(const SweepInfo& sw) { return sw.k == kDmaTileQubits && sw.c <= kDmaTileQubits; }
-
-void emit_sweep_dma(std::ostringstream& o, const Program& prog, uint32_t i)
-{
-    const SweepInfo& sw = prog.sweeps[i];
-    const uint32_t nt = kDmaThreads, kt = 1u << kDmaTileQubits, rows = kt >> sw.c;
-    const uint32_t cmask = (1u << sw.c) - 1u;
-    o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ", 1)\n"
-      << "svmi_jit_" << i << "(c64* __restrict__ s, const c64* __restrict__ coef, const uint64_t* __restrict__ hitab, "
-         "uint64_t n_tiles)\n{\n"
-      << "    __shared__ __align__(16) c64 tb[" << 2 * kt << "];\n"
-      << "    __shared__ __align__(16) uint64_t ht[" << rows << "];\n"
-      << "    __shared__ __align__(16) c64 xf[" << (sw.n_xf ? sw.n_xf : 1u) << "];\n"
-      << "    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;\n"
-      << "    for (uint32_t i = tid; i < " << rows << "u; i += " << nt << "u) ht[i] = hitab[" << sw.hitab << "u + i];\n"
-      << "    __syncthreads();\n"
-      << "    const uint32_t lds0 = lds_address(tb);\n"
-      << "    uint64_t t = blockIdx.x;\n"
-      << "    {\n";
-    emit_base(o, sw, "b0", "t", "        ");
-    o << "        tile_dma(s, ht, " << sw.c << "u, b0, lds0, wave, lane);\n    }\n"
-      << "    uint32_t cur = 0;\n    bool first = true;\n    for (;;) {\n"
-      << "        if (first) asm volatile(\"s_waitcnt vmcnt(0)\" ::: \"memory\");\n"
-      << "        else asm volatile(\"s_waitcnt vmcnt(16)\" ::: \"memory\");\n"
-      << "        __syncthreads();\n";
-    emit_base(o, sw, "base", "t", "        ");
-    o << "        const uint64_t tn = t + gridDim.x;\n        const bool more = tn < n_tiles;\n";
-    emit_factors(o, prog, sw, nt, "        ");
-    o << "        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): no load of the factors still in flight\n"
-      << "        if (more) {\n";
-    emit_base(o, sw, "bn", "tn", "            ");
-    o << "            tile_dma(s, ht, " << sw.c << "u, bn, lds0 + (cur ^ 1u) * " << kt * 16 << "u, wave, lane);\n"
-      << "        }\n        __syncthreads();\n"
-      << "        c64* t0 = tb + cur * " << kt << "u;\n";
-    emit_phases(o, prog, sw);
-    o << "#pragma unroll\n        for (int j = 0; j < " << kRegs << "; j++) {\n"
-      << "            const uint32_t l = tid + " << nt << "u * j;\n"
-      << "            s[base | ht[l >> " << sw.c << "] | (l & " << cmask << "u)] = t0[lds_slot(l)];\n        }\n"
-      << "        if (!more) break;\n        t = tn;\n        cur ^= 1u;\n        first = false;\n    }\n}\n\n";
+      << "    const uint32_t tid = threadIdx.x, lane = tid & 63u;\n"
+      << "    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);\n"
+      << "    const uint64_t tile = tile0 + blockIdx.x;\n    uint64_t base = 0;\n";
+    for (uint32_t r = 0; r < io.n_runs; r++)
+        o << "    base |= ((tile << " << io.run[r].shl << ") >> " << io.run[r].shr << ") & " << io.run[r].mask
+          << "ull;\n";
+    o << "    const uint32_t vhi = uint32_t(tile >> " << io.vhi_shift << ");\n    (void)vhi;\n";
+    if (sw.n_xf) {   // as tile_factors (svmi_kernels.hip)
+        const uint32_t nlt = 16u * sw.n_lt;
+        if (nlt)
+            o << "    for (uint32_t i = tid; i < " << nlt << "u; i += " << nt << "u) xf[" << (sw.n_xf - nlt)
+              << "u + i] = coef[" << sw.lt_coef << "u + i];\n";
+        o << "    const uint64_t xbits = extract_bits(base, " << sw.extmask << "ull);\n"
+          << "    for (uint32_t o = " << sw.op_begin << "u + tid; o < " << sw.op_end << "u; o += " << nt << "u) {\n"
+          << "        const DOpHdr h = ops[o].h;\n"
+          << "        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef, base, xbits);\n    }\n";
+    }
+    o << "    c64 a[kRegs];\n";
+    emit_io(o, io, 0, nt);
+    if (sw.n_xf) o << "    __syncthreads();\n";
+    for (uint32_t p = io.ph_begin; p < io.ph_end; p++) emit_phase(o, prog, sw, p, p == io.ph_begin, nt);
+    if (io.store_guard) o << "    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)\n    __syncthreads();\n";
+    emit_io(o, io, 1, nt);
+    o << "}\n\n";
 }
 
 struct Rtc {
@@ -327,46 +309,40 @@ void JitSweeps::release()
     if (module) hipModuleUnload(module);
     module = nullptr;
     fn.clear();
-    dma.clear();
-    dma_grid = 0;
 }
 
-std::string jit_source(const Program& prog, std::vector<char>& covered, uint64_t dma_grid)
+std::string jit_source(const Program& prog, std::vector<char>& covered)
 {
     covered.assign(prog.sweeps.size(), 0);
     std::ostringstream o;
-    o << "#include \"svmi_exec.hpp\"\nusing namespace svmi;\n\n";
+    o << "#include \"svmi_exec.hpp\"\nusing namespace svmi;\n"
+      << "#define AMP(off) (*reinterpret_cast<c64*>(reinterpret_cast<char*>(s) + (off)))\n"
+      << "#define LDS(off) (*reinterpret_cast<double*>(ex + (off)))\n"
+      << "#define SCHED() __builtin_amdgcn_sched_barrier(0)\n"
+      << "#define ORDER() asm volatile(\"\" ::: \"memory\")\n\n";
     if (prog.n_states != 1) return o.str();
     for (uint32_t i = 0; i < prog.sweeps.size(); i++) {
         const SweepInfo& sw = prog.sweeps[i];
-        if (sw.k > kJitMaxTileQubits || sw.mapped) continue;   // tile maps: interpreted
-        if (dma_grid && dma_eligible(sw) && sw.n_tiles >= 2 * dma_grid) {
-            emit_sweep_dma(o, prog, i);
-            covered[i] = 2;
-        } else {
-            emit_sweep(o, prog, i);
-            covered[i] = 1;
-        }
+        if (sw.k > kJitMaxTileQubits) continue;
+        emit_sweep(o, prog, i);
+        covered[i] = 1;
     }
     return o.str();
 }
 
-size_t jit_compile_only(const Program& prog, const char* arch, double* ms, std::string& err, uint64_t dma_grid)
+size_t jit_compile_only(const Program& prog, const char* arch, double* ms, std::string& err)
 {
     std::vector<char> covered, code;
-    const std::string src = jit_source(prog, covered, dma_grid);
+    const std::string src = jit_source(prog, covered);
     if (!compile(src, arch, code, ms, err)) return 0;
     return code.size();
 }
 
-bool jit_build(const Program& prog, const char* arch, JitSweeps& out, std::string& err, uint64_t dma_grid)
+bool jit_build(const Program& prog, const char* arch, JitSweeps& out, std::string& err)
 {
     out.release();
     std::vector<char> covered, code;
-    const std::string src = jit_source(prog, covered, dma_grid);
-    out.dma.assign(prog.sweeps.size(), 0);
-    for (size_t i = 0; i < covered.size(); i++) out.dma[i] = covered[i] == 2;
-    out.dma_grid = dma_grid;
+    const std::string src = jit_source(prog, covered);
     bool any = false;
     for (char c : covered) any = any || c;
     if (!any) return false;
@@ -389,21 +365,18 @@ bool jit_build(const Program& prog, const char* arch, JitSweeps& out, std::strin
     return true;
 }
 
-hipError_t jit_launch(hipStream_t st, const JitSweeps& j, uint32_t i, const SweepInfo& sw, c64* s, const c64* coef,
-                      const uint64_t* hitab)
+hipError_t jit_launch(hipStream_t st, const JitSweeps& j, uint32_t i, const SweepInfo& sw, c64* s,
+                      const SweepTables& t)
 {
-    if (i < j.dma.size() && j.dma[i]) {   // persistent: one workgroup per CU
-        const uint32_t grid = uint32_t(sw.n_tiles < j.dma_grid ? sw.n_tiles : j.dma_grid);
-        uint64_t n_tiles = sw.n_tiles;
-        void* args[] = {&s, &coef, &hitab, &n_tiles};
-        return hipModuleLaunchKernel(j.fn[i], grid, 1, 1, kDmaThreads, 1, 1, 0, st, args, nullptr);
-    }
     const uint32_t nt = 1u << (sw.k - kRegBits);
     const uint64_t max_grid = 1ull << 30;
+    const c64* coef = t.coef;
+    const DOp* ops = t.ops;
+    const uint64_t *ltab = t.lane_tab, *wtab = t.wave_tab;
     for (uint64_t t0 = 0; t0 < sw.n_tiles; t0 += max_grid) {
         const uint32_t cnt = uint32_t(sw.n_tiles - t0 < max_grid ? sw.n_tiles - t0 : max_grid);
         uint64_t tile0 = t0;
-        void* args[] = {&s, &coef, &hitab, &tile0};
+        void* args[] = {&s, &coef, &ops, &ltab, &wtab, &tile0};
         const hipError_t e = hipModuleLaunchKernel(j.fn[i], cnt, 1, 1, nt, 1, 1, 0, st, args, nullptr);
         if (e != hipSuccess) return e;
     }

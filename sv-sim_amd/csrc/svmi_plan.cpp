@@ -1813,16 +1813,6 @@ void build_adjoint_program(const std::vector<AdjEntry>& entries, int n, const Pl
     build_layouts(prog);
 }
 
-void build_row_tables(Program& prog)
-{
-    prog.hitab.clear();
-    for (SweepInfo& sw : prog.sweeps) {
-        sw.hitab = uint32_t(prog.hitab.size());
-        const uint64_t tile = ((uint64_t(1) << prog.n) - 1) & ~sw.extmask & ~((uint64_t(1) << sw.c) - 1);
-        for (uint64_t h = 0; h < (uint64_t(1) << (sw.k - sw.c)); h++) prog.hitab.push_back(deposit_bits(h, tile));
-    }
-}
-
 // FP64 multiply-adds per amplitude the program's state ops execute (a
 // complex multiply counted as 4, a real shear as 1 per component pair...):
 // the arithmetic the sweeps do per amplitude, summed over the program.

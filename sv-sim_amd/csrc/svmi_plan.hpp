@@ -53,7 +53,6 @@ struct Program {
     std::vector<PhaseInfo> phases;
     std::vector<DOp> ops;
     std::vector<c64> coef;
-    std::vector<uint64_t> hitab;       // build_row_tables
     std::vector<StandaloneOp> standalone;
     std::vector<MeasureStep> measures;
     // register layouts of the sweeps (build_layouts): io[i] for sweeps[i]
@@ -92,10 +91,6 @@ struct AdjEntry {
 // Backward program over (phi, lambda); entries in execution order.
 void build_adjoint_program(const std::vector<AdjEntry>& entries, int n, const PlanOptions& opt,
                            Program& prog);
-
-// prog.hitab and SweepInfo::hitab: the amplitude offsets of a tile's rows,
-// which compiled sweeps (svmi_jit.cpp) read.
-void build_row_tables(Program& prog);
 
 // FP64 multiply-adds per amplitude of the program's state ops.
 double program_fma_per_amp(const Program& prog);
