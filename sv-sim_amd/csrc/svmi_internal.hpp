@@ -90,7 +90,7 @@ constexpr int kMaxTileQubits = 13;          // 512 threads, 64 KiB of exchange a
 constexpr int kMaxTileQubitsAdj = 12;       // two states (phi, lambda): the same threads and LDS
 constexpr int kMaxBatchAdjTile = 11;        // largest svmi_batch_item::adj_tile
 // Two-state phases have 3 register bits; their fourth register "bit" is k,
-// the bit above the tile, which selects lambda's half of the LDS (phi at
+// the bit above the tile, which selects the state (phi at positions
 // [0, 2^k), lambda at [2^k, 2^(k+1))).  A thread's 16-amplitude group is then
 // phi's 8 amplitudes then lambda's, every op acts on both, and a tile has
 // 2^(k-3) threads -- the register footprint of a one-state group.
@@ -238,12 +238,11 @@ struct PhaseInfo {
     // scatter map: register rho is written to tile-local offset off[rho] ^ sxor
     // (the quarter turns a phase keeps in its register coordinates)
     uint32_t sxor;
-    // Tile map (two-state sweeps): the amplitude of tile-local index x sits at
-    // LDS index M(x), M linear over GF(2) (tile-local CX and SWAP ops folded
-    // into the addressing instead of run).  scol[s] = M(1 << r[s]) and gm[i] =
-    // M of the group number's bit i (the i-th non-register tile bit); gcol,
-    // gxor and sxor above are then LDS offsets in the span of scol.  One-state
-    // phases keep M the identity.
+    // Tile map: the amplitude of tile-local index x sits at position M(x) of
+    // the tile, M linear over GF(2) (tile-local CX and SWAP ops folded into the
+    // addressing instead of run).  scol[s] = M(1 << r[s]) and gm[i] = M of the
+    // group number's bit i (the i-th non-register tile bit); gcol, gxor and
+    // sxor above are then positions in the span of scol.
     uint32_t scol[4];
     uint16_t gm[10];
     uint32_t mapped;     // M differs from the identity
@@ -272,9 +271,8 @@ struct SweepInfo {
                          // with max_dense <= 2 run a kernel compiled without wider blocks
     uint32_t lt_coef;    // coef offset of a contiguous copy of those lane tables (16 c64 each),
     uint32_t n_lt;       // which every tile copies into the end of its factor area
-    uint32_t mapped;     // some phase or the tile's store addresses LDS through a tile map M
+    uint32_t mapped;     // some phase or the tile's store goes through a tile map M
     uint16_t fcol[14];   // M after the last phase: fcol[b] = M(1 << b)
-    uint16_t fj[16];     // M(j nt) (nt = the tile's threads): the store's per-register part
     uint32_t stage;      // largest coefficient count of a phase
 };
 constexpr uint32_t kMaxStage = 2048;   // coefficients of a phase that the latency builds stage in LDS

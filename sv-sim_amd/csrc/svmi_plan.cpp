@@ -1185,7 +1185,7 @@ void map_inverse(const uint32_t* col, int k, uint32_t* inv)
 }
 
 // A sweep cut into parts reloads the tile in the plain layout at every part
-// after the first: the part's phases address LDS through N o M_p, N the
+// after the first: the part's phases address the tile through N o M_p, N the
 // inverse of the map at the part's first phase, and its store through
 // N o (map at the part's end).  The first part loads the sweep's input, to
 // which the maps already refer (N = identity; folds made before the sweep's
@@ -1222,11 +1222,8 @@ void rebase_part(Program& prog, SweepInfo& part, int rb, bool first, const uint3
         part.mapped |= fin[l] != (1u << l) ? 1u : 0u;
     }
     for (int l = 0; l < 14; l++) part.fcol[l] = 0;
-    for (int j = 0; j < 16; j++) part.fj[j] = 0;
-    if (part.mapped) {
+    if (part.mapped)
         for (int l = 0; l < k; l++) part.fcol[l] = uint16_t(fin[l]);
-        for (uint32_t j = 0; j < (1u << rb); j++) part.fj[j] = uint16_t(map_apply(fin + (k - rb), rb, j));
-    }
 }
 
 void fold_leading_permutations(const Program& prog, PhaseInfo& pi)
@@ -1300,12 +1297,12 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
         int fold;         // tile-map candidate: 1 CX (control fc, target ft), 2 SWAP, 0 neither
         int fc, ft;       // tile-local bits of a candidate
     };
-    // Tile map of a sweep: the amplitude of tile-local index x sits at LDS
-    // index M(x) = XOR of mcol[b] over the set bits b of x.  A CX or SWAP on
+    // Tile map of a sweep: the amplitude of tile-local index x sits at
+    // position M(x) = XOR of mcol[b] over the set bits b of x.  A CX or SWAP on
     // two tile bits that are not both register bits of the phase taking it is
     // not run: after the phase, M becomes M o P (CX: mcol[c] ^= mcol[t]; SWAP:
-    // two columns exchanged), and later phases and the tile's store address
-    // LDS through M.
+    // two columns exchanged), and later phases and the tile's store take
+    // their amplitudes through M (svmi_layout.cpp).
     const bool fold_map = opt.tile_map;
     uint32_t mcol[32];
     for (int l = 0; l < k; l++) mcol[l] = 1u << l;
@@ -1549,19 +1546,12 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
         remaining.swap(rest);
     }
     sw.phase_end = uint32_t(prog.phases.size());
-    // mapped: some phase or the store addresses LDS through a map (fcol = the
+    // mapped: some phase or the store goes through a map (fcol = the
     // final one, which may be the identity)
     for (int l = 0; l < k; l++) sw.mapped |= mcol[l] != (1u << l) ? 1u : 0u;
     for (uint32_t p = sw.phase_begin; p < sw.phase_end; p++) sw.mapped |= prog.phases[p].mapped;
-    if (sw.mapped) {
+    if (sw.mapped)
         for (int l = 0; l < k; l++) sw.fcol[l] = uint16_t(mcol[l]);
-        for (uint32_t j = 0; j < (1u << rb); j++) {   // M(j << (k - rb)): the store's register part
-            uint32_t m = 0;
-            for (int b = 0; b < rb; b++)
-                if ((j >> b) & 1u) m ^= mcol[k - rb + b];
-            sw.fj[j] = uint16_t(m);
-        }
-    }
     // qubits that select register-table variants become the tile id's high
     // bits: workgroups running at the same time then read the same variants
     for (size_t o = sw.op_begin; o < prog.ops.size(); o++)
@@ -1881,7 +1871,7 @@ std::string describe_program(const Program& prog)
                     first = false;
                 }
             ss << "]";
-            if (sw.mapped) ss << " [m]";   // phases or the store address LDS through a tile map
+            if (sw.mapped) ss << " [m]";   // phases or the store go through a tile map
             ss << "\n";
             for (uint32_t p = sw.phase_begin; p < sw.phase_end; p++) {
                 const PhaseInfo& ph = prog.phases[p];
@@ -1889,7 +1879,7 @@ std::string describe_program(const Program& prog)
                 bool plain_gather = ph.gxor == 0;
                 for (int b = 0; b < kRegBits; b++) plain_gather = plain_gather && ph.gcol[b] == ph.scol[b];
                 if (!plain_gather) ss << " [g]";   // leading permutations folded into the gather
-                if (ph.mapped) ss << " [m]";       // LDS addressed through a tile map
+                if (ph.mapped) ss << " [m]";       // positions through a tile map
                 if (ph.sxor) ss << " [q]";         // quarter turns: scatter map r ^ f
                 ss << " :";
                 for (uint32_t o = ph.op_begin; o < ph.op_end; o++) {

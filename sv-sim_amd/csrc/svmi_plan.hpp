@@ -11,7 +11,7 @@ namespace svmi {
 
 struct PlanOptions {
     bool fusion = true;        // tiled multi-op sweeps; false = one pass per op
-    int tile_qubits = 12;      // k: qubits per LDS tile (13 allowed: one 128 KiB tile per CU)
+    int tile_qubits = 12;      // k: qubits per tile (at most 13, two states 12)
     int low_qubits = 4;        // c: physical qubits 0..c-1 in every tile
     long sweep_budget = 0;     // per-amplitude FMA budget of one sweep (0 = none)
     long op_overhead = 2;      // fusion cost model: per-op cost on top of its FMAs (per amplitude)
@@ -21,7 +21,7 @@ struct PlanOptions {
                                // merged register tables where the cost model prefers it
     int merge_qubits = 2;      // widest dense block the register-run merging may form (1..4)
     bool tile_map = true;      // tile-local CX and SWAP ops outside a phase's register bits become
-                               // a relabelling of the tile's LDS indices, not a phase
+                               // a relabelling of the tile's positions, not a phase
 };
 
 // One step of a program: a tiled sweep or a standalone full-state op.
