@@ -20,7 +20,7 @@ struct PauliTerm {
     uint64_t zmask;
     double cre, cim;     // coeff * i^{|x & z|} * (-1)^{|x & z|}
     uint32_t jsign;      // bit j: parity of zmask on register j's offset (PauliPass::col[j])
-    uint32_t pad;
+    uint32_t last;       // the last of the group's terms with this jsign (they are neighbours)
 };
 constexpr int kPauliTileQubits = 12;   // 2^12 amplitudes: 64 KiB of LDS, two workgroups per CU
 constexpr int kPauliThreadBits = 9;    // tile-local bits of the 512 threads, the rest are registers

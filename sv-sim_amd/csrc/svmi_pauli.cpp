@@ -120,6 +120,10 @@ void plan_pauli(const svmi_pauli_term* terms, size_t n_terms, int n, int tile_qu
             plan.terms.push_back(o);
         }
         G.end = uint32_t(plan.terms.size());
+        std::stable_sort(plan.terms.begin() + G.begin, plan.terms.end(),
+                         [](const PauliTerm& a, const PauliTerm& b) { return a.jsign < b.jsign; });
+        for (uint32_t e = G.begin; e < G.end; e++)
+            plan.terms[e].last = e + 1 == G.end || plan.terms[e + 1].jsign != plan.terms[e].jsign ? 1u : 0u;
         plan.groups.push_back(G);
     };
     for (size_t ps = 0; ps < tiles.size(); ps++) {
