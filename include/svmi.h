@@ -98,9 +98,9 @@ typedef struct svmi_stats {
 typedef enum svmi_option {
     SVMI_OPT_FUSION = 0,      /* 1 = tiled multi-gate sweeps (default), 0 = one pass per op */
     SVMI_OPT_TILE_QUBITS = 1, /* qubits per tile (4..13, two states up to 12; default by state size:
-                                 12, from 20 qubits on 13 (two states 11 and 12))             */
-    SVMI_OPT_LOW_QUBITS = 2,  /* low qubits every tile keeps for coalescing (0..8, default 4, from
-                                 20 qubits on 3 with the default tile)                        */
+                                 12, from 20 qubits on 13; two states 11, from 19 on 12)      */
+    SVMI_OPT_LOW_QUBITS = 2,  /* low qubits every tile keeps for coalescing (0..8, default 4; 3
+                                 with the default tile)                                       */
     SVMI_OPT_SWEEP_FLOPS = 3, /* per-amplitude FMA budget of one sweep (0 = unlimited)      */
     SVMI_OPT_PROFILE = 4,     /* 1 = time every launch with HIP events (svmi_stats)         */
     SVMI_OPT_PIPELINE = 5,    /* 0..64, no effect: every sweep holds its tile in registers and

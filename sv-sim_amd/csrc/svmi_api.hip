@@ -500,7 +500,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 PlanOptions of;
                 of.tile_qubits = it.fwd_tile ? it.fwd_tile : tu.fwd_tile;
                 of.op_overhead = it.op_cost ? it.op_cost - 1 : tu.op_cost;
-                if (ni[i] >= 18) of.low_qubits = 3;   // as default_tile
+                if (!it.fwd_tile) of.low_qubits = 3;   // as default_tile
                 plan_forward(it.gates, it.n_gates, ni[i], of, bp.fwd[i]);
                 std::vector<AdjEntry> entries;
                 adjoint_entries(it.gates, it.n_gates, it.param_slots, entries);
@@ -508,7 +508,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 // (16 circuits of 20-22 qubits with backward tiles of 11 / 12: 15.1 / 14.5 ms)
                 oa.tile_qubits = it.adj_tile ? it.adj_tile : ni[i] >= 18 ? kMaxTileQubitsAdj : tu.adj_tile;
                 oa.op_overhead = of.op_overhead;
-                oa.low_qubits = of.low_qubits;
+                if (!it.adj_tile) oa.low_qubits = 3;
                 build_adjoint_program(entries, ni[i], oa, bp.adj[i]);
                 plan_pauli(it.terms, it.n_terms, ni[i], kPauliTileQubits, true, 1, pauli[i]);
             }
@@ -1161,18 +1161,22 @@ svmi_status svmi_get_amplitudes(svmi_handle h, const uint64_t* idx, size_t count
     return SVMI_OK;
 }
 
-// Default tile and low qubits.  Tiles of 13 qubits (two states: 12) from 20
-// qubits on, where a state has at least 128 of them; on smaller states the
-// tiles of 12 (11) keep more CUs busy.  The large tiles keep 3 low qubits
-// (128-byte segments), which leaves one more for the circuit: at the copy
-// rate of 256-byte segments still, and fewer sweeps.  12 and 4 / 13 and 4 /
-// 13 and 3: u3 brick wall at 30 qubits 180 / 167 / 164 ms, QFT at 31 87.6 /
-// 93.6 / 81.8 ms, 20 random layers at 28 75.8 / 64.0 / 65.8 ms, at 18 361 /
-// 395 us.
+// Default tile and low qubits.  Tiles of 13 qubits from 20 qubits on (two
+// states: 12 from 19), where a state has at least 128 of them; on smaller
+// states the tiles of 12 (11) keep more CUs busy.  3 low qubits (128-byte
+// segments) leave one more than 4 for the circuit: at the copy rate of
+// 256-byte segments still, and fewer sweeps.  12 and 4 / 13 and 4 / 13 and 3:
+// u3 brick wall at 30 qubits 180 / 167 / 164 ms, QFT at 31 87.6 / 93.6 / 81.8
+// ms, 20 random layers at 28 75.8 / 64.0 / 65.8 ms, at 18 361 / 395 us.
+// 12 and 4 / 12 and 3: ansatz of 8 layers at 15, 17, 19 qubits 129 / 123, 154 /
+// 152, 211 / 200 us, 10 random layers 119 / 118, 151 / 148, 213 / 194 us;
+// the ansatz's adjoint with 11 and 4 / 11 and 3 / 12 and 3: at 15 482 / 461 /
+// 480, at 18 707 / 634 / 660, at 19 869 / 822 / 783 us.  (2 low qubits: random
+// layers of 17 qubits 159 us.)
 void default_tile(svmi_handle h, int n, bool two, PlanOptions& o)
 {
-    if (!h->tile_set) o.tile_qubits = n >= 20 ? (two ? 12 : 13) : (two ? 11 : 12);
-    if (!h->low_set && !h->tile_set && n >= 20) o.low_qubits = 3;
+    if (!h->tile_set) o.tile_qubits = n >= 20 ? (two ? 12 : 13) : n == 19 || !two ? 12 : 11;
+    if (!h->low_set && !h->tile_set) o.low_qubits = 3;
 }
 
 // Planner options of the forward program.  Specialised sweeps pay almost
