@@ -1182,16 +1182,14 @@ void default_tile(svmi_handle h, int n, bool two, PlanOptions& o)
 // Planner options of the forward program.  Specialised sweeps pay almost
 // nothing per op (no dispatch), so unless the caller set an op cost their
 // fusion model counts FMAs only (the u3 brickwall and the random layers of 27
-// qubits take the same 15.8 and 32.6 ms with the interpreted sweeps' 2).
+// qubits take the same 15.8 and 32.6 ms in 12-qubit tiles with the interpreted sweeps' 2).
 //
-// Compiled sweeps keep tiles of 12 qubits, and from 20 qubits on 3 low ones
-// where the tile is the default (QFT of 27 qubits 4.38 -> 4.16 ms, u3
-// brickwall of 27, 20 layers, 17.1 -> 16.0 ms).  They use tile maps only below
+// Compiled sweeps keep 3 low qubits from 20 qubits on where the tile is the
+// default (QFT of 27 qubits 4.38 -> 4.16 ms, u3 brickwall of 27, 20 layers,
+// 17.1 -> 16.0 ms).  They use tile maps only below
 // 20 qubits: there a phase less shows (QFT of 16 qubits 25.4 -> 21.7 us), while
 // a sweep of a large state is bound by its pass over memory (QFT of 27 qubits
 // 4.16 ms without, 4.26 ms with maps).
-constexpr int kJitLargeQubits = 20;
-
 PlanOptions forward_options(svmi_handle h)
 {
     PlanOptions o = h->opt;
@@ -1205,6 +1203,25 @@ PlanOptions forward_options(svmi_handle h)
         o.tile_map = false;
     }
     return o;
+}
+
+// h->prog.  Compiled sweeps of 12- and 13-qubit tiles pass over memory at the
+// same rate, and more of the smaller workgroups fit a CU, so the larger tile is
+// taken where it saves a pass.  12 / 13: QFT of 27 qubits 4.19 / 4.53 ms (5
+// passes each), of 30 41.1 / 35.2 (6 / 5); u3 brickwall of 30 172 / 153 (21 /
+// 19); random layers of 27 32.7 / 27.4 (37 / 30), of 20 0.282 / 0.240 (12 / 9).
+// The second plan costs well under a thousandth of the compilation.  From 32
+// qubits on (64 GiB) tiles that span 10 high qubits read memory slower than
+// they save: QFT of 32 158 / 175, of 33 313 / 405 ms (6 / 5 passes).
+void plan_circuit(svmi_handle h, const svmi_gate* gates, size_t n_gates)
+{
+    PlanOptions o = forward_options(h);
+    plan_forward(gates, n_gates, h->n_int, o, h->prog);
+    if (!h->specialize || h->tile_set || h->n_int < kJitLargeQubits || h->n_int > 31) return;
+    Program large;
+    o.tile_qubits = kMaxTileQubits;
+    plan_forward(gates, n_gates, h->n_int, o, large);
+    if (large.steps.size() < h->prog.steps.size()) h->prog = std::move(large);
 }
 
 // Device copy of h->prog and, with SVMI_OPT_SPECIALIZE, its compiled sweeps.
@@ -1233,7 +1250,7 @@ svmi_status svmi_upload(svmi_handle h, const svmi_gate* gates, size_t n_gates)
     SVMI_TRY(check_gates(gates, n_gates, h->n));
     h->gates.assign(gates, gates + n_gates);
     h->adj_valid = false;
-    plan_forward(gates, n_gates, h->n_int, forward_options(h), h->prog);
+    plan_circuit(h, gates, n_gates);
     SVMI_TRY(install_program(h));
     h->uploaded = true;
     h->stats.gates = n_gates;
@@ -1743,7 +1760,7 @@ svmi_status svmi_set_option(svmi_handle h, int option, int64_t value)
     }
     h->adj_valid = false;
     if (h->uploaded) {
-        plan_forward(h->gates.data(), h->gates.size(), h->n_int, forward_options(h), h->prog);
+        plan_circuit(h, h->gates.data(), h->gates.size());
         SVMI_TRY(use_device(h));
         SVMI_TRY(install_program(h));
         h->stats.ops = h->prog.n_lowered;

@@ -18,7 +18,6 @@ extern const int kJitHeaderCount;
 
 namespace {
 
-constexpr uint32_t kJitMaxTileQubits = 12;   // wider tiles are interpreted
 
 // Registers r (0..15) whose register bits satisfy `rsel`, as a list.
 std::vector<int> selected(uint32_t rsel)
@@ -221,8 +220,8 @@ void emit_phase(std::ostringstream& o, const Program& prog, const SweepInfo& sw,
 // no dispatch and no address arithmetic per register, so that a sweep of a
 // QFT runs at the copy rate.  Compiled kernels with the tile in LDS before /
 // now: QFT of 27 qubits 5.00 / 4.17 ms (5 sweeps of 4.3 GB: 5.1 TB/s),
-// u3 brickwall of 27, 20 layers, 18.3 / 15.8 ms, 20 random layers of 27 35.7 /
-// 32.6 ms, QFT of 16 23.9 / 21.4 us.  (Double-buffered persistent kernels that
+// u3 brickwall of 27, 20 layers, 18.3 / 14.7 ms, 20 random layers of 27 35.7 /
+// 27.4 ms (with tiles of 13 qubits), QFT of 16 23.9 / 21.4 us.  (Double-buffered persistent kernels that
 // fetched the next tile by LDS DMA took 6.2, 22.2 and 39.8 ms.)
 void emit_sweep(std::ostringstream& o, const Program& prog, uint32_t i)
 {
@@ -323,7 +322,7 @@ std::string jit_source(const Program& prog, std::vector<char>& covered)
     if (prog.n_states != 1) return o.str();
     for (uint32_t i = 0; i < prog.sweeps.size(); i++) {
         const SweepInfo& sw = prog.sweeps[i];
-        if (sw.k > kJitMaxTileQubits) continue;
+        if (sw.k > (prog.n >= kJitLargeQubits ? 13u : 12u)) continue;
         emit_sweep(o, prog, i);
         covered[i] = 1;
     }

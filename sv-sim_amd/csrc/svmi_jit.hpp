@@ -29,6 +29,10 @@
 
 namespace svmi {
 
+// From this many qubits on sweeps of 13-qubit tiles are compiled too (below, a
+// state has too few of them to fill the chip).
+constexpr int kJitLargeQubits = 20;
+
 struct JitSweeps {
     hipModule_t module = nullptr;
     std::vector<hipFunction_t> fn;   // per sweep of the program; nullptr: run by k_sweep1
@@ -38,7 +42,7 @@ struct JitSweeps {
 
 // HIP source of the specialised kernels (`svmi_jit_<i>` for sweep i) of a
 // forward program; sweeps the generator does not cover (two states, tiles
-// above 12 qubits) get no kernel.  covered[i] = 1 for the sweeps it emits.
+// above 12 qubits on small states) get no kernel.  covered[i] = 1 for the sweeps it emits.
 std::string jit_source(const Program& prog, std::vector<char>& covered);
 
 // Compile with hipRTC for `arch` and load the module on the current device.

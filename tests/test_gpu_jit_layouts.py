@@ -1,6 +1,7 @@
 """Compiled sweeps on the register layouts, where addresses can go wrong:
 tiles of less than a wave up to several waves, sweeps that only move
-amplitudes (with and without tile maps: below and from 20 qubits on), and
+amplitudes (with and without tile maps: below and from 20 qubits on), 13-qubit
+tiles (from 20 qubits on), and
 phase products read from the staged lane tables.
 
 Permutation circuits only move numbers, so their states equal the oracle's
@@ -32,7 +33,7 @@ def _run(n, gates, state, tile=None, low=None):
 
 
 CASES = [(5, None, None), (9, None, None), (10, None, None), (11, None, None), (13, None, None), (13, 5, 0),
-         (14, 9, 3), (19, None, None), (20, None, None)]
+         (14, 9, 3), (19, None, None), (20, None, None), (20, 13, 3), (20, 12, 3)]
 
 
 @pytest.mark.parametrize("n,tile,low", CASES)
