@@ -1069,6 +1069,8 @@ svmi_status svmi_destroy(svmi_handle h)
     h->jit.release();
     h->adj_dprog.release();
     h->adj_gsum.release();
+    h->qir_dprog.release();
+    h->qir_meas.release();
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
