@@ -42,7 +42,13 @@ svmi_status svmi_debug_emulate_batch(const svmi_batch_item* items, size_t n_item
 svmi_status svmi_debug_plan_batch(const svmi_batch_item* items, size_t n_items, uint64_t* n_levels,
                                   uint64_t* n_launches, uint64_t* n_tasks, uint64_t* state_bytes);
 
-/* The same for the backward (adjoint) program svmi_adjoint builds. */
+/* Coefficients of the batch's plan, and the largest offset (in coefficients)
+ * that a sweep adds in 32 bits of bytes to the base it reads an op's
+ * coefficients from: below 2^28 minus the largest op's own coefficients. */
+svmi_status svmi_debug_batch_coefs(const svmi_batch_item* items, size_t n_items, uint64_t* n_coefs,
+                                   uint64_t* max_offset);
+
+/* Planner summary (as svmi_debug_plan) of the backward program svmi_adjoint builds. */
 svmi_status svmi_debug_plan_adjoint(int n, const svmi_gate* gates, size_t n_gates, const int32_t* param_slots,
                                     size_t n_params, int tile_qubits, int low_qubits, uint64_t* n_passes,
                                     char* buf, size_t buflen);

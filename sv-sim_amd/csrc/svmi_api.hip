@@ -444,8 +444,11 @@ svmi_status verify_batch(const BatchPlan& bp)
                 if (L.op_begin > L.op_end ||
                     (L.op_begin < L.op_end && (L.op_begin < sw.op_begin || L.op_end > sw.op_end)))
                     return fail(SVMI_ERR_STATE, "batch plan: bad phase");
+                if (uint64_t(L.coef_begin) + L.coef_n > bp.coef.size())
+                    return fail(SVMI_ERR_STATE, "batch plan: bad coefficient range");
                 for (uint32_t o = L.op_begin; o < L.op_end; o++)
-                    if (bp.ops[o].h.coef > bp.coef.size()) return fail(SVMI_ERR_STATE, "batch plan: bad coef offset");
+                    if (bp.ops[o].h.coef >= kMaxPhaseCoefs || bp.ops[o].h.coef > L.coef_n)
+                        return fail(SVMI_ERR_STATE, "batch plan: bad coef offset");
             }
         } else if (b.kind == BSTEP_PAULI) {
             if (b.partial + b.n_tasks > bp.n_e_partials) return fail(SVMI_ERR_STATE, "batch plan: bad E partials");
@@ -531,8 +534,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
         const uint32_t lp_base = uint32_t(bp.lphases.size());
         const uint32_t sw_base = uint32_t(bp.sweeps.size());
         for (DOp d : pr.ops) {
-            d.h.coef += coef_base;
-            if (d.h.type == DOP_ROT && d.h.s0) d.h.grad += coef_base;   // its table
+            if (has_tile_factor(d.h)) d.qphys[0] += coef_base;
             bp.ops.push_back(d);
         }
         for (LayoutPhase L : pr.lphases) {
@@ -1846,7 +1848,8 @@ void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, c
     const uint64_t xbits = ext_index(sw, base);
     for (uint32_t i = 0; i < 16u * sw.n_lt; i++) xf[sw.n_xf - 16u * sw.n_lt + i] = coef[sw.lt_coef + i];
     for (uint32_t o = sw.op_begin; o < sw.op_end; o++)
-        if (has_tile_factor(ops[o].h)) xf[ops[o].h.grad] = tile_factor(ops[o].h, coef, base, xbits);
+        if (has_tile_factor(ops[o].h))
+            xf[ops[o].h.grad] = tile_factor(ops[o].h, coef + ops[o].qphys[0], base, xbits);
     struct Group {
         c64 a[kRegs];
     };
@@ -1900,14 +1903,15 @@ void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, c
             g.swap(h);
         }
         const RegOffsets off{L.rcol};
+        const c64* cf = coef + L.coef_begin;
         for (uint32_t t = 0; t < nt; t++) {
             const uint32_t goff = uint32_t(entry(t) >> 32) & 0xffffu, grp = uint32_t(entry(t) >> 48);
             for (uint32_t o = L.op_begin; o < L.op_end; o++) {
                 const DOp& op = ops[o];
                 if (op.h.type == DOP_GRAD_DENSE || op.h.type == DOP_GRAD_DIAG)
-                    gsum_tile[op.h.grad] += exec_grad_op<kRegBits, kRegsAdj>(op.h, &op, g[t].a, coef, goff, off, base);
+                    gsum_tile[op.h.grad] += exec_grad_op<kRegBits, kRegsAdj>(op.h, &op, g[t].a, cf, goff, off, base);
                 else
-                    exec_state_op(op.h, &op, g[t].a, coef, goff, grp, off, base, xf.data(), sw.exthi, vhi);
+                    exec_state_op(op.h, &op, g[t].a, cf, goff, grp, off, base, xf.data(), sw.exthi, vhi);
             }
         }
     }
@@ -2174,6 +2178,21 @@ svmi_status svmi_debug_plan_batch(const svmi_batch_item* items, size_t n_items, 
     if (n_launches) *n_launches = bp.launches.size();
     if (n_tasks) *n_tasks = bp.n_tasks;
     if (state_bytes) *state_bytes = bp.state_bytes;
+    return SVMI_OK;
+}
+
+svmi_status svmi_debug_batch_coefs(const svmi_batch_item* items, size_t n_items, uint64_t* n_coefs,
+                                   uint64_t* max_offset)
+{
+    if (n_items == 0) return fail(SVMI_ERR_ARG, "empty batch");
+    std::vector<double> ev(n_items), gr(1);
+    BatchPlan bp;
+    SVMI_TRY(build_batch(items, n_items, ev.data(), gr.data(), bp));
+    uint64_t off = 0;
+    for (const LayoutPhase& L : bp.lphases)
+        for (uint32_t o = L.op_begin; o < L.op_end; o++) off = std::max<uint64_t>(off, bp.ops[o].h.coef);
+    if (n_coefs) *n_coefs = bp.coef.size();
+    if (max_offset) *max_offset = off;
     return SVMI_OK;
 }
 

@@ -178,7 +178,8 @@ struct DOpHdr {
     uint32_t type;
     uint32_t smask;      // DENSE / GRAD_DENSE: register slot mask
     uint32_t s0, s1;     // X/CX/SWAP/SRN slots
-    uint32_t coef;       // offset into the coefficient array (c64 units)
+    uint32_t coef;       // first coefficient (c64 units), counted from LayoutPhase::coef_begin;
+                         // 0 for ops without one
     uint32_t grad;       // GRAD_*: accumulator slot within the sweep
     uint32_t rsel;       // CPHASE/DIAG/CDENSE: registers rho whose register bits satisfy the op
     uint32_t gmask;      // CPHASE/DIAG/CDENSE: non-register tile-local bits that must be 1
@@ -221,7 +222,8 @@ struct DOp {
     uint32_t nq;         // DIAG: number of qubits
     uint32_t targets;    // adjoint: DOP_TO_* (forward sweeps: DOP_TO_PSI)
     int32_t qloc[5];     // DIAG: tile-local bit of qubit i, or -1 if outside the tile
-    uint32_t qphys[5];   // DIAG: physical position of qubit i
+    uint32_t qphys[5];   // DIAG: physical position of qubit i; ops with a tile factor:
+                         // qphys[0] is the first coefficient counted from the program's
 };
 static_assert(sizeof(DOpHdr) == 40 && sizeof(DOp) == 88, "DOp layout");
 
@@ -407,8 +409,13 @@ struct SlotMask {
     }
 };
 
+// Coefficients of one phase before another phase of the same registers begins
+// (svmi_layout.cpp): an op's first one is below this, so byte offsets from a
+// phase's first coefficient fit 32 bits however many the program has.
+constexpr uint32_t kMaxPhaseCoefs = 1u << 16;
+
 // coef + i as base and 32-bit byte offset (one scalar shift instead of a
-// 64-bit shift and add per access).
+// 64-bit shift and add per access).  coef: the phase's first coefficient.
 SVMI_HD inline const c64* coef_at(const c64* coef, uint32_t i)
 {
     return reinterpret_cast<const c64*>(reinterpret_cast<const char*>(coef) + uint32_t(i * 16u));

@@ -46,8 +46,11 @@ std::string variant(uint64_t emask, const SweepInfo& sw)
 
 // One op as direct code: the templates of svmi_exec.hpp / svmi_internal.hpp
 // with every slot, mask and offset a literal, so no dispatch is compiled.
-void emit_state_op(std::ostringstream& o, const DOp& d, const LayoutPhase& ph, const SweepInfo& sw)
+// Coefficient offsets count from the program's first one.
+void emit_state_op(std::ostringstream& o, DOp d, const LayoutPhase& ph, const SweepInfo& sw)
 {
+    d.h.coef += ph.coef_begin;
+    if (d.h.type == DOP_ROT && d.h.s0) d.h.grad += ph.coef_begin;   // its table
     const DOpHdr& h = d.h;
     const std::string cond = "(base & " + std::to_string(h.emask) + "ull) == " + std::to_string(h.emask) +
                              "ull && (goff & " + std::to_string(h.gmask) + "u) == " + std::to_string(h.gmask) + "u";
@@ -252,7 +255,7 @@ void emit_sweep(std::ostringstream& o, const Program& prog, uint32_t i)
         o << "    const uint64_t xbits = extract_bits(base, " << sw.extmask << "ull);\n"
           << "    for (uint32_t o = " << sw.op_begin << "u + tid; o < " << sw.op_end << "u; o += " << nt << "u) {\n"
           << "        const DOpHdr h = ops[o].h;\n"
-          << "        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef, base, xbits);\n    }\n";
+          << "        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef + ops[o].qphys[0], base, xbits);\n    }\n";
     }
     o << "    c64 a[kRegs];\n";
     emit_io(o, io, 0, nt);

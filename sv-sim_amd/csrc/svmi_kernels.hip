@@ -56,7 +56,7 @@ tile_factors(c64* xf, const SweepInfo& sw, const DOp* __restrict__ ops, const c6
     const uint64_t x = ext_index(sw, base);
     for (uint32_t o = sw.op_begin + tid; o < sw.op_end; o += blockDim.x) {
         const DOpHdr h = ops[o].h;
-        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef, base, x);
+        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef + ops[o].qphys[0], base, x);
     }
 }
 
@@ -211,7 +211,7 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
         // kLat: this phase's coefficients in one half of the stage; the next
         // one's are on their way, up to kPre per thread in registers
         constexpr uint32_t kPre = 4;
-        const c64* __restrict__ cf = coef;
+        const c64* __restrict__ cf = coef + L.coef_begin;
         c64 pre[kLat ? kPre : 1];
         uint32_t pre_n = 0, pre_c = 0;
         DOpHdr nxt;
@@ -231,8 +231,6 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
             if constexpr (kLat) {   // (op arrays end with an unused record)
                 h = nxt;
                 nxt = op[1].h;
-                if (h.type == DOP_ROT && h.s0) h.grad -= L.coef_begin;   // its table
-                h.coef -= L.coef_begin;
             } else {
                 h = op->h;
             }

@@ -52,7 +52,8 @@ EXPORTS = ["svmi_create", "svmi_destroy", "svmi_num_qubits", "svmi_reset_state",
            "svmi_set_option", "svmi_get_stats", "svmi_last_error", "svmi_abi_version", "svmi_qir_run", "svmi_qasm_parse",
            "svmi_debug_emulate", "svmi_debug_emulate_adjoint", "svmi_debug_emulate_batch", "svmi_debug_plan",
            "svmi_debug_plan_batch", "svmi_debug_plan_adjoint", "svmi_debug_emulate_qir", "svmi_debug_plan_qir",
-           "svmi_debug_jit", "svmi_dm_qir_run", "svmi_debug_emulate_dm_qir", "svmi_debug_step_times", "svmi_debug_fp64_rates", "svmi_expval_static"]
+           "svmi_debug_jit", "svmi_dm_qir_run", "svmi_debug_emulate_dm_qir", "svmi_debug_step_times", "svmi_debug_fp64_rates", "svmi_expval_static",
+           "svmi_debug_batch_coefs"]
 
 
 class SvmiError(RuntimeError):
@@ -126,6 +127,8 @@ def lib():
         L.svmi_debug_emulate_adjoint.argtypes = [ctypes.c_int, _vp, _sz, _vp, _sz, _vp, _sz, ctypes.c_int,
                                                  ctypes.c_int, _vp, _vp, _vp, _vp]
         L.svmi_debug_emulate_batch.argtypes = [_vp, _sz, _vp, _vp]
+        L.svmi_debug_batch_coefs.argtypes = [_vp, _sz, ctypes.POINTER(ctypes.c_uint64),
+                                             ctypes.POINTER(ctypes.c_uint64)]
         L.svmi_debug_plan.argtypes = [ctypes.c_int, _vp, _sz, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                       ctypes.c_int64, ctypes.POINTER(ctypes.c_uint64), ctypes.c_char_p, _sz]
         L.svmi_debug_plan_adjoint.argtypes = [ctypes.c_int, _vp, _sz, _vp, _sz, ctypes.c_int, ctypes.c_int,
@@ -406,6 +409,15 @@ def plan_batch(items):
     v = [ctypes.c_uint64() for _ in range(4)]
     _check(lib().svmi_debug_plan_batch(ctypes.cast(arr, _vp), len(items), *[ctypes.byref(x) for x in v]))
     return dict(zip(("levels", "launches", "tasks", "state_bytes"), (x.value for x in v)))
+
+
+def batch_coefs(items):
+    """(coefficients of the batch plan, largest offset of an op's first one from its phase's)."""
+    arr, keep, _ = _batch_items(items)
+    v = [ctypes.c_uint64() for _ in range(2)]
+    _check(lib().svmi_debug_batch_coefs(ctypes.cast(arr, _vp), len(items), *[ctypes.byref(x) for x in v]))
+    return tuple(x.value for x in v)
+
 
 def emulate(n, gates, state, fusion=True, tile_qubits=12, low_qubits=4, sweep_budget=0):
     g = as_gates(gates)
