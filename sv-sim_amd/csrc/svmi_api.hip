@@ -529,6 +529,17 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                                 "batch item " + std::to_string(i) +
                                     ": an op does not fit a tile (a 5-qubit gate such as C4X, or a tile too small "
                                     "for the 4 low qubits plus the op's qubits)");
+    // the chunk's tables are indexed with 32 bits
+    uint64_t n_ops = 0, n_coefs = 0, n_phases = 0;
+    for (size_t i = 0; i < n_items; i++)
+        for (const Program* pr : {&bp.fwd[i], &bp.adj[i]}) {
+            n_ops += pr->ops.size();
+            n_coefs += pr->coef.size();
+            n_phases += pr->lphases.size();
+        }
+    if (std::max({n_ops, n_coefs, n_phases}) > UINT32_MAX)
+        return fail(SVMI_ERR_UNSUPPORTED, "batch: more than 2^32 ops or coefficients planned together; give the "
+                                          "circuits to several calls");
     auto append_program = [&](const Program& pr) {
         const uint32_t op_base = uint32_t(bp.ops.size()), coef_base = uint32_t(bp.coef.size());
         const uint32_t lp_base = uint32_t(bp.lphases.size());

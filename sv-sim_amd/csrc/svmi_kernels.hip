@@ -161,12 +161,12 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
         for (uint32_t i = tid; i < n; i += nt) stage[i] = coef[c0 + i];
     }
     if (kLat || sw.n_xf) __syncthreads();
-    uint64_t le = ltab[ph_begin * uint32_t(kLaneEntries) + lane];
+    uint64_t le = ltab[size_t(ph_begin) * kLaneEntries + lane];
     for (uint32_t p = ph_begin; p < ph_end; p++) {
         const LayoutPhase& L = lph[p];
-        const uint64_t te = le ^ wtab[p * uint32_t(kWaveEntries) + wave];
+        const uint64_t te = le ^ wtab[size_t(p) * kWaveEntries + wave];
         const uint32_t pn = p + 1 < ph_end ? p + 1 : p;
-        le = ltab[pn * uint32_t(kLaneEntries) + lane];
+        le = ltab[size_t(pn) * kLaneEntries + lane];
         if (p != ph_begin) {
             uint32_t w = uint32_t(te) & 0xffffu, rd = uint32_t(te) >> 16;
             const uint32_t flags = L.flags;
