@@ -256,7 +256,7 @@ struct SweepInfo {
     uint32_t k;          // tile qubits
     uint32_t c;          // low physical qubits 0..c-1 always in the tile
     uint32_t n_ext;      // number of physical qubits outside the tile
-    uint32_t pad;
+    uint32_t whole;      // set at the launch of a latency build: exchanges move whole amplitudes
     uint32_t n_grad;     // adjoint: accumulators used by this sweep
     uint32_t grad_base;  // adjoint: first global accumulator of this sweep
     uint64_t extmask;    // physical qubits outside the tile
@@ -277,7 +277,6 @@ struct SweepInfo {
     uint16_t fcol[14];   // M after the last phase: fcol[b] = M(1 << b)
     uint32_t stage;      // largest coefficient count of a phase
 };
-constexpr uint32_t kMaxStage = 2048;   // coefficients of a phase that the latency builds stage in LDS
 
 // ----------------------------------------------------------------------------
 // Register layouts (svmi_layout.cpp): how a sweep runs on the device.  The

@@ -11,6 +11,8 @@
 //   state fills are simple grid-stride kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "svmi_exec.hpp"
 #include "svmi_kernels.hpp"
 
@@ -60,7 +62,8 @@ tile_factors(c64* xf, const SweepInfo& sw, const DOp* __restrict__ ops, const c6
     }
 }
 
-// LDS of a tile: exchange area (8 bytes per amplitude of every state) | phase
+// LDS of a tile: exchange area (8 bytes per amplitude of every state, 16 where
+// whole amplitudes change threads) | phase
 // factors | gradient accumulators.
 size_t sweep_smem_bytes(const SweepInfo& sw, int ns)
 {
@@ -103,16 +106,27 @@ __device__ __attribute__((always_inline)) inline double& lds_at(unsigned char* s
 // kLat: the build for sweeps of few tiles, which leave the chip idle and are
 // bound by latency: a cold scalar load takes a microsecond, a register table
 // four of them in a row.  Every phase's coefficients are staged in LDS during
-// the phase before it and the next op's header is loaded during an op.
+// the phase before it and the next op's header is loaded during an op.  Where
+// LDS allows (sw.whole), exchanges move whole amplitudes: one round trip and
+// one barrier instead of two and three (ansatz of 20 u3 layers at 13 qubits
+// 83.9 -> 82.2 us, random layers at 17 qubits 156.7 -> 151.9).
 template <int NS, int kMaxQ, bool kLat = false>
 __device__ __attribute__((always_inline)) inline void
 sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, const SweepIO* __restrict__ io, SVMI_TABLES,
            double* __restrict__ grad_partials, uint64_t tile, unsigned char* smem, bool init_zero)
 {
-    const uint32_t tid = threadIdx.x, nt = blockDim.x, lane = tid & 63u;
+    // kLat: a tile of less than a wave's threads has a whole wave; the others
+    // repeat its threads (same values to the same places) but for the tables,
+    // which all of them load (stid of snt): one thread took 33 of the 67 us of
+    // 10 random layers at 4 qubits to stage them
+    const uint32_t stid = threadIdx.x, snt = blockDim.x;
+    const uint32_t nt = kLat ? min(snt, sweep_threads(sw.k, NS)) : snt, tid = kLat ? stid & (nt - 1) : stid;
+    const uint32_t lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nwaves = (nt + 63) / 64;
-    c64* xf = reinterpret_cast<c64*>(smem + (size_t(8 * NS) << sw.k));
+    const uint32_t plane = uint32_t(8 * NS) << sw.k;
+    const bool whole = kLat && sw.whole;   // uniform
+    c64* xf = reinterpret_cast<c64*>(smem + (size_t(plane) << (whole ? 1 : 0)));
     double* gacc = reinterpret_cast<double*>(xf + sw.n_xf);
     uint64_t base = 0;
     for (uint32_t i = 0; i < io->n_runs; i++) {
@@ -128,7 +142,7 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
     };
     const auto amp = [](c64* s, uint64_t off) { return reinterpret_cast<c64*>(reinterpret_cast<char*>(s) + off); };
     // the tile's factors before its loads: their tables take 64 registers
-    tile_factors(xf, sw, ops, coef, base, tid);
+    tile_factors(xf, sw, ops, coef, base, stid);
     c64 a[kRegs];
     {
         // in batches of four, so that addresses do not hold registers long
@@ -158,7 +172,7 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
     c64* const stage = reinterpret_cast<c64*>(gacc + sw.n_grad * nwaves + (sw.n_grad * nwaves & 1u));
     if constexpr (kLat) {
         const uint32_t n = lph[ph_begin].coef_n, c0 = lph[ph_begin].coef_begin;
-        for (uint32_t i = tid; i < n; i += nt) stage[i] = coef[c0 + i];
+        for (uint32_t i = stid; i < n; i += snt) stage[i] = coef[c0 + i];
     }
     if (kLat || sw.n_xf) __syncthreads();
     uint64_t le = ltab[size_t(ph_begin) * kLaneEntries + lane];
@@ -177,31 +191,49 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
                 if (cross) __syncthreads();
                 else asm volatile("" ::: "memory");
             };
-            if (flags & LPH_GUARD) __syncthreads();
+            if (whole) {   // (kLat's barrier after a phase's ops is the guard)
 #pragma unroll
-            for (int r = 0; r < kRegs; r++) {
-                lds_at(smem, w ^ L.w[r]) = a[r].re;
-                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-            }
-            meet();
+                for (int r = 0; r < kRegs; r++) {
+                    const uint32_t at = w ^ L.w[r];
+                    lds_at(smem, at) = a[r].re;
+                    lds_at(smem, at + plane) = a[r].im;
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+                meet();
 #pragma unroll
-            for (int r = 0; r < kRegs; r++) {
-                a[r].re = lds_at(smem, rd ^ L.rd[r]);
-                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-            }
-            // fresh copies, or 32 addresses would stay in registers from the first half
-            asm volatile("" : "+v"(w), "+v"(rd));
-            meet();
+                for (int r = 0; r < kRegs; r++) {
+                    const uint32_t at = rd ^ L.rd[r];
+                    a[r].re = lds_at(smem, at);
+                    a[r].im = lds_at(smem, at + plane);
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                if (!kLat && (flags & LPH_GUARD)) __syncthreads();
 #pragma unroll
-            for (int r = 0; r < kRegs; r++) {
-                lds_at(smem, w ^ L.w[r]) = a[r].im;
-                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-            }
-            meet();
+                for (int r = 0; r < kRegs; r++) {
+                    lds_at(smem, w ^ L.w[r]) = a[r].re;
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+                meet();
 #pragma unroll
-            for (int r = 0; r < kRegs; r++) {
-                a[r].im = lds_at(smem, rd ^ L.rd[r]);
-                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                for (int r = 0; r < kRegs; r++) {
+                    a[r].re = lds_at(smem, rd ^ L.rd[r]);
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+                // fresh copies, or 32 addresses would stay in registers from the first half
+                asm volatile("" : "+v"(w), "+v"(rd));
+                meet();
+#pragma unroll
+                for (int r = 0; r < kRegs; r++) {
+                    lds_at(smem, w ^ L.w[r]) = a[r].im;
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+                meet();
+#pragma unroll
+                for (int r = 0; r < kRegs; r++) {
+                    a[r].im = lds_at(smem, rd ^ L.rd[r]);
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
         const uint32_t goff = uint32_t(te >> 32) & 0xffffu, grp = uint32_t(te >> 48);
@@ -223,7 +255,7 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
             }
 #pragma unroll
             for (uint32_t i = 0; i < kPre; i++)
-                pre[i] = coef[tid + nt * i < pre_n ? pre_c + tid + nt * i : 0u];
+                pre[i] = coef[stid + snt * i < pre_n ? pre_c + stid + snt * i : 0u];
             nxt = op->h;
         }
         for (uint32_t o = L.op_begin; o < op_end; o++, op++) {
@@ -256,8 +288,8 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
             c64* const to = stage + ((p + 1 - ph_begin) & 1u) * sw.stage;
 #pragma unroll
             for (uint32_t i = 0; i < kPre; i++)
-                if (tid + nt * i < pre_n) to[tid + nt * i] = c64{pre[i].re, pre[i].im};   // (by value: see k_pauli)
-            for (uint32_t i = tid + nt * kPre; i < pre_n; i += nt) to[i] = coef[pre_c + i];
+                if (stid + snt * i < pre_n) to[stid + snt * i] = c64{pre[i].re, pre[i].im};   // (by value: see k_pauli)
+            for (uint32_t i = stid + snt * kPre; i < pre_n; i += snt) to[i] = coef[pre_c + i];
             __syncthreads();
         }
     }
@@ -323,7 +355,20 @@ k_sweep2(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo sw, const S
                                             smem, false);
 }
 
-constexpr uint64_t kLatTiles = 256;   // sweeps of at most this many tiles run the latency builds
+// Sweeps run the latency build where all their waves fit the chip at its two
+// per SIMD (2^17 threads, a wave per tile at least); where a phase has at most
+// 8 coefficients per thread to stage; and not in the 512-thread tiles of one
+// state on up to 64 CUs, whose two waves per SIMD hide the scalar loads
+// themselves.  Latency / ordinary build: gradient of a 20-qubit ansatz with
+// 11-qubit tiles (2^17 threads) 583 / 695 us, random layers of 22 qubits (2^18)
+// 697 / 516 us; QFT of 20 qubits in 10-qubit tiles (up to 25 coefficients per
+// thread) 164 / 120 us; random layers in 13-qubit tiles at 16 qubits (8 tiles)
+// 174 / 160 us, at 20 (128) 333 / 359 us.
+constexpr uint64_t kLatThreads = 1u << 17;
+constexpr uint32_t kLatStage = 8;
+// LDS of a CU's tiles up to which they exchange whole amplitudes (QFT of 21
+// qubits, one 13-qubit tile of 136 KiB on each CU: 101 us, 94 by halves).
+constexpr size_t kWholeBytes = 96 * 1024;
 static size_t g_max_smem = 64 * 1024;  // dynamic LDS the sweep kernels may use
 
 // --------------------------------------------------------------- batching
@@ -612,25 +657,27 @@ hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L
     return hipGetLastError();
 }
 
-hipError_t launch_sweep(hipStream_t st, int ns, c64* s0, c64* s1, const SweepInfo& sw, const SweepIO* io,
+hipError_t launch_sweep(hipStream_t st, int ns, c64* s0, c64* s1, const SweepInfo& info, const SweepIO* io,
                         const SweepTables& t, double* grad_partials)
 {
-    const uint32_t nt = sweep_threads(sw.k, ns);
+    SweepInfo sw = info;
+    const uint32_t nt = sweep_threads(sw.k, ns), threads = std::max(nt, 64u);
     size_t smem = sweep_smem_bytes(sw, ns);
-    // at most one tile per CU (256): the latency build, if the phases'
-    // coefficients fit its stage (blocks of three and four register qubits
-    // from LDS would not fit its registers)
-    const bool lat = sw.max_dense <= 2 && sw.n_tiles <= kLatTiles && sw.stage <= kMaxStage && smem + 8 + 32 * sw.stage <= g_max_smem;
-    if (lat) smem += 8 + 32 * sw.stage;
+    const size_t lat_smem = smem + 8 + 32 * sw.stage, whole = (size_t(8) << sw.k) * ns;
+    // (blocks of three and four register qubits from LDS would not fit its registers)
+    const bool lat = sw.max_dense <= 2 && sw.n_tiles * threads <= kLatThreads && sw.stage <= kLatStage * threads &&
+                     !(ns == 1 && nt == 512 && sw.n_tiles <= 64) && lat_smem <= g_max_smem;
+    sw.whole = lat && (lat_smem + whole) * ((sw.n_tiles + 255) / 256) <= kWholeBytes ? 1u : 0u;
+    if (lat) smem = lat_smem + (sw.whole ? whole : 0);
     if (smem > g_max_smem || nt > uint32_t(kMaxTileThreads)) return hipErrorInvalidConfiguration;
     const uint64_t max_grid = 1ull << 30;
     for (uint64_t t0 = 0; t0 < sw.n_tiles; t0 += max_grid) {
         const uint64_t cnt = sw.n_tiles - t0 < max_grid ? sw.n_tiles - t0 : max_grid;
         if (ns == 1) {
             auto* fn = lat ? &k_sweep1<2, true> : sw.max_dense <= 2 ? &k_sweep1<2, false> : &k_sweep1<kRegBits, false>;
-            hipLaunchKernelGGL(fn, dim3(uint32_t(cnt)), dim3(nt), smem, st, s0, sw, io, SVMI_TABLES_OF(t), t0);
+            hipLaunchKernelGGL(fn, dim3(uint32_t(cnt)), dim3(lat ? threads : nt), smem, st, s0, sw, io, SVMI_TABLES_OF(t), t0);
         } else {
-            hipLaunchKernelGGL(lat ? &k_sweep2<true> : &k_sweep2<false>, dim3(uint32_t(cnt)), dim3(nt), smem, st, s0,
+            hipLaunchKernelGGL(lat ? &k_sweep2<true> : &k_sweep2<false>, dim3(uint32_t(cnt)), dim3(lat ? threads : nt), smem, st, s0,
                                s1, sw, io, SVMI_TABLES_OF(t), grad_partials, t0);
         }
     }
