@@ -43,8 +43,8 @@ svmi_status svmi_debug_plan_batch(const svmi_batch_item* items, size_t n_items, 
                                   uint64_t* n_launches, uint64_t* n_tasks, uint64_t* state_bytes);
 
 /* Coefficients of the batch's plan, and the largest offset (in coefficients)
- * that a sweep adds in 32 bits of bytes to the base it reads an op's
- * coefficients from: below 2^28 minus the largest op's own coefficients. */
+ * of an op's first one from its sweep's, which the sweeps add as 32 bits of
+ * bytes. */
 svmi_status svmi_debug_batch_coefs(const svmi_batch_item* items, size_t n_items, uint64_t* n_coefs,
                                    uint64_t* max_offset);
 

@@ -430,7 +430,8 @@ svmi_status verify_batch(const BatchPlan& bp)
             if (two && b.partial + sw.n_tiles * sw.n_grad > bp.n_grad_partials)
                 return fail(SVMI_ERR_STATE, "batch plan: bad gradient partial range");
             if (sw.op_begin > sw.op_end || sw.op_end > bp.ops.size() || sw.n_xf > uint32_t(kMaxXfSlots) ||
-                16u * sw.n_lt > sw.n_xf || sw.lt_coef + 16ull * sw.n_lt > bp.coef.size())
+                16u * sw.n_lt > sw.n_xf || sw.coef_base > bp.coef.size() ||
+                sw.lt_coef + 16ull * sw.n_lt > bp.coef.size() - sw.coef_base)
                 return fail(SVMI_ERR_STATE, "batch plan: bad sweep op range");
             for (uint32_t o = sw.op_begin; o < sw.op_end; o++)
                 if ((has_tile_factor(bp.ops[o].h) && bp.ops[o].h.grad >= sw.n_xf) ||
@@ -444,10 +445,10 @@ svmi_status verify_batch(const BatchPlan& bp)
                 if (L.op_begin > L.op_end ||
                     (L.op_begin < L.op_end && (L.op_begin < sw.op_begin || L.op_end > sw.op_end)))
                     return fail(SVMI_ERR_STATE, "batch plan: bad phase");
-                if (uint64_t(L.coef_begin) + L.coef_n > bp.coef.size())
+                if (uint64_t(L.coef_begin) + L.coef_n > bp.coef.size() - sw.coef_base)
                     return fail(SVMI_ERR_STATE, "batch plan: bad coefficient range");
                 for (uint32_t o = L.op_begin; o < L.op_end; o++)
-                    if (bp.ops[o].h.coef >= kMaxPhaseCoefs || bp.ops[o].h.coef > L.coef_n)
+                    if (bp.ops[o].h.coef > bp.coef.size() - sw.coef_base)
                         return fail(SVMI_ERR_STATE, "batch plan: bad coef offset");
             }
         } else if (b.kind == BSTEP_PAULI) {
@@ -544,14 +545,10 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
         const uint32_t op_base = uint32_t(bp.ops.size()), coef_base = uint32_t(bp.coef.size());
         const uint32_t lp_base = uint32_t(bp.lphases.size());
         const uint32_t sw_base = uint32_t(bp.sweeps.size());
-        for (DOp d : pr.ops) {
-            if (has_tile_factor(d.h)) d.qphys[0] += coef_base;
-            bp.ops.push_back(d);
-        }
+        bp.ops.insert(bp.ops.end(), pr.ops.begin(), pr.ops.end());
         for (LayoutPhase L : pr.lphases) {
             L.op_begin += op_base;
             L.op_end += op_base;
-            L.coef_begin += coef_base;
             bp.lphases.push_back(L);
         }
         for (SweepIO io : pr.io) {
@@ -562,7 +559,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
         for (SweepInfo sw : pr.sweeps) {
             sw.op_begin += op_base;
             sw.op_end += op_base;
-            sw.lt_coef += coef_base;
+            sw.coef_base += coef_base;
             bp.sweeps.push_back(sw);
         }
         bp.coef.insert(bp.coef.end(), pr.coef.begin(), pr.coef.end());
@@ -1854,13 +1851,13 @@ void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, c
 {
     const uint32_t nt = sweep_threads(sw.k, ns);
     for (uint32_t i = 0; i < sw.n_grad; i++) gsum_tile[i] = 0.0;
+    coef += sw.coef_base;
     const uint64_t base = tile_base(sw, tile);
     std::vector<c64> xf(std::max<uint32_t>(sw.n_xf, 1));
     const uint64_t xbits = ext_index(sw, base);
     for (uint32_t i = 0; i < 16u * sw.n_lt; i++) xf[sw.n_xf - 16u * sw.n_lt + i] = coef[sw.lt_coef + i];
     for (uint32_t o = sw.op_begin; o < sw.op_end; o++)
-        if (has_tile_factor(ops[o].h))
-            xf[ops[o].h.grad] = tile_factor(ops[o].h, coef + ops[o].qphys[0], base, xbits);
+        if (has_tile_factor(ops[o].h)) xf[ops[o].h.grad] = tile_factor(ops[o].h, coef, base, xbits);
     struct Group {
         c64 a[kRegs];
     };
@@ -1914,15 +1911,14 @@ void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, c
             g.swap(h);
         }
         const RegOffsets off{L.rcol};
-        const c64* cf = coef + L.coef_begin;
         for (uint32_t t = 0; t < nt; t++) {
             const uint32_t goff = uint32_t(entry(t) >> 32) & 0xffffu, grp = uint32_t(entry(t) >> 48);
             for (uint32_t o = L.op_begin; o < L.op_end; o++) {
                 const DOp& op = ops[o];
                 if (op.h.type == DOP_GRAD_DENSE || op.h.type == DOP_GRAD_DIAG)
-                    gsum_tile[op.h.grad] += exec_grad_op<kRegBits, kRegsAdj>(op.h, &op, g[t].a, cf, goff, off, base);
+                    gsum_tile[op.h.grad] += exec_grad_op<kRegBits, kRegsAdj>(op.h, &op, g[t].a, coef, goff, off, base);
                 else
-                    exec_state_op(op.h, &op, g[t].a, cf, goff, grp, off, base, xf.data(), sw.exthi, vhi);
+                    exec_state_op(op.h, &op, g[t].a, coef, goff, grp, off, base, xf.data(), sw.exthi, vhi);
             }
         }
     }

@@ -294,11 +294,10 @@ SVMI_HD inline void apply_phasetab(const DOpHdr& h, c64 (&a)[N], const c64* __re
 // The tile base's bits outside the tile, packed in ascending qubit order.
 SVMI_HD inline uint64_t ext_index(const SweepInfo& sw, uint64_t base) { return extract_bits(base, sw.extmask); }
 
-// Factor slot of a DOP_PHASETAB op (own: its coefficients) for the tile with
-// external bits x.
-SVMI_HD inline c64 phasetab_factor(const DOpHdr& h, const c64* __restrict__ own, uint64_t x)
+// Factor slot of a DOP_PHASETAB op for the tile with external bits x.
+SVMI_HD inline c64 phasetab_factor(const DOpHdr& h, const c64* __restrict__ coef, uint64_t x)
 {
-    const c64* E = own + 16u * h.s0;
+    const c64* E = coef + h.coef + 16u * h.s0;
     c64 f{1.0, 0.0};
     if (h.smask == 0) return f;
     // every table's entry is loaded before the first product, so the loads
@@ -313,11 +312,11 @@ SVMI_HD inline c64 phasetab_factor(const DOpHdr& h, const c64* __restrict__ own,
     return f;
 }
 
-// Factor slot of a DOP_PHASESET op (own: its coefficients) for the tile at
-// `base`: the product of its h.s1 entries that follow the per-lane ones.
-SVMI_HD inline c64 phase_factor(const DOpHdr& h, const c64* __restrict__ own, uint64_t base)
+// Factor slot of a DOP_PHASESET op for the tile at `base`: the product of
+// its h.s1 entries that follow the per-lane ones.
+SVMI_HD inline c64 phase_factor(const DOpHdr& h, const c64* __restrict__ coef, uint64_t base)
 {
-    const PhaseEntry* pe = reinterpret_cast<const PhaseEntry*>(own) + h.s0;
+    const PhaseEntry* pe = reinterpret_cast<const PhaseEntry*>(coef + h.coef) + h.s0;
     double pr = 1.0, pi = 0.0;
     for (uint32_t e = 0; e < h.s1; e++) {
         const PhaseEntry E = pe[e];
@@ -330,11 +329,11 @@ SVMI_HD inline c64 phase_factor(const DOpHdr& h, const c64* __restrict__ own, ui
     return c64{pr, pi};
 }
 
-// The tile factor of op h (DOP_PHASESET / DOP_PHASETAB with s1, own: its
-// coefficients) for the tile at `base` with external bits x.
-SVMI_HD inline c64 tile_factor(const DOpHdr& h, const c64* __restrict__ own, uint64_t base, uint64_t x)
+// The tile factor of op h (DOP_PHASESET / DOP_PHASETAB with s1) for the
+// tile at `base` with external bits x.
+SVMI_HD inline c64 tile_factor(const DOpHdr& h, const c64* __restrict__ coef, uint64_t base, uint64_t x)
 {
-    return h.type == DOP_PHASETAB ? phasetab_factor(h, own, x) : phase_factor(h, own, base);
+    return h.type == DOP_PHASETAB ? phasetab_factor(h, coef, x) : phase_factor(h, coef, base);
 }
 
 // DOP_ROT: optional register table, then the lifts of the slots in smask.

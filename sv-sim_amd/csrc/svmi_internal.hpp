@@ -104,6 +104,7 @@ constexpr int kThreads = 256;               // threads of the reduction / Pauli 
 constexpr int kMaxTileThreads = 1 << (kMaxTileQubits - kRegBits);   // 512
 constexpr int kMaxDenseQubits = 5;          // standalone dense ops
 constexpr int kMaxGradsPerSweep = 256;      // adjoint accumulators per sweep (LDS)
+constexpr size_t kMaxSweepOps = size_t(1) << 18;   // lowered ops of a sweep (coef_at)
 
 // Device op types.
 enum DOpType : uint16_t {
@@ -178,8 +179,7 @@ struct DOpHdr {
     uint32_t type;
     uint32_t smask;      // DENSE / GRAD_DENSE: register slot mask
     uint32_t s0, s1;     // X/CX/SWAP/SRN slots
-    uint32_t coef;       // first coefficient (c64 units), counted from LayoutPhase::coef_begin;
-                         // 0 for ops without one
+    uint32_t coef;       // first coefficient (c64 units), counted from SweepInfo::coef_base
     uint32_t grad;       // GRAD_*: accumulator slot within the sweep
     uint32_t rsel;       // CPHASE/DIAG/CDENSE: registers rho whose register bits satisfy the op
     uint32_t gmask;      // CPHASE/DIAG/CDENSE: non-register tile-local bits that must be 1
@@ -222,8 +222,7 @@ struct DOp {
     uint32_t nq;         // DIAG: number of qubits
     uint32_t targets;    // adjoint: DOP_TO_* (forward sweeps: DOP_TO_PSI)
     int32_t qloc[5];     // DIAG: tile-local bit of qubit i, or -1 if outside the tile
-    uint32_t qphys[5];   // DIAG: physical position of qubit i; ops with a tile factor:
-                         // qphys[0] is the first coefficient counted from the program's
+    uint32_t qphys[5];   // DIAG: physical position of qubit i
 };
 static_assert(sizeof(DOpHdr) == 40 && sizeof(DOp) == 88, "DOp layout");
 
@@ -271,6 +270,7 @@ struct SweepInfo {
     uint32_t op_end;
     uint32_t max_dense;  // register qubits of the sweep's widest DOP_DENSE (0 = none): sweeps
                          // with max_dense <= 2 run a kernel compiled without wider blocks
+    uint32_t coef_base;  // the sweep's first coefficient: its ops, phases and lt_coef count from it
     uint32_t lt_coef;    // coef offset of a contiguous copy of those lane tables (16 c64 each),
     uint32_t n_lt;       // which every tile copies into the end of its factor area
     uint32_t mapped;     // some phase or the tile's store goes through a tile map M
@@ -311,7 +311,7 @@ struct LayoutPhase {
     uint32_t w[kRegs], rd[kRegs];   // exchange before the phase: LDS byte offset of each register
     uint32_t op_begin, op_end;
     uint32_t flags;                 // LPH_*
-    uint32_t coef_n;                // the phase's coefficients: [coef_begin, coef_begin + coef_n)
+    uint32_t coef_n;                // the phase's coefficients: [coef_begin, coef_begin + coef_n) of the sweep's
     uint32_t rcol[4];               // 1 << register bit (tile-local; two states: the last is 1 << k)
     uint32_t coef_begin;
     uint32_t pad[3];
@@ -408,13 +408,10 @@ struct SlotMask {
     }
 };
 
-// Coefficients of one phase before another phase of the same registers begins
-// (svmi_layout.cpp): an op's first one is below this, so byte offsets from a
-// phase's first coefficient fit 32 bits however many the program has.
-constexpr uint32_t kMaxPhaseCoefs = 1u << 16;
-
 // coef + i as base and 32-bit byte offset (one scalar shift instead of a
-// 64-bit shift and add per access).  coef: the phase's first coefficient.
+// 64-bit shift and add per access).  coef: the sweep's first coefficient; a
+// sweep takes at most kMaxSweepOps ops of well under 1024 coefficients each,
+// so the offset fits however many the program has.
 SVMI_HD inline const c64* coef_at(const c64* coef, uint32_t i)
 {
     return reinterpret_cast<const c64*>(reinterpret_cast<const char*>(coef) + uint32_t(i * 16u));

@@ -49,8 +49,8 @@ std::string variant(uint64_t emask, const SweepInfo& sw)
 // Coefficient offsets count from the program's first one.
 void emit_state_op(std::ostringstream& o, DOp d, const LayoutPhase& ph, const SweepInfo& sw)
 {
-    d.h.coef += ph.coef_begin;
-    if (d.h.type == DOP_ROT && d.h.s0) d.h.grad += ph.coef_begin;   // its table
+    d.h.coef += sw.coef_base;
+    if (d.h.type == DOP_ROT && d.h.s0) d.h.grad += sw.coef_base;   // its table
     const DOpHdr& h = d.h;
     const std::string cond = "(base & " + std::to_string(h.emask) + "ull) == " + std::to_string(h.emask) +
                              "ull && (goff & " + std::to_string(h.gmask) + "u) == " + std::to_string(h.gmask) + "u";
@@ -251,11 +251,11 @@ void emit_sweep(std::ostringstream& o, const Program& prog, uint32_t i)
         const uint32_t nlt = 16u * sw.n_lt;
         if (nlt)
             o << "    for (uint32_t i = tid; i < " << nlt << "u; i += " << nt << "u) xf[" << (sw.n_xf - nlt)
-              << "u + i] = coef[" << sw.lt_coef << "u + i];\n";
+              << "u + i] = coef[" << (sw.coef_base + sw.lt_coef) << "u + i];\n";
         o << "    const uint64_t xbits = extract_bits(base, " << sw.extmask << "ull);\n"
           << "    for (uint32_t o = " << sw.op_begin << "u + tid; o < " << sw.op_end << "u; o += " << nt << "u) {\n"
           << "        const DOpHdr h = ops[o].h;\n"
-          << "        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef + ops[o].qphys[0], base, xbits);\n    }\n";
+          << "        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef + " << sw.coef_base << "u, base, xbits);\n    }\n";
     }
     o << "    c64 a[kRegs];\n";
     emit_io(o, io, 0, nt);

@@ -58,7 +58,7 @@ tile_factors(c64* xf, const SweepInfo& sw, const DOp* __restrict__ ops, const c6
     const uint64_t x = ext_index(sw, base);
     for (uint32_t o = sw.op_begin + tid; o < sw.op_end; o += blockDim.x) {
         const DOpHdr h = ops[o].h;
-        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef + ops[o].qphys[0], base, x);
+        if (has_tile_factor(h)) xf[h.grad] = tile_factor(h, coef, base, x);
     }
 }
 
@@ -124,6 +124,7 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
     const uint32_t lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nwaves = (nt + 63) / 64;
+    coef += sw.coef_base;
     const uint32_t plane = uint32_t(8 * NS) << sw.k;
     const bool whole = kLat && sw.whole;   // uniform
     c64* xf = reinterpret_cast<c64*>(smem + (size_t(plane) << (whole ? 1 : 0)));
@@ -243,7 +244,7 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
         // kLat: this phase's coefficients in one half of the stage; the next
         // one's are on their way, up to kPre per thread in registers
         constexpr uint32_t kPre = 4;
-        const c64* __restrict__ cf = coef + L.coef_begin;
+        const c64* __restrict__ cf = coef;
         c64 pre[kLat ? kPre : 1];
         uint32_t pre_n = 0, pre_c = 0;
         DOpHdr nxt;
@@ -263,6 +264,8 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
             if constexpr (kLat) {   // (op arrays end with an unused record)
                 h = nxt;
                 nxt = op[1].h;
+                if (h.type == DOP_ROT && h.s0) h.grad -= L.coef_begin;   // its table
+                h.coef -= L.coef_begin;
             } else {
                 h = op->h;
             }

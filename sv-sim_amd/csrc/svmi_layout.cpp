@@ -149,16 +149,15 @@ struct Builder {
         for (int s = 0; s < kRegBits; s++) col[t + s] = p.sreg[s];
     }
 
-    // The phase pi, cut where an op's coefficients would begin kMaxPhaseCoefs or
-    // more after the part's: the parts after the first one hold the same
-    // amplitudes in the same registers, so the exchange between them moves
-    // nothing.  The ops' coefficient offsets become relative to their part's.
     void take(const PhaseInfo& pi)
     {
         Phase p;
         p.op_begin = pi.op_begin;
-        p.coef_begin = pi.coef_begin;
+        p.op_end = pi.op_end;
+        p.coef_begin = pi.coef_begin - sw.coef_base;
+        p.coef_end = pi.coef_end - sw.coef_base;
         p.gx = pi.gxor;
+        p.sx = pi.sxor;
         uint32_t R = 0;
         for (int s = 0; s < kRegBits; s++) {
             p.r[s] = pi.r[s];
@@ -172,32 +171,7 @@ struct Builder {
                 p.grp[gi] = Group{pi.gm[gi], 1u << l, 1u << gi};
                 gi++;
             }
-        for (uint32_t o = pi.op_begin; o < pi.op_end; o++) {
-            DOp& d = prog.ops[o];
-            if (!has_coef(d.h)) continue;
-            if (d.h.coef - p.coef_begin >= kMaxPhaseCoefs) {
-                p.op_end = o;
-                p.coef_end = d.h.coef;
-                ph.push_back(p);
-                p.op_begin = o;
-                p.coef_begin = d.h.coef;
-                p.gx = 0;
-                for (int s = 0; s < kRegBits; s++) p.greg[s] = p.sreg[s];
-            }
-            if (has_tile_factor(d.h)) d.qphys[0] = d.h.coef;
-            if (d.h.type == DOP_ROT && d.h.s0) d.h.grad -= p.coef_begin;   // its table
-            d.h.coef -= p.coef_begin;
-        }
-        p.op_end = pi.op_end;
-        p.coef_end = pi.coef_end;
-        p.sx = pi.sxor;
         ph.push_back(p);
-    }
-
-    static bool has_coef(const DOpHdr& h)
-    {
-        constexpr uint32_t none = 1u << DOP_NOP | 1u << DOP_X | 1u << DOP_CX | 1u << DOP_SWAP | 1u << DOP_SRN;
-        return !((none >> h.type) & 1u);
     }
 
     // a phase without ops on the columns col[0..K): lanes and waves first, then registers

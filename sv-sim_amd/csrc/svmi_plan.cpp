@@ -1278,6 +1278,7 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
     sw.c = uint32_t(c);
     sw.phase_begin = uint32_t(prog.phases.size());
     sw.op_begin = uint32_t(prog.ops.size());
+    sw.coef_base = uint32_t(prog.coef.size());
     sw.n_ext = 0;
     sw.extmask = 0;
     for (int p = 0; p < n; p++)
@@ -1566,7 +1567,7 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
         for (size_t o = sw.op_begin; o < prog.ops.size(); o++)
             if (prog.ops[o].h.type == DOP_PHASETAB) ntab += prog.ops[o].h.s0;
         if (ntab && sw.n_xf + 16u * ntab <= uint32_t(kMaxXfSlots)) {
-            sw.lt_coef = uint32_t(prog.coef.size());
+            sw.lt_coef = uint32_t(prog.coef.size()) - sw.coef_base;
             sw.n_lt = ntab;
             uint32_t slot = sw.n_xf;
             for (size_t o = sw.op_begin; o < prog.ops.size(); o++) {
@@ -1581,6 +1582,13 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
         }
     }
     sw.op_end = uint32_t(prog.ops.size());
+    for (uint32_t o = sw.op_begin; o < sw.op_end; o++) {   // offsets from the sweep's first coefficient
+        DOpHdr& h = prog.ops[o].h;
+        constexpr uint32_t none = 1u << DOP_NOP | 1u << DOP_X | 1u << DOP_CX | 1u << DOP_SWAP | 1u << DOP_SRN;
+        if ((none >> h.type) & 1u) continue;
+        h.coef -= sw.coef_base;
+        if (h.type == DOP_ROT && h.s0) h.grad -= sw.coef_base;   // its table
+    }
     prog.n_grad += n_grad_sweep;
     // The coefficients a tile reads while it runs the sweep go through the
     // small scalar cache that a few CUs share; when their total exceeds
@@ -1684,7 +1692,7 @@ void schedule(std::vector<SOp>& sops, int n, const PlanOptions& opt, Program& pr
             const SOp* s = pending[i];
             if (blocked == all) break;
             const bool over = (opt.sweep_budget > 0 && cost >= opt.sweep_budget && !taken.empty()) ||
-                              (s->grad && grads >= kMaxGradsPerSweep);
+                              (s->grad && grads >= kMaxGradsPerSweep) || taken.size() >= kMaxSweepOps;
             if ((s->dep & blocked) || s->standalone || over) {
                 blocked |= s->dep;
                 if (over) blocked = all;

@@ -412,7 +412,7 @@ def plan_batch(items):
 
 
 def batch_coefs(items):
-    """(coefficients of the batch plan, largest offset of an op's first one from its phase's)."""
+    """(coefficients of the batch plan, largest offset of an op's first one from its sweep's)."""
     arr, keep, _ = _batch_items(items)
     v = [ctypes.c_uint64() for _ in range(2)]
     _check(lib().svmi_debug_batch_coefs(ctypes.cast(arr, _vp), len(items), *[ctypes.byref(x) for x in v]))
