@@ -54,8 +54,7 @@ bool gf2_insert(uint32_t (&basis)[32], uint32_t v)
 // the (thread, register) columns of the writes and of the reads are
 // independent and below the exchange area's size, and the loads and stores
 // reach every tile qubit and no other.
-bool layout_valid(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, const uint64_t* lane_tab,
-                  const uint64_t* wave_tab, bool two)
+bool layout_valid(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, const ThreadCols* cols, bool two)
 {
     const uint32_t K = sw.k + (two ? 1u : 0u), t = K - kRegBits;
     const uint32_t tl = std::min<uint32_t>(t, kLaneBits), tw = t - tl;
@@ -85,22 +84,21 @@ bool layout_valid(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph
             return false;
     }
     for (uint32_t p = io.ph_begin + 1; p < io.ph_end; p++) {
-        const uint64_t* lt = lane_tab + size_t(p) * kLaneEntries;
-        const uint64_t* wt = wave_tab + size_t(p) * kWaveEntries;
+        const ThreadCols& tc = cols[p];
         for (int rd = 0; rd < 2; rd++) {
             uint32_t basis[32] = {};
             const auto ok = [&](uint32_t v) { return !(v & 7u) && v < (8u << K) && gf2_insert(basis, v); };
             for (uint32_t i = 0; i < tl; i++)
-                if (!ok(uint32_t(lt[1u << i] >> (16 * rd)) & 0xffffu)) return false;
+                if (!ok(uint32_t(tc.lane[i] >> (16 * rd)) & 0xffffu)) return false;
             for (uint32_t i = 0; i < tw; i++)
-                if (!ok(uint32_t((wt[1u << i] ^ wt[0]) >> (16 * rd)) & 0xffffu)) return false;
+                if (!ok(uint32_t(tc.wave[i] >> (16 * rd)) & 0xffffu)) return false;
             const uint32_t* reg = rd ? lph[p].rd : lph[p].w;
             for (int s = 0; s < kRegBits; s++)
                 if (!ok(reg[1u << s])) return false;
             for (int r = 0; r < kRegs; r++)
                 if (reg[r] >= (8u << K)) return false;
         }
-        if ((uint32_t(wt[0]) >> 16) >= (8u << K)) return false;
+        if ((uint32_t(tc.zero) >> 16) >= (8u << K)) return false;
     }
     return true;
 }
@@ -195,9 +193,20 @@ struct DeviceProgram {
         o_ops = put(p.ops, sizeof(DOp));
         o_coef = put(p.coef, 16);
         o_lph = put(p.lphases, 16);
-        o_lane = put(p.lane_tab, 16);
-        o_wave = put(p.wave_tab, 16);
         o_io = put(p.io, 16);
+        o_lane = (host.size() + 255) & ~size_t(255);
+        o_wave = o_lane + p.cols.size() * kLaneEntries * 8;
+        host.resize(o_wave + p.cols.size() * kWaveEntries * 8 + 16);
+        uint64_t* lane = reinterpret_cast<uint64_t*>(host.data() + o_lane);
+        uint64_t* wave = reinterpret_cast<uint64_t*>(host.data() + o_wave);
+        for (const ThreadCols& c : p.cols) {
+            *lane++ = 0;
+            for (uint32_t v = 1; v < uint32_t(kLaneEntries); v++, lane++)
+                *lane = lane[-int(v & (~v + 1))] ^ c.lane[__builtin_ctz(v)];
+            *wave++ = c.zero;
+            for (uint32_t v = 1; v < uint32_t(kWaveEntries); v++, wave++)
+                *wave = wave[-int(v & (~v + 1))] ^ c.wave[__builtin_ctz(v)];
+        }
         SVMI_TRY(buf.ensure(host.size()));
         SVMI_HIP(hipMemcpyAsync(buf.p, host.data(), host.size(), hipMemcpyHostToDevice, st));
         SVMI_HIP(hipStreamSynchronize(st));
@@ -352,7 +361,7 @@ struct BatchPlan {
     std::vector<SweepInfo> sweeps;
     std::vector<SweepIO> io;
     std::vector<LayoutPhase> lphases;
-    std::vector<uint64_t> lane_tab, wave_tab;
+    std::vector<ThreadCols> cols;
     std::vector<DOp> ops;
     std::vector<c64> coef;
     std::vector<PauliGroup> groups;
@@ -438,7 +447,7 @@ svmi_status verify_batch(const BatchPlan& bp)
                     (bp.ops[o].h.type == DOP_PHASETAB && bp.ops[o].h.gmask != kLaneTabGlobal &&
                      uint64_t(bp.ops[o].h.gmask) + 16ull * bp.ops[o].h.s0 > sw.n_xf))
                     return fail(SVMI_ERR_STATE, "batch plan: bad phase factor slot");
-            if (!layout_valid(sw, io, bp.lphases.data(), bp.lane_tab.data(), bp.wave_tab.data(), two))
+            if (!layout_valid(sw, io, bp.lphases.data(), bp.cols.data(), two))
                 return fail(SVMI_ERR_STATE, "batch plan: bad register layout");
             for (uint32_t p = io.ph_begin; p < io.ph_end; p++) {
                 const LayoutPhase& L = bp.lphases[p];
@@ -531,16 +540,23 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                                     ": an op does not fit a tile (a 5-qubit gate such as C4X, or a tile too small "
                                     "for the 4 low qubits plus the op's qubits)");
     // the chunk's tables are indexed with 32 bits
-    uint64_t n_ops = 0, n_coefs = 0, n_phases = 0;
+    uint64_t n_ops = 0, n_coefs = 0, n_phases = 0, n_sweeps = 0;
     for (size_t i = 0; i < n_items; i++)
         for (const Program* pr : {&bp.fwd[i], &bp.adj[i]}) {
             n_ops += pr->ops.size();
             n_coefs += pr->coef.size();
             n_phases += pr->lphases.size();
+            n_sweeps += pr->sweeps.size();
         }
     if (std::max({n_ops, n_coefs, n_phases}) > UINT32_MAX)
         return fail(SVMI_ERR_UNSUPPORTED, "batch: more than 2^32 ops or coefficients planned together; give the "
                                           "circuits to several calls");
+    bp.ops.reserve(n_ops + 1);
+    bp.coef.reserve(n_coefs);
+    bp.lphases.reserve(n_phases);
+    bp.cols.reserve(n_phases);
+    bp.sweeps.reserve(n_sweeps);
+    bp.io.reserve(n_sweeps);
     auto append_program = [&](const Program& pr) {
         const uint32_t op_base = uint32_t(bp.ops.size()), coef_base = uint32_t(bp.coef.size());
         const uint32_t lp_base = uint32_t(bp.lphases.size());
@@ -563,8 +579,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
             bp.sweeps.push_back(sw);
         }
         bp.coef.insert(bp.coef.end(), pr.coef.begin(), pr.coef.end());
-        bp.lane_tab.insert(bp.lane_tab.end(), pr.lane_tab.begin(), pr.lane_tab.end());
-        bp.wave_tab.insert(bp.wave_tab.end(), pr.wave_tab.begin(), pr.wave_tab.end());
+        bp.cols.insert(bp.cols.end(), pr.cols.begin(), pr.cols.end());
         return sw_base;
     };
     bp.circs.resize(n_items);
@@ -1615,11 +1630,11 @@ svmi_status svmi_batch_adjoint(int device, const svmi_batch_item* items, size_t 
         std::vector<size_t> idx;                  // original item indices
         std::vector<svmi_batch_item> items;
         BatchPlan bp;
-        DevBuf dsteps, dcircs, dsweeps, dio, dlph, dlane, dwave, dops, dcoef, dgroups, dterms, dpart, dsegs, dout;
+        DevBuf dsteps, dcircs, dsweeps, dio, dlph, dcols, dlane, dwave, dops, dcoef, dgroups, dterms, dpart, dsegs, dout;
         void release()
         {
-            for (DevBuf* b : {&dsteps, &dcircs, &dsweeps, &dio, &dlph, &dlane, &dwave, &dops, &dcoef, &dgroups, &dterms,
-                              &dpart, &dsegs, &dout})
+            for (DevBuf* b : {&dsteps, &dcircs, &dsweeps, &dio, &dlph, &dcols, &dlane, &dwave, &dops, &dcoef, &dgroups,
+                              &dterms, &dpart, &dsegs, &dout})
                 b->release();
         }
     };
@@ -1657,8 +1672,11 @@ svmi_status svmi_batch_adjoint(int device, const svmi_batch_item* items, size_t 
         SVMI_TRY(put(k.dsweeps, bp.sweeps.data(), bp.sweeps.size() * sizeof(SweepInfo)));
         SVMI_TRY(put(k.dio, bp.io.data(), bp.io.size() * sizeof(SweepIO)));
         SVMI_TRY(put(k.dlph, bp.lphases.data(), bp.lphases.size() * sizeof(LayoutPhase)));
-        SVMI_TRY(put(k.dlane, bp.lane_tab.data(), bp.lane_tab.size() * sizeof(uint64_t)));
-        SVMI_TRY(put(k.dwave, bp.wave_tab.data(), bp.wave_tab.size() * sizeof(uint64_t)));
+        SVMI_TRY(put(k.dcols, bp.cols.data(), bp.cols.size() * sizeof(ThreadCols)));
+        SVMI_TRY(k.dlane.ensure(std::max<size_t>(bp.cols.size() * kLaneEntries * 8, 16)));
+        SVMI_TRY(k.dwave.ensure(std::max<size_t>(bp.cols.size() * kWaveEntries * 8, 16)));
+        SVMI_HIP(launch_thread_tables(st, k.dcols.as<ThreadCols>(), bp.cols.size(), k.dlane.as<uint64_t>(),
+                                      k.dwave.as<uint64_t>()));
         SVMI_TRY(put(k.dops, bp.ops.data(), bp.ops.size() * sizeof(DOp)));
         SVMI_TRY(put(k.dcoef, bp.coef.data(), bp.coef.size() * sizeof(c64)));
         SVMI_TRY(put(k.dgroups, bp.groups.data(), bp.groups.size() * sizeof(PauliGroup)));
@@ -1845,8 +1863,7 @@ void host_standalone(std::vector<c64>& s, int n, const StandaloneOp& so, const s
 // holds the real parts, then the imaginary ones).  An exchange without
 // LPH_CROSS that reads another wave's slot, a slot written twice or never
 // throws.  gsum_tile receives the tile's gradient accumulators (ns == 2).
-void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, const uint64_t* lane_tab,
-               const uint64_t* wave_tab, const DOp* ops, const c64* coef, int ns, c64* s0, c64* s1, uint64_t tile,
+void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, const ThreadCols* cols, const DOp* ops, const c64* coef, int ns, c64* s0, c64* s1, uint64_t tile,
                bool init_zero, double* gsum_tile)
 {
     const uint32_t nt = sweep_threads(sw.k, ns);
@@ -1881,11 +1898,11 @@ void host_tile(const SweepInfo& sw, const SweepIO& io, const LayoutPhase* lph, c
         }
     const uint32_t slots = (1u << sw.k) * uint32_t(ns);
     std::vector<uint32_t> by(slots);   // writer (thread * 16 + register) of a slot
+    std::vector<uint64_t> entries(nt);
     for (uint32_t p = io.ph_begin; p < io.ph_end; p++) {
         const LayoutPhase& L = lph[p];
-        const auto entry = [&](uint32_t t) {
-            return lane_tab[size_t(p) * kLaneEntries + (t & 63u)] ^ wave_tab[size_t(p) * kWaveEntries + (t >> 6)];
-        };
+        for (uint32_t t = 0; t < nt; t++) entries[t] = lane_entry(cols[p], t & 63u) ^ wave_entry(cols[p], t >> 6);
+        const auto entry = [&](uint32_t t) { return entries[t]; };
         const auto slot = [&](uint32_t b, const uint32_t (&reg)[kRegs], int r) {
             b ^= reg[r];
             if ((b & 7u) || (b >> 3) >= slots) throw std::logic_error("layout: slot out of range");
@@ -1983,7 +2000,7 @@ void host_program(Program& prog, std::vector<c64>& s0, std::vector<c64>& s1, std
         const SweepInfo& sw = prog.sweeps[st.index];
         std::vector<double> g(sw.n_grad);
         for (uint64_t tile = 0; tile < sw.n_tiles; tile++) {
-            host_tile(sw, prog.io[st.index], prog.lphases.data(), prog.lane_tab.data(), prog.wave_tab.data(),
+            host_tile(sw, prog.io[st.index], prog.lphases.data(), prog.cols.data(),
                       prog.ops.data(), prog.coef.data(), ns, s0.data(), ns == 2 ? s1.data() : nullptr, tile, false,
                       g.data());
             for (uint32_t i = 0; i < sw.n_grad; i++) gsum[sw.grad_base + i] += g[i];
@@ -2124,7 +2141,7 @@ svmi_status svmi_debug_emulate_batch(const svmi_batch_item* items, size_t n_item
             if (st.kind == BSTEP_FWD || st.kind == BSTEP_ADJ) {
                 const SweepInfo& sw = bp.sweeps[st.sweep];
                 std::vector<double> g(sw.n_grad);
-                host_tile(sw, bp.io[st.sweep], bp.lphases.data(), bp.lane_tab.data(), bp.wave_tab.data(),
+                host_tile(sw, bp.io[st.sweep], bp.lphases.data(), bp.cols.data(),
                           bp.ops.data(), bp.coef.data(), st.kind == BSTEP_ADJ ? 2 : 1, ph,
                           st.kind == BSTEP_ADJ ? lm : nullptr, task, L.init != 0, g.data());
                 for (uint32_t i = 0; i < sw.n_grad; i++) g_part[st.partial + i * sw.n_tiles + task] = g[i];

@@ -301,6 +301,27 @@ SVMI_HD inline uint64_t thread_entry(uint32_t w, uint32_t r, uint32_t goff, uint
     return uint64_t(w) | uint64_t(r) << 16 | uint64_t(goff) << 32 | uint64_t(grp) << 48;
 }
 
+// The thread entries of a phase: `zero` XOR the columns of the thread's set
+// lane and wave bits.  The kernels read them from a table by lane and one by
+// wave (which holds `zero`); programs keep the columns, an eighth of their size.
+struct ThreadCols {
+    uint64_t lane[kLaneBits], wave[kMaxWaveBits], zero;
+};
+SVMI_HD inline uint64_t lane_entry(const ThreadCols& c, uint32_t lane)
+{
+    uint64_t e = 0;
+#pragma unroll
+    for (int i = 0; i < kLaneBits; i++) e ^= ((lane >> i) & 1u) ? c.lane[i] : uint64_t(0);
+    return e;
+}
+SVMI_HD inline uint64_t wave_entry(const ThreadCols& c, uint32_t wave)
+{
+    uint64_t e = c.zero;
+#pragma unroll
+    for (int i = 0; i < kMaxWaveBits; i++) e ^= ((wave >> i) & 1u) ? c.wave[i] : uint64_t(0);
+    return e;
+}
+
 enum : uint32_t {
     LPH_CROSS = 1,     // the exchange moves amplitudes between waves
     LPH_GUARD = 2,     // other waves may still read this wave's part of LDS
@@ -334,7 +355,7 @@ struct SweepIO {
     uint64_t lane[2][kLaneBits];
     uint64_t wave[2][kWaveEntries];
     uint64_t reg[2][kRegs];      // two states: the first 8, for either state
-    uint32_t ph_begin, ph_end;   // into the layout phases; lane and wave tables run parallel to them
+    uint32_t ph_begin, ph_end;   // into the layout phases; their thread entries run parallel to them
     uint32_t store_guard;        // a wave stores where another one loads, and no exchange between the
                                  // waves lies in between: the workgroup meets before the stores
     uint32_t additive;

@@ -182,19 +182,16 @@ void emit_io(std::ostringstream& o, const SweepIO& io, int side, uint32_t thread
 
 // One phase: the exchange that leads into it (the real parts, then the
 // imaginary parts), its ops.
-void emit_phase(std::ostringstream& o, const Program& prog, const SweepInfo& sw, uint32_t p, bool first,
-                uint32_t threads)
+void emit_phase(std::ostringstream& o, const Program& prog, const SweepInfo& sw, uint32_t p, bool first)
 {
     const LayoutPhase& L = prog.lphases[p];
-    const uint64_t* lt = &prog.lane_tab[size_t(p) * kLaneEntries];
-    const uint64_t* wt = &prog.wave_tab[size_t(p) * kWaveEntries];
+    const ThreadCols& tc = prog.cols[p];
     o << "    {\n        const uint64_t te = ltab[" << uint64_t(p) * kLaneEntries << "u + lane] ^ wtab["
       << uint64_t(p) * kWaveEntries << "u + wave];\n";
     if (!first) {
-        uint64_t span = 0;
-        const uint32_t lanes = threads < uint32_t(kLaneEntries) ? threads : uint32_t(kLaneEntries);
-        for (uint32_t i = 0; i < lanes; i++) span |= lt[i];
-        for (uint32_t i = 0; i < threads / lanes; i++) span |= wt[i];
+        uint64_t span = tc.zero;
+        for (uint64_t c : tc.lane) span |= c;
+        for (uint64_t c : tc.wave) span |= c;
         o << "        const uint32_t w = uint32_t(te) & 0xffffu, rd = uint32_t(te) >> 16;\n";
         const char* meet = (L.flags & LPH_CROSS) ? "        __syncthreads();\n" : "        ORDER();\n";
         if (L.flags & LPH_GUARD) o << "        __syncthreads();\n";
@@ -260,7 +257,7 @@ void emit_sweep(std::ostringstream& o, const Program& prog, uint32_t i)
     o << "    c64 a[kRegs];\n";
     emit_io(o, io, 0, nt);
     if (sw.n_xf) o << "    __syncthreads();\n";
-    for (uint32_t p = io.ph_begin; p < io.ph_end; p++) emit_phase(o, prog, sw, p, p == io.ph_begin, nt);
+    for (uint32_t p = io.ph_begin; p < io.ph_end; p++) emit_phase(o, prog, sw, p, p == io.ph_begin);
     if (io.store_guard) o << "    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)\n    __syncthreads();\n";
     emit_io(o, io, 1, nt);
     o << "}\n\n";

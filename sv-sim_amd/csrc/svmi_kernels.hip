@@ -401,6 +401,31 @@ __device__ inline uint32_t batch_step_of(const BatchStep* __restrict__ steps, ui
     const BatchStep *__restrict__ steps, const BatchCircuit *__restrict__ circuits,                 \
         const SweepInfo *__restrict__ sweeps, const SweepIO *__restrict__ ios
 
+// One wave per phase (a batch has thousands of short ones: their tables by
+// copy were two thirds of what its calls upload).
+__global__ void __launch_bounds__(kThreads)
+k_thread_tables(const ThreadCols* __restrict__ cols, uint64_t n, uint64_t* __restrict__ lane_tab,
+                uint64_t* __restrict__ wave_tab)
+{
+    const uint64_t p = blockIdx.x * uint64_t(kThreads / 64) + (threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u;
+    if (p >= n) return;
+    lane_tab[p * kLaneEntries + lane] = lane_entry(cols[p], lane);
+    if (lane < uint32_t(kWaveEntries)) wave_tab[p * kWaveEntries + lane] = wave_entry(cols[p], lane);
+}
+
+hipError_t launch_thread_tables(hipStream_t st, const ThreadCols* cols, uint64_t n, uint64_t* lane_tab,
+                                uint64_t* wave_tab)
+{
+    constexpr uint64_t per = kThreads / 64, max_grid = 1ull << 30;
+    for (uint64_t p0 = 0; p0 < n; p0 += max_grid * per) {
+        const uint64_t cnt = n - p0 < max_grid * per ? n - p0 : max_grid * per;
+        hipLaunchKernelGGL(k_thread_tables, dim3(uint32_t((cnt + per - 1) / per)), dim3(kThreads), 0, st, cols + p0, cnt,
+                           lane_tab + p0 * kLaneEntries, wave_tab + p0 * kWaveEntries);
+    }
+    return hipGetLastError();
+}
+
 // kInit: the steps are first forward sweeps (tiles generated as |0..0>).
 template <bool kInit, int kMaxQ>
 __global__ void __launch_bounds__(kMaxTileThreads, kSweepWaves<kMaxQ>)

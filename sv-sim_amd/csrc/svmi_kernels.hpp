@@ -98,6 +98,9 @@ struct BatchLaunch {
     uint32_t max_dense;     // FWD: widest dense block of the group's sweeps
     uint64_t task_begin, n_tasks;
 };
+// The lane and wave tables of a batch's n phases from their columns.
+hipError_t launch_thread_tables(hipStream_t st, const ThreadCols* cols, uint64_t n, uint64_t* lane_tab,
+                                uint64_t* wave_tab);
 size_t batch_launch_smem(uint32_t kind, uint32_t k, uint32_t max_grad, uint32_t max_xf);
 hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L);
 

@@ -462,17 +462,13 @@ struct Builder {
                 after_cross = !in;
                 crossed = crossed || !in;
             }
-            uint64_t lane_col[kLaneBits] = {}, wave_col[kMaxWaveBits] = {};
+            ThreadCols tc;
+            std::memset(&tc, 0, sizeof(tc));
+            tc.zero = thread_entry(0, rc, 0, 0);
             for (int j = 0; j < t; j++)
-                (j < tl ? lane_col[j] : wave_col[j - tl]) =
+                (j < tl ? tc.lane[j] : tc.wave[j - tl]) =
                     thread_entry(wt[j], rt[j], p.grp[p.order[j]].goff, p.grp[p.order[j]].grp);
-            uint64_t tab[kLaneEntries];
-            tab[0] = 0;
-            for (int v = 1; v < kLaneEntries; v++) tab[v] = tab[v & (v - 1)] ^ lane_col[__builtin_ctz(v)];
-            prog.lane_tab.insert(prog.lane_tab.end(), tab, tab + kLaneEntries);
-            tab[0] = thread_entry(0, rc, 0, 0);
-            for (int v = 1; v < kWaveEntries; v++) tab[v] = tab[v & (v - 1)] ^ wave_col[__builtin_ctz(v)];
-            prog.wave_tab.insert(prog.wave_tab.end(), tab, tab + kWaveEntries);
+            prog.cols.push_back(tc);
             prog.lphases.push_back(L);
         }
         io.ph_end = uint32_t(prog.lphases.size());
@@ -494,12 +490,10 @@ void build_layouts(Program& prog)
 {
     prog.io.resize(prog.sweeps.size());
     prog.lphases.clear();
-    prog.lane_tab.clear();
-    prog.wave_tab.clear();
+    prog.cols.clear();
     const size_t most = prog.phases.size() + 2 * prog.sweeps.size();
     prog.lphases.reserve(most);
-    prog.lane_tab.reserve(most * kLaneEntries);
-    prog.wave_tab.reserve(most * kWaveEntries);
+    prog.cols.reserve(most);
     for (size_t i = 0; i < prog.sweeps.size(); i++) {
         Builder b(prog, prog.sweeps[i]);
         b.ph.reserve(b.sw.phase_end - b.sw.phase_begin + 2);

@@ -5,7 +5,7 @@
 
 namespace svmi {
 
-// Fills prog.io, lphases, lane_tab and wave_tab for every sweep of prog.
+// Fills prog.io, lphases and cols for every sweep of prog.
 void build_layouts(Program& prog);
 
 }  // namespace svmi

@@ -58,8 +58,7 @@ struct Program {
     // register layouts of the sweeps (build_layouts): io[i] for sweeps[i]
     std::vector<SweepIO> io;
     std::vector<LayoutPhase> lphases;
-    std::vector<uint64_t> lane_tab;    // kLaneEntries per layout phase
-    std::vector<uint64_t> wave_tab;    // kWaveEntries per layout phase
+    std::vector<ThreadCols> cols;      // per layout phase
     // adjoint: accumulator g of sweep s -> gradient parameter index
     std::vector<int32_t> grad_param;
     uint32_t n_grad = 0;
