@@ -399,7 +399,7 @@ svmi_status verify_batch(const BatchPlan& bp)
         if (L.step_begin != next || L.step_end <= L.step_begin || L.step_end > bp.steps.size() ||
             level_of[L.step_begin] != level_of[L.step_end - 1] ||
             L.task_begin != bp.steps[L.step_begin].task_begin ||
-            batch_launch_smem(L.kind, L.k, L.max_grad, L.max_xf) > size_t(160) * 1024)
+            batch_launch_smem(L) > size_t(160) * 1024)
             return fail(SVMI_ERR_STATE, "batch plan: bad launch");
         uint64_t nt = 0;
         for (uint32_t s = L.step_begin; s < L.step_end; s++) {
@@ -408,7 +408,7 @@ svmi_status verify_batch(const BatchPlan& bp)
             if (b.kind != L.kind || (sweep && bp.sweeps[b.sweep].k != L.k) || b.init_zero != L.init ||
                 (b.kind == BSTEP_ADJ && bp.sweeps[b.sweep].n_grad > L.max_grad) ||
                 (sweep && bp.sweeps[b.sweep].n_xf > L.max_xf) ||
-                (sweep && bp.sweeps[b.sweep].max_dense > L.max_dense))
+                (sweep && (bp.sweeps[b.sweep].max_dense > L.max_dense || bp.sweeps[b.sweep].stage > L.max_stage)))
                 return fail(SVMI_ERR_STATE, "batch plan: mixed launch");
             nt += b.n_tasks;
         }
@@ -690,6 +690,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
             const uint32_t ng = b.kind == BSTEP_ADJ ? bp.sweeps[b.sweep].n_grad : 0u;
             const uint32_t nx = (b.kind == BSTEP_FWD || b.kind == BSTEP_ADJ) ? bp.sweeps[b.sweep].n_xf : 0u;
             const uint32_t md = (b.kind == BSTEP_FWD || b.kind == BSTEP_ADJ) ? bp.sweeps[b.sweep].max_dense : 0u;
+            const uint32_t ms = (b.kind == BSTEP_FWD || b.kind == BSTEP_ADJ) ? bp.sweeps[b.sweep].stage : 0u;
             if (!bp.launches.empty() && bp.launches.back().step_end == idx &&
                 bp.launches.back().step_begin >= bp.level_begin.back() && bp.launches.back().kind == b.kind &&
                 bp.launches.back().k == k && bp.launches.back().init == b.init_zero) {
@@ -699,6 +700,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 L.max_grad = std::max(L.max_grad, ng);
                 L.max_xf = std::max(L.max_xf, nx);
                 L.max_dense = std::max(L.max_dense, md);
+                L.max_stage = std::max(L.max_stage, ms);
             } else {
                 BatchLaunch L;
                 std::memset(&L, 0, sizeof(L));
@@ -709,6 +711,7 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 L.max_grad = ng;
                 L.max_xf = nx;
                 L.max_dense = md;
+                L.max_stage = ms;
                 L.init = b.init_zero;
                 L.task_begin = b.task_begin;
                 L.n_tasks = b.n_tasks;
@@ -1677,6 +1680,7 @@ svmi_status svmi_batch_adjoint(int device, const svmi_batch_item* items, size_t 
         SVMI_TRY(k.dwave.ensure(std::max<size_t>(bp.cols.size() * kWaveEntries * 8, 16)));
         SVMI_HIP(launch_thread_tables(st, k.dcols.as<ThreadCols>(), bp.cols.size(), k.dlane.as<uint64_t>(),
                                       k.dwave.as<uint64_t>()));
+        bp.ops.push_back(DOp{});   // past the end: the latency builds read one header ahead
         SVMI_TRY(put(k.dops, bp.ops.data(), bp.ops.size() * sizeof(DOp)));
         SVMI_TRY(put(k.dcoef, bp.coef.data(), bp.coef.size() * sizeof(c64)));
         SVMI_TRY(put(k.dgroups, bp.groups.data(), bp.groups.size() * sizeof(PauliGroup)));

@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 
 #include "svmi_exec.hpp"
 #include "svmi_kernels.hpp"
@@ -427,30 +428,34 @@ hipError_t launch_thread_tables(hipStream_t st, const ThreadCols* cols, uint64_t
 }
 
 // kInit: the steps are first forward sweeps (tiles generated as |0..0>).
-template <bool kInit, int kMaxQ>
-__global__ void __launch_bounds__(kMaxTileThreads, kSweepWaves<kMaxQ>)
-k_batch_fwd(SVMI_BATCH_TABLES, SVMI_TABLES, uint32_t s0, uint32_t s1, uint64_t task0)
+// kLat, whole: see sweep_tile.
+template <bool kInit, int kMaxQ, bool kLat>
+__global__ void __launch_bounds__(kMaxTileThreads, kLat ? 2 : kSweepWaves<kMaxQ>)
+k_batch_fwd(SVMI_BATCH_TABLES, SVMI_TABLES, uint32_t s0, uint32_t s1, uint64_t task0, uint32_t whole)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint64_t t = task0 + blockIdx.x;
     const BatchStep st = steps[batch_step_of(steps, s0, s1, t)];
-    const SweepInfo sw = sweeps[st.sweep];
+    SweepInfo sw = sweeps[st.sweep];
+    sw.whole = whole;
     const SweepIO* __restrict__ io = ios + st.sweep;
-    sweep_tile<1, kMaxQ>(circuits[st.circuit].phi, nullptr, sw, io, SVMI_TABLE_ARGS, nullptr, t - st.task_begin, smem,
+    sweep_tile<1, kMaxQ, kLat>(circuits[st.circuit].phi, nullptr, sw, io, SVMI_TABLE_ARGS, nullptr, t - st.task_begin, smem,
                          kInit);
 }
 
-__global__ void __launch_bounds__(kMaxTileThreads, 4)
+template <bool kLat>
+__global__ void __launch_bounds__(kMaxTileThreads, kLat ? 2 : 4)
 k_batch_adj(SVMI_BATCH_TABLES, SVMI_TABLES, double* __restrict__ grad_partials, uint32_t s0, uint32_t s1,
-            uint64_t task0)
+            uint64_t task0, uint32_t whole)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint64_t t = task0 + blockIdx.x;
     const BatchStep st = steps[batch_step_of(steps, s0, s1, t)];
-    const SweepInfo sw = sweeps[st.sweep];
+    SweepInfo sw = sweeps[st.sweep];
+    sw.whole = whole;
     const SweepIO* __restrict__ io = ios + st.sweep;
     const BatchCircuit& c = circuits[st.circuit];
-    sweep_tile<2, kMaxDenseQubitsAdj>(c.phi, c.lam, sw, io, SVMI_TABLE_ARGS, grad_partials + st.partial,
+    sweep_tile<2, kMaxDenseQubitsAdj, kLat>(c.phi, c.lam, sw, io, SVMI_TABLE_ARGS, grad_partials + st.partial,
                                       t - st.task_begin, smem, false);
 }
 
@@ -635,48 +640,83 @@ k_batch_pauli(BatchArgs a, uint32_t s0, uint32_t s1, uint64_t task0)
     if (tid == 0) a.e_partials[st.partial + task] = red[0];
 }
 
-size_t batch_launch_smem(uint32_t kind, uint32_t k, uint32_t max_grad, uint32_t max_xf)
+// The largest of a launch's sweeps.
+static SweepInfo batch_sweep(const BatchLaunch& L)
 {
-    if (kind != BSTEP_FWD && kind != BSTEP_ADJ) return size_t(16) * kPauliChunk;
-    SweepInfo sw;   // the largest of the launch's sweeps
-    sw.k = k;
-    sw.n_xf = max_xf;
-    sw.n_grad = kind == BSTEP_ADJ ? max_grad : 0;
-    return sweep_smem_bytes(sw, kind == BSTEP_ADJ ? 2 : 1);
+    SweepInfo sw;
+    std::memset(&sw, 0, sizeof(sw));
+    sw.k = L.k;
+    sw.n_xf = L.max_xf;
+    sw.n_grad = L.kind == BSTEP_ADJ ? L.max_grad : 0;
+    sw.stage = L.max_stage;
+    sw.max_dense = L.max_dense;
+    sw.n_tiles = L.n_tasks;
+    return sw;
+}
+
+// Whether a launch of sw.n_tiles tiles runs the latency build, its threads
+// per tile and bytes of LDS.  (A batch's launch counts the tiles of all its
+// circuits: 4 circuits of 12 qubits 2.33 -> 2.04 ms, 64 of 12 4.07 -> 3.95.)
+struct SweepLaunch {
+    bool lat;
+    uint32_t whole, threads;
+    size_t smem;
+};
+static SweepLaunch sweep_launch(const SweepInfo& sw, int ns)
+{
+    const uint32_t nt = sweep_threads(sw.k, ns), threads = std::max(nt, 64u);
+    const size_t smem = sweep_smem_bytes(sw, ns), lat_smem = smem + 8 + 32 * sw.stage;
+    const size_t whole = lat_smem + (size_t(8) << sw.k) * ns;
+    SweepLaunch l;
+    l.lat = sw.max_dense <= 2 && sw.n_tiles * threads <= kLatThreads && sw.stage <= kLatStage * threads &&
+            !(ns == 1 && nt == 512 && sw.n_tiles <= 64) && lat_smem <= g_max_smem;
+    l.whole = l.lat && whole * ((sw.n_tiles + 255) / 256) <= kWholeBytes ? 1u : 0u;
+    l.threads = l.lat ? threads : nt;
+    l.smem = l.whole ? whole : l.lat ? lat_smem : smem;
+    return l;
+}
+
+size_t batch_launch_smem(const BatchLaunch& L)
+{
+    if (L.kind != BSTEP_FWD && L.kind != BSTEP_ADJ) return size_t(16) * kPauliChunk;
+    return sweep_smem_bytes(batch_sweep(L), L.kind == BSTEP_ADJ ? 2 : 1);
 }
 
 // The k_batch_fwd build of a forward launch.
-using BatchFwdFn = void (*)(SVMI_BATCH_TABLES, SVMI_TABLES, uint32_t, uint32_t, uint64_t);
-BatchFwdFn batch_fwd_kernel(const BatchLaunch& L)
+using BatchFwdFn = void (*)(SVMI_BATCH_TABLES, SVMI_TABLES, uint32_t, uint32_t, uint64_t, uint32_t);
+BatchFwdFn batch_fwd_kernel(const BatchLaunch& L, bool lat)
 {
-    if (L.init) return L.max_dense <= 2 ? &k_batch_fwd<true, 2> : &k_batch_fwd<true, kRegBits>;
-    return L.max_dense <= 2 ? &k_batch_fwd<false, 2> : &k_batch_fwd<false, kRegBits>;
+    if (lat) return L.init ? &k_batch_fwd<true, 2, true> : &k_batch_fwd<false, 2, true>;
+    if (L.init) return L.max_dense <= 2 ? &k_batch_fwd<true, 2, false> : &k_batch_fwd<true, kRegBits, false>;
+    return L.max_dense <= 2 ? &k_batch_fwd<false, 2, false> : &k_batch_fwd<false, kRegBits, false>;
 }
 
 hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L)
 {
-    const size_t smem = batch_launch_smem(L.kind, L.k, L.max_grad, L.max_xf);
-    if (smem > g_max_smem) return hipErrorInvalidConfiguration;
-    const uint32_t threads = L.kind == BSTEP_FWD ? sweep_threads(L.k, 1)
-                             : L.kind == BSTEP_ADJ ? sweep_threads(L.k, 2)
-                                                   : kPauliThreads;
+    SweepLaunch l{false, 0, uint32_t(kPauliThreads), batch_launch_smem(L)};
+    if (L.kind != BSTEP_PAULI) l = sweep_launch(batch_sweep(L), L.kind == BSTEP_ADJ ? 2 : 1);
+    if (l.smem > g_max_smem) return hipErrorInvalidConfiguration;
+    const dim3 threads(l.threads);
+    const size_t smem = l.smem;
     const uint64_t max_grid = 1ull << 30;
     for (uint64_t t0 = 0; t0 < L.n_tasks; t0 += max_grid) {
         const uint32_t cnt = uint32_t(L.n_tasks - t0 < max_grid ? L.n_tasks - t0 : max_grid);
         const uint64_t first = L.task_begin + t0;
         switch (L.kind) {
         case BSTEP_FWD: {
-            auto* fn = batch_fwd_kernel(L);
-            hipLaunchKernelGGL(fn, dim3(cnt), dim3(threads), smem, st, a.steps, a.circuits, a.sweeps, a.io,
-                               SVMI_TABLES_OF(a.t), L.step_begin, L.step_end, first);
+            auto* fn = batch_fwd_kernel(L, l.lat);
+            hipLaunchKernelGGL(fn, dim3(cnt), threads, smem, st, a.steps, a.circuits, a.sweeps, a.io,
+                               SVMI_TABLES_OF(a.t), L.step_begin, L.step_end, first, l.whole);
             break;
         }
-        case BSTEP_ADJ:
-            hipLaunchKernelGGL(k_batch_adj, dim3(cnt), dim3(threads), smem, st, a.steps, a.circuits, a.sweeps, a.io,
-                               SVMI_TABLES_OF(a.t), a.grad_partials, L.step_begin, L.step_end, first);
+        case BSTEP_ADJ: {
+            auto* fn = l.lat ? &k_batch_adj<true> : &k_batch_adj<false>;
+            hipLaunchKernelGGL(fn, dim3(cnt), threads, smem, st, a.steps, a.circuits, a.sweeps, a.io,
+                               SVMI_TABLES_OF(a.t), a.grad_partials, L.step_begin, L.step_end, first, l.whole);
             break;
+        }
         case BSTEP_PAULI:
-            hipLaunchKernelGGL(k_batch_pauli, dim3(cnt), dim3(threads), smem, st, a, L.step_begin, L.step_end, first);
+            hipLaunchKernelGGL(k_batch_pauli, dim3(cnt), threads, smem, st, a, L.step_begin, L.step_end, first);
             break;
         default:
             return hipErrorInvalidValue;
@@ -689,24 +729,21 @@ hipError_t launch_sweep(hipStream_t st, int ns, c64* s0, c64* s1, const SweepInf
                         const SweepTables& t, double* grad_partials)
 {
     SweepInfo sw = info;
-    const uint32_t nt = sweep_threads(sw.k, ns), threads = std::max(nt, 64u);
-    size_t smem = sweep_smem_bytes(sw, ns);
-    const size_t lat_smem = smem + 8 + 32 * sw.stage, whole = (size_t(8) << sw.k) * ns;
-    // (blocks of three and four register qubits from LDS would not fit its registers)
-    const bool lat = sw.max_dense <= 2 && sw.n_tiles * threads <= kLatThreads && sw.stage <= kLatStage * threads &&
-                     !(ns == 1 && nt == 512 && sw.n_tiles <= 64) && lat_smem <= g_max_smem;
-    sw.whole = lat && (lat_smem + whole) * ((sw.n_tiles + 255) / 256) <= kWholeBytes ? 1u : 0u;
-    if (lat) smem = lat_smem + (sw.whole ? whole : 0);
-    if (smem > g_max_smem || nt > uint32_t(kMaxTileThreads)) return hipErrorInvalidConfiguration;
+    const SweepLaunch l = sweep_launch(sw, ns);
+    sw.whole = l.whole;
+    if (l.smem > g_max_smem || l.threads > uint32_t(kMaxTileThreads)) return hipErrorInvalidConfiguration;
     const uint64_t max_grid = 1ull << 30;
     for (uint64_t t0 = 0; t0 < sw.n_tiles; t0 += max_grid) {
         const uint64_t cnt = sw.n_tiles - t0 < max_grid ? sw.n_tiles - t0 : max_grid;
+        const dim3 grid{uint32_t(cnt)}, threads(l.threads);
         if (ns == 1) {
-            auto* fn = lat ? &k_sweep1<2, true> : sw.max_dense <= 2 ? &k_sweep1<2, false> : &k_sweep1<kRegBits, false>;
-            hipLaunchKernelGGL(fn, dim3(uint32_t(cnt)), dim3(lat ? threads : nt), smem, st, s0, sw, io, SVMI_TABLES_OF(t), t0);
+            auto* fn = l.lat               ? &k_sweep1<2, true>
+                       : sw.max_dense <= 2 ? &k_sweep1<2, false>
+                                           : &k_sweep1<kRegBits, false>;
+            hipLaunchKernelGGL(fn, grid, threads, l.smem, st, s0, sw, io, SVMI_TABLES_OF(t), t0);
         } else {
-            hipLaunchKernelGGL(lat ? &k_sweep2<true> : &k_sweep2<false>, dim3(uint32_t(cnt)), dim3(lat ? threads : nt), smem, st, s0,
-                               s1, sw, io, SVMI_TABLES_OF(t), grad_partials, t0);
+            hipLaunchKernelGGL(l.lat ? &k_sweep2<true> : &k_sweep2<false>, grid, threads, l.smem, st, s0, s1, sw, io,
+                               SVMI_TABLES_OF(t), grad_partials, t0);
         }
     }
     return hipGetLastError();
@@ -734,11 +771,15 @@ hipError_t init_sweep_kernels()
           raise(reinterpret_cast<const void*>(&k_sweep1<kRegBits, false>)) &&
           raise(reinterpret_cast<const void*>(&k_sweep1<2, true>)) &&
           raise(reinterpret_cast<const void*>(&k_sweep2<false>)) &&
-          raise(reinterpret_cast<const void*>(&k_sweep2<true>)) && raise(reinterpret_cast<const void*>(&k_batch_adj)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, 2>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, 2>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, kRegBits>)) &&
-          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, kRegBits>)))) {
+          raise(reinterpret_cast<const void*>(&k_sweep2<true>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_adj<false>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_adj<true>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, 2, false>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, 2, false>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, 2, true>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, 2, true>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<true, kRegBits, false>)) &&
+          raise(reinterpret_cast<const void*>(&k_batch_fwd<false, kRegBits, false>)))) {
         (void)hipGetLastError();
         want = 64 * 1024;
     }

@@ -95,13 +95,14 @@ struct BatchLaunch {
     uint32_t max_grad;      // ADJ: largest n_grad of the group's sweeps
     uint32_t init;          // FWD: first sweeps (tiles start as |0..0>)
     uint32_t max_xf;        // largest n_xf of the group's sweeps
-    uint32_t max_dense;     // FWD: widest dense block of the group's sweeps
+    uint32_t max_dense;     // widest dense block of the group's sweeps
+    uint32_t max_stage;     // largest SweepInfo::stage of the group's sweeps
     uint64_t task_begin, n_tasks;
 };
 // The lane and wave tables of a batch's n phases from their columns.
 hipError_t launch_thread_tables(hipStream_t st, const ThreadCols* cols, uint64_t n, uint64_t* lane_tab,
                                 uint64_t* wave_tab);
-size_t batch_launch_smem(uint32_t kind, uint32_t k, uint32_t max_grad, uint32_t max_xf);
+size_t batch_launch_smem(const BatchLaunch& L);   // without what the latency builds add
 hipError_t launch_batch(hipStream_t st, const BatchArgs& a, const BatchLaunch& L);
 
 hipError_t init_sweep_kernels();

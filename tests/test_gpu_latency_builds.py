@@ -49,3 +49,24 @@ def test_small_gradients_match_shifted_energies(n, tile):
             g[("theta", "phi", "lambda")[f]][i] += s
             v.append(O.expval(n, *O.run(n, g), terms))
         assert abs(grad[k] - (v[0] - v[1]) / 2) < TOL * len(terms)
+
+
+@pytest.mark.parametrize("count,n,kw", [(1, 4, {}), (3, 5, {}), (3, 7, {"fwd_tile": 6, "adj_tile": 6}), (2, 9, {}),
+                                        (4, 12, {}), (300, 4, {}), (6, 12, {"fwd_tile": 6, "adj_tile": 7}),
+                                        (2, 15, {}), (3, 17, {"fwd_tile": 12, "adj_tile": 11})])
+def test_small_batches_match_single_circuits(count, n, kw):
+    rng = np.random.default_rng(count + 100 * n)
+    items = []
+    for i in range(count):
+        gates, slots, p = W.hea(n, 1 + i % 3, rng)
+        terms = [(float(c), x, z) for c, x, z in W.ising_terms(n, rng)]
+        items.append(dict({"n": n, "gates": gates, "param_slots": slots, "n_params": p, "terms": terms}, **kw))
+    ev, grads = svmi.batch_adjoint(items)
+    for i, it in enumerate(items):
+        tol = TOL * len(it["terms"])
+        assert abs(ev[i] - O.expval(n, *O.run(n, it["gates"]), it["terms"])) < tol
+        if i < 4:
+            with svmi.Engine(n) as e:
+                e.upload(it["gates"])
+                _, g = e.adjoint(it["terms"], it["param_slots"], it["n_params"])
+            assert np.abs(g - grads[i]).max() < tol
