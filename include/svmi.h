@@ -98,7 +98,8 @@ typedef struct svmi_stats {
 typedef enum svmi_option {
     SVMI_OPT_FUSION = 0,      /* 1 = tiled multi-gate sweeps (default), 0 = one pass per op */
     SVMI_OPT_TILE_QUBITS = 1, /* qubits per tile (4..13, two states up to 12; default by state size:
-                                 12, from 20 qubits on 13; two states 11, from 19 on 12;
+                                 12, from 21 qubits on 13; two states 11, from 19 on 12, which
+                                 is also the most that a given tile has there;
                                  with SVMI_OPT_SPECIALIZE 13 only up to
                                  31 and where it saves a pass)                                */
     SVMI_OPT_LOW_QUBITS = 2,  /* low qubits every tile keeps for coalescing (0..8, default 4; 3

@@ -1191,9 +1191,10 @@ svmi_status svmi_get_amplitudes(svmi_handle h, const uint64_t* idx, size_t count
     return SVMI_OK;
 }
 
-// Default tile and low qubits.  Tiles of 13 qubits from 20 qubits on (two
-// states: 12 from 19), where a state has at least 128 of them; on smaller
-// states the tiles of 12 (11) keep more CUs busy.  3 low qubits (128-byte
+// Default tile and low qubits.  Tiles of 13 qubits from 21 qubits on (two
+// states: 12 from 19), where a state has at least 256 (128) of them; on smaller
+// states the tiles of 12 (11) keep more CUs busy, and a given tile of two
+// states is held to the same sizes.  3 low qubits (128-byte
 // segments) leave one more than 4 for the circuit: at the copy rate of
 // 256-byte segments still, and fewer sweeps.  12 and 4 / 13 and 4 / 13 and 3:
 // u3 brick wall at 30 qubits 180 / 167 / 164 ms, QFT at 31 87.6 / 93.6 / 81.8
@@ -1202,10 +1203,13 @@ svmi_status svmi_get_amplitudes(svmi_handle h, const uint64_t* idx, size_t count
 // 152, 211 / 200 us, 10 random layers 119 / 118, 151 / 148, 213 / 194 us;
 // the ansatz's adjoint with 11 and 4 / 11 and 3 / 12 and 3: at 15 482 / 461 /
 // 480, at 18 707 / 634 / 660, at 19 869 / 822 / 783 us.  (2 low qubits: random
-// layers of 17 qubits 159 us.)
+// layers of 17 qubits 159 us.)  12 and 3 / 13 and 3: 30 random layers at 20
+// qubits 831 / 921, QFT 89 / 98, 25 u3 layers 406 / 423, ansatz 294 / 296 us;
+// ansatz at 21 377 / 329, QFT 109 / 96 us.
 void default_tile(svmi_handle h, int n, bool two, PlanOptions& o)
 {
-    if (!h->tile_set) o.tile_qubits = n >= 20 ? (two ? 12 : 13) : n == 19 || !two ? 12 : 11;
+    const int largest = two ? (n >= 19 ? 12 : 11) : n >= 21 ? 13 : 12;
+    if (!h->tile_set || (two && o.tile_qubits > largest)) o.tile_qubits = largest;
     if (!h->low_set && !h->tile_set) o.low_qubits = 3;
 }
 
