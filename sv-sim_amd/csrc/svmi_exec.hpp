@@ -342,7 +342,7 @@ SVMI_HD inline c64 tile_factor(const DOpHdr& h, const c64* __restrict__ coef, ui
 template <int N>
 SVMI_HD inline void apply_rot(const DOpHdr& h, c64 (&a)[N], const c64* __restrict__ coef, uint32_t v)
 {
-    if (h.s0) apply_rtab<N>(a, coef_at(coef, h.grad + 16u * v));
+    if (h.s0) apply_rtab<N>(a, coef_at(coef, h.coef + 4u + 16u * v));
     const c64* L = coef_at(coef, h.coef);
     const c64 f0 = L[0], f1 = L[1], f2 = L[2], f3 = L[3];
 #define SVMI_ROT_SLOT(S, F)                                              \

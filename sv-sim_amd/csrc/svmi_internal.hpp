@@ -143,7 +143,7 @@ enum DOpType : uint16_t {
                          // gmask = the factor-area slot where the tile keeps the T_j, or
                          // kLaneTabGlobal to read them from coef
     DOP_ROT = 16,        // a run of rotations in one dispatch: if s0, first the register
-                         // table coef + grad + 16*v (v as DOP_RTAB, from emask); then the
+                         // table coef + 4 + 16*v (v as DOP_RTAB, from emask); then the
                          // lifting steps on every slot of smask in ascending order, three
                          // shears where s1 has the slot's bit, {u, l} = coef[h.coef + slot]
 };

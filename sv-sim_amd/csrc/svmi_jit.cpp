@@ -50,7 +50,6 @@ std::string variant(uint64_t emask, const SweepInfo& sw)
 void emit_state_op(std::ostringstream& o, DOp d, const LayoutPhase& ph, const SweepInfo& sw)
 {
     d.h.coef += sw.coef_base;
-    if (d.h.type == DOP_ROT && d.h.s0) d.h.grad += sw.coef_base;   // its table
     const DOpHdr& h = d.h;
     const std::string cond = "(base & " + std::to_string(h.emask) + "ull) == " + std::to_string(h.emask) +
                              "ull && (goff & " + std::to_string(h.gmask) + "u) == " + std::to_string(h.gmask) + "u";
@@ -70,7 +69,7 @@ void emit_state_op(std::ostringstream& o, DOp d, const LayoutPhase& ph, const Sw
         return;
     case DOP_ROT:
         if (h.s0)
-            o << "        apply_rtab(a, coef + " << h.grad << "u + 16u * " << variant(h.emask, sw) << ");\n";
+            o << "        apply_rtab(a, coef + " << (h.coef + 4u) << "u + 16u * " << variant(h.emask, sw) << ");\n";
         for (int sl = 0; sl < kRegBits; sl++)
             if ((h.smask >> sl) & 1u)
                 o << "        apply_lift<" << sl << ", " << (((h.s1 >> sl) & 1u) ? "true" : "false") << ">(a, coef["

@@ -265,7 +265,6 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
             if constexpr (kLat) {   // (op arrays end with an unused record)
                 h = nxt;
                 nxt = op[1].h;
-                if (h.type == DOP_ROT && h.s0) h.grad -= L.coef_begin;   // its table
                 h.coef -= L.coef_begin;
             } else {
                 h = op->h;

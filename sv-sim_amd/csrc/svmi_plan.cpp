@@ -1474,7 +1474,6 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
                     if (!em[i].s) {
                         DOp d = em[i].d;
                         d.h.coef = enc.push_coef(em[i].coef);
-                        if (d.h.type == DOP_ROT && d.h.s0) d.h.grad = d.h.coef + 4;
                         prog.ops.push_back(d);
                         i++;
                         continue;
@@ -1585,9 +1584,7 @@ void emit_sweep(Program& prog, const std::vector<const SOp*>& taken, uint64_t T,
     for (uint32_t o = sw.op_begin; o < sw.op_end; o++) {   // offsets from the sweep's first coefficient
         DOpHdr& h = prog.ops[o].h;
         constexpr uint32_t none = 1u << DOP_NOP | 1u << DOP_X | 1u << DOP_CX | 1u << DOP_SWAP | 1u << DOP_SRN;
-        if ((none >> h.type) & 1u) continue;
-        h.coef -= sw.coef_base;
-        if (h.type == DOP_ROT && h.s0) h.grad -= sw.coef_base;   // its table
+        if (!((none >> h.type) & 1u)) h.coef -= sw.coef_base;
     }
     prog.n_grad += n_grad_sweep;
     // The coefficients a tile reads while it runs the sweep go through the
