@@ -48,6 +48,12 @@ svmi_status svmi_debug_plan_batch(const svmi_batch_item* items, size_t n_items, 
 svmi_status svmi_debug_batch_coefs(const svmi_batch_item* items, size_t n_items, uint64_t* n_coefs,
                                    uint64_t* max_offset);
 
+/* How <H> runs on a state of n qubits (lam != 0: with H psi written, as
+ * svmi_adjoint): passes over the state, qubits of their tiles, X masks
+ * read from a tile and masks read from memory. */
+svmi_status svmi_debug_plan_pauli(int n, const svmi_pauli_term* terms, size_t n_terms, int lam, uint64_t* n_passes,
+                                  uint64_t* tile_qubits, uint64_t* in_tile, uint64_t* from_memory);
+
 /* Planner summary (as svmi_debug_plan) of the backward program svmi_adjoint builds. */
 svmi_status svmi_debug_plan_adjoint(int n, const svmi_gate* gates, size_t n_gates, const int32_t* param_slots,
                                     size_t n_params, int tile_qubits, int low_qubits, uint64_t* n_passes,

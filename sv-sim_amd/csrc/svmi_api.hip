@@ -890,7 +890,7 @@ svmi_status exec_program(svmi_handle h, const Program& prog, DeviceProgram& dp, 
 // copies: the caller synchronises).
 svmi_status pauli_upload(svmi_handle h, const svmi_pauli_term* terms, size_t n_terms, bool lam, PauliPlan& plan)
 {
-    plan_pauli(terms, n_terms, h->n_int, pauli_tile_qubits(h->n_int), lam, kMaxPauliPasses, plan);
+    plan_pauli_state(terms, n_terms, h->n_int, lam, plan);
     SVMI_TRY(h->scratch[0].ensure(std::max<size_t>(plan.groups.size(), 1) * sizeof(PauliGroup)));
     SVMI_TRY(h->scratch[1].ensure(std::max<size_t>(plan.terms.size(), 1) * sizeof(PauliTerm)));
     if (!plan.groups.empty()) {
@@ -1493,7 +1493,7 @@ svmi_status svmi_expval_static(svmi_handle h, const svmi_pauli_term* terms, size
         return fail(SVMI_ERR_ARG, "svmi_expval_static takes at most " + std::to_string(kStaticMaxTerms) +
                                       " Pauli terms (got " + std::to_string(n_terms) + "); use svmi_expval");
     PauliPlan plan;
-    plan_pauli(terms, n_terms, h->n_int, pauli_tile_qubits(h->n_int), false, kMaxPauliPasses, plan);
+    plan_pauli_state(terms, n_terms, h->n_int, false, plan);
     // scratch layout: groups | terms | block partials, each 256-B aligned
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t np = pauli_partials(h, plan);
@@ -2210,6 +2210,22 @@ svmi_status svmi_debug_plan_batch(const svmi_batch_item* items, size_t n_items, 
     if (n_launches) *n_launches = bp.launches.size();
     if (n_tasks) *n_tasks = bp.n_tasks;
     if (state_bytes) *state_bytes = bp.state_bytes;
+    return SVMI_OK;
+}
+
+svmi_status svmi_debug_plan_pauli(int n, const svmi_pauli_term* terms, size_t n_terms, int lam, uint64_t* n_passes,
+                                  uint64_t* tile_qubits, uint64_t* in_tile, uint64_t* from_memory)
+{
+    if (n < 1 || n > kMaxQubits) return fail(SVMI_ERR_ARG, "n must be in [1, " + std::to_string(kMaxQubits) + "]");
+    SVMI_TRY(check_terms(terms, n_terms, n));
+    PauliPlan plan;
+    plan_pauli_state(terms, n_terms, std::max(n, kRegBits), lam != 0, plan);
+    uint64_t tile = 0, mem = 0;
+    for (const PauliPass& p : plan.passes) tile += p.tile_end - p.begin, mem += p.end - p.tile_end;
+    if (n_passes) *n_passes = plan.passes.size();
+    if (tile_qubits) *tile_qubits = plan.passes[0].k;
+    if (in_tile) *in_tile = tile;
+    if (from_memory) *from_memory = mem;
     return SVMI_OK;
 }
 

@@ -58,15 +58,10 @@ void group_terms(const svmi_pauli_term* terms, size_t n_terms, std::vector<Pauli
     }
 }
 
-}  // namespace
+// Every seed looks at all masks after it: the search stays linear in them.
+constexpr int kMaxFailedSeeds = 256;
 
-int pauli_tile_qubits(int n)
-{
-    // 12-qubit tiles need 20 qubits for a workgroup on every CU; below, smaller
-    // tiles (2 or 1 amplitudes per thread) keep the chip busy and the masks
-    // above them are read from L2
-    return n >= 20 ? 12 : n >= 18 ? 10 : std::min(n, 8);
-}
+}  // namespace
 
 void plan_pauli(const svmi_pauli_term* terms, size_t n_terms, int n, int tile_qubits, bool lam, int max_passes,
                 PauliPlan& plan)
@@ -80,18 +75,15 @@ void plan_pauli(const svmi_pauli_term* terms, size_t n_terms, int n, int tile_qu
     const int k = std::min(tile_qubits, n);
     const uint64_t low = (uint64_t(1) << k) - 1, keep = (uint64_t(1) << std::min(kPauliLow, k)) - 1;
     // a further pass reads psi once (and reads and writes lam), a mask left to
-    // the first pass reads psi once more; states of up to 21 qubits (32 MiB)
-    // stay in the last-level cache, where those reads cost less than a pass
+    // the first pass reads psi once more
     const size_t worth = lam ? 4 : 2;
-    const bool more = n >= 22 || k < kPauliTileQubits;
     std::vector<uint64_t> tiles{low};
     std::vector<int> pass_of(g.size(), -1);   // -1: read from memory in the first pass
     for (size_t i = 0; i < g.size(); i++)
         if (!(g[i].xmask & ~low)) pass_of[i] = 0;
-    std::vector<char> tried(g.size(), 0);
-    for (size_t s = 0; more && s < g.size() && tiles.size() < size_t(max_passes); s++) {
-        if (pass_of[s] >= 0 || tried[s]) continue;
-        tried[s] = 1;
+    int failed = 0;   // seeds that found too few masks to share a tile with
+    for (size_t s = 0; s < g.size() && tiles.size() < size_t(max_passes) && failed < kMaxFailedSeeds; s++) {
+        if (pass_of[s] >= 0 || __builtin_popcountll(keep | g[s].xmask) > k) continue;
         uint64_t tile = keep;
         size_t covered = 0;
         for (size_t i = s; i < g.size(); i++)
@@ -99,7 +91,10 @@ void plan_pauli(const svmi_pauli_term* terms, size_t n_terms, int n, int tile_qu
                 tile |= g[i].xmask;
                 covered++;
             }
-        if (covered < worth) continue;
+        if (covered < worth) {
+            failed++;
+            continue;
+        }
         for (int q = 0; q < n && __builtin_popcountll(tile) < k; q++) tile |= uint64_t(1) << q;
         for (size_t i = 0; i < g.size(); i++)
             if (pass_of[i] < 0 && !(g[i].xmask & ~tile)) pass_of[i] = int(tiles.size());
@@ -141,6 +136,27 @@ void plan_pauli(const svmi_pauli_term* terms, size_t n_terms, int n, int tile_qu
         p.end = uint32_t(plan.groups.size());
         plan.passes.push_back(p);
     }
+}
+
+void plan_pauli_state(const svmi_pauli_term* terms, size_t n_terms, int n, bool lam, PauliPlan& plan)
+{
+    // 12-qubit tiles need 20 qubits for a workgroup on every CU; below, smaller
+    // tiles (2 or 1 amplitudes per thread) keep the chip busy.  States of up to
+    // 21 qubits (32 MiB) stay in the last-level cache, where reading psi once
+    // more for a mask costs less than a pass: one pass / several, 50 random
+    // masks at 14 qubits 61 / 100 us, Heisenberg chain of 18 qubits 47 / 54.
+    const int k = n >= 20 ? kPauliTileQubits : n >= 18 ? 10 : std::min(n, 8);
+    const int passes = n >= 22 ? kMaxPauliPasses : 1;
+    plan_pauli(terms, n_terms, n, k, lam, passes, plan);
+    if (k < kPauliTileQubits) return;
+    // Where few masks lie in a tile, the reads from memory want more workgroups
+    // on a CU than the LDS of 12-qubit tiles lets in.  12 / 10 qubits: 50 random
+    // masks at 24 qubits (none in a tile) 2.07 / 1.82 ms, all masks of 23 of 24
+    // qubits 829 / 601 us; 1191 masks of 4 random qubits at 20 (a fifth in a
+    // tile) 1.88 / 2.05 ms.
+    size_t in_tile = 0, read = 0;
+    for (const PauliPass& p : plan.passes) in_tile += p.tile_end - p.begin, read += p.end - p.tile_end;
+    if (read > 8 * in_tile) plan_pauli(terms, n_terms, n, 10, lam, passes, plan);
 }
 
 }  // namespace svmi

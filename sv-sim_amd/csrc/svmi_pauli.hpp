@@ -14,13 +14,13 @@ struct PauliPlan {
     std::vector<PauliPass> passes;    // the first covers every amplitude of lam; at least one
 };
 
-// Plan for a state of n qubits with tiles of up to tile_qubits (<= kPauliTileQubits);
-// lam: H psi is written, not only summed.  max_passes 1: one pass whose tiles
-// are the lowest qubits.
+// Plan for a state of n qubits with tiles of up to tile_qubits (<= kPauliTileQubits)
+// and up to max_passes passes, the first one's tiles the lowest qubits; lam:
+// H psi is written, not only summed.
 void plan_pauli(const svmi_pauli_term* terms, size_t n_terms, int n, int tile_qubits, bool lam, int max_passes,
                 PauliPlan& plan);
 
-// Tile size for a state of n qubits.
-int pauli_tile_qubits(int n);
+// The same with the tiles and passes that run a state of n qubits fastest.
+void plan_pauli_state(const svmi_pauli_term* terms, size_t n_terms, int n, bool lam, PauliPlan& plan);
 
 }  // namespace svmi

@@ -53,7 +53,7 @@ EXPORTS = ["svmi_create", "svmi_destroy", "svmi_num_qubits", "svmi_reset_state",
            "svmi_debug_emulate", "svmi_debug_emulate_adjoint", "svmi_debug_emulate_batch", "svmi_debug_plan",
            "svmi_debug_plan_batch", "svmi_debug_plan_adjoint", "svmi_debug_emulate_qir", "svmi_debug_plan_qir",
            "svmi_debug_jit", "svmi_dm_qir_run", "svmi_debug_emulate_dm_qir", "svmi_debug_step_times", "svmi_debug_fp64_rates", "svmi_expval_static",
-           "svmi_debug_batch_coefs"]
+           "svmi_debug_batch_coefs", "svmi_debug_plan_pauli"]
 
 
 class SvmiError(RuntimeError):
@@ -127,6 +127,7 @@ def lib():
         L.svmi_debug_emulate_adjoint.argtypes = [ctypes.c_int, _vp, _sz, _vp, _sz, _vp, _sz, ctypes.c_int,
                                                  ctypes.c_int, _vp, _vp, _vp, _vp]
         L.svmi_debug_emulate_batch.argtypes = [_vp, _sz, _vp, _vp]
+        L.svmi_debug_plan_pauli.argtypes = [ctypes.c_int, _vp, _sz, ctypes.c_int] + [ctypes.POINTER(ctypes.c_uint64)] * 4
         L.svmi_debug_batch_coefs.argtypes = [_vp, _sz, ctypes.POINTER(ctypes.c_uint64),
                                              ctypes.POINTER(ctypes.c_uint64)]
         L.svmi_debug_plan.argtypes = [ctypes.c_int, _vp, _sz, ctypes.c_int, ctypes.c_int, ctypes.c_int,
@@ -417,6 +418,14 @@ def batch_coefs(items):
     v = [ctypes.c_uint64() for _ in range(2)]
     _check(lib().svmi_debug_batch_coefs(ctypes.cast(arr, _vp), len(items), *[ctypes.byref(x) for x in v]))
     return tuple(x.value for x in v)
+
+
+def plan_pauli(n, terms, lam=False):
+    """{passes, tile_qubits, in_tile, from_memory} of <H> on a state of n qubits."""
+    t = as_terms(terms)
+    v = [ctypes.c_uint64() for _ in range(4)]
+    _check(lib().svmi_debug_plan_pauli(int(n), _ptr(t), len(t), int(lam), *[ctypes.byref(x) for x in v]))
+    return dict(zip(("passes", "tile_qubits", "in_tile", "from_memory"), (x.value for x in v)))
 
 
 def emulate(n, gates, state, fusion=True, tile_qubits=12, low_qubits=4, sweep_budget=0):
