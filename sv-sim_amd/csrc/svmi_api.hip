@@ -942,16 +942,22 @@ svmi_status pauli_device(svmi_handle h, const c64* psi, const svmi_pauli_term* t
 }
 
 // Host copies of the state (AoS device <-> SoA host) in chunks through pinned
-// slots.  Worker w moves chunks w, w + workers, ... through slot w: its share
-// of the (un)interleaving, and of the page faults of a new host array, runs
-// while the other workers' chunks are on the bus.  A state of 2^21 amplitudes:
-// set 1.9 -> 0.9 ms, get 3.5 -> 1.0 ms (one slot allocated per call, one thread).
+// slots.  From 8 chunks on four workers take a quarter each (neighbours in the
+// host arrays, whose large pages they then fault in alone): a worker's share of
+// the (un)interleaving and of the page faults of a new host array runs while
+// the others' chunks are on the bus.  Below, starting threads costs more than
+// it saves, and one worker fills a slot while the slots before it are copied.
+// A state of 2^21 amplitudes: set 1.9 -> 0.9 ms, get 3.5 -> 1.0 ms (one slot
+// allocated per call, one thread).
 constexpr size_t kChunk = size_t(1) << 17;   // amplitudes of a slot (2 MiB)
 constexpr int kIoSlots = 4;
+constexpr uint64_t kIoThreadedChunks = 8;
 
-// The slots of a call come from a pool of the process (a new handle would pay
-// some milliseconds to pin its own) of at most kIoKept idle sets, freed with
-// the last handle.
+// The slots of a call come from a pool of the process: pinning a set and
+// faulting in its 8 MiB costs up to 4 ms (set_state of 19 qubits on a new
+// handle 3.7 ms, from the pool 0.27).  At most kIoKept idle sets are kept while
+// there are handles, one of them for the programs that make one handle after
+// another.
 struct IoPool {
     std::mutex mu;
     std::vector<c64*> idle;
@@ -968,13 +974,13 @@ struct IoPool {
                 return hipSuccess;
             }
         }
-        return hipHostMalloc(reinterpret_cast<void**>(out), kIoSlots * kChunk * sizeof(c64), hipHostMallocPortable);
+        return hipHostMalloc(reinterpret_cast<void**>(out), kIoSlots * kChunk * sizeof(c64), hipHostMallocDefault);
     }
     void give(c64* p)
     {
         {
             std::lock_guard<std::mutex> lk(mu);
-            if (handles > 0 && idle.size() < kIoKept) {
+            if (idle.size() < (handles > 0 ? kIoKept : 1)) {
                 idle.push_back(p);
                 return;
             }
@@ -988,19 +994,23 @@ struct IoPool {
     }
     void leave()
     {
-        std::vector<c64*> last;
+        c64* extra = nullptr;
         {
             std::lock_guard<std::mutex> lk(mu);
-            if (--handles == 0) last.swap(idle);
+            if (--handles == 0 && idle.size() > 1) {
+                extra = idle.back();
+                idle.pop_back();
+            }
         }
-        for (c64* p : last) (void)hipHostFree(p);
+        if (extra) (void)hipHostFree(extra);
     }
 };
 IoPool g_io;
 
-// move(first, count, slot, w): one chunk through slot w, done on return
+// to_device: pack(first, count, slot) fills a slot, which goes to dev + first;
+// else dev + first comes to a slot, which pack takes.
 template <class F>
-svmi_status io_chunks(svmi_handle h, uint64_t dim, const char* what, F move)
+svmi_status io_chunks(svmi_handle h, uint64_t dim, c64* dev, bool to_device, const char* what, F pack)
 {
     for (hipEvent_t& e : h->io_ev)
         if (!e) SVMI_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -1008,13 +1018,43 @@ svmi_status io_chunks(svmi_handle h, uint64_t dim, const char* what, F move)
     c64* slots = nullptr;
     SVMI_HIP(g_io.take(&slots));
     const uint64_t chunks = (dim + kChunk - 1) / kChunk;
-    const int workers = int(std::min<uint64_t>(kIoSlots, chunks));
+    const int workers = chunks >= kIoThreadedChunks ? kIoSlots : 1, ring = kIoSlots / workers;
     std::atomic<int> err{int(hipSuccess)};
     const auto work = [&](int w) {
         hipError_t e = hipSetDevice(h->device);
-        for (uint64_t c = uint64_t(w); c < chunks && e == hipSuccess && err == int(hipSuccess); c += uint64_t(workers)) {
-            const uint64_t x0 = c * kChunk;
-            e = move(x0, size_t(std::min<uint64_t>(kChunk, dim - x0)), slots + size_t(w) * kChunk, w);
+        const uint64_t c0 = chunks * uint64_t(w) / uint64_t(workers), c1 = chunks * uint64_t(w + 1) / uint64_t(workers);
+        const auto count = [&](uint64_t c) { return size_t(std::min<uint64_t>(kChunk, dim - c * kChunk)); };
+        const auto index = [&](uint64_t c) { return w * ring + int((c - c0) % uint64_t(ring)); };
+        const auto copy = [&](uint64_t c) {
+            c64 *slot = slots + size_t(index(c)) * kChunk, *at = dev + c * kChunk;
+            e = hipMemcpyAsync(to_device ? at : slot, to_device ? slot : at, count(c) * sizeof(c64),
+                               to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, h->stream);
+            if (e == hipSuccess) e = hipEventRecord(h->io_ev[index(c)], h->stream);
+        };
+        const auto wait = [&](uint64_t c) {
+            if (e == hipSuccess) e = hipEventSynchronize(h->io_ev[index(c)]);
+        };
+        const auto go = [&]() { return e == hipSuccess && err == int(hipSuccess); };
+        uint64_t issued = c0;   // chunks whose copies were given to the stream
+        if (to_device) {
+            for (uint64_t c = c0; c < c1 && go(); c++) {
+                if (c >= c0 + uint64_t(ring)) wait(c - uint64_t(ring));
+                if (e != hipSuccess) break;
+                pack(c * kChunk, count(c), slots + size_t(index(c)) * kChunk);
+                copy(c);
+                issued = c + 1;
+            }
+        } else {
+            for (uint64_t c = c0; c < c1 && go(); c++) {
+                while (issued < c1 && issued < c + uint64_t(ring) && e == hipSuccess) copy(issued++);
+                wait(c);
+                if (e == hipSuccess) pack(c * kChunk, count(c), slots + size_t(index(c)) * kChunk);
+            }
+        }
+        // the slots are given back with no copy under way
+        for (uint64_t c = issued > c0 + uint64_t(ring) ? issued - uint64_t(ring) : c0; c < issued; c++) {
+            const hipError_t s = hipEventSynchronize(h->io_ev[index(c)]);
+            if (e == hipSuccess) e = s;
         }
         if (e != hipSuccess) err = int(e);
     };
@@ -1143,11 +1183,8 @@ svmi_status svmi_set_state(svmi_handle h, const double* re, const double* im)
     if (h->n_int != h->n) {
         SVMI_HIP(launch_fill_basis(h->stream, h->sv, h->dim));
     }
-    return io_chunks(h, dim_user, "set_state", [&](uint64_t x0, size_t cnt, c64* slot, int w) -> hipError_t {
+    return io_chunks(h, dim_user, h->sv, true, "set_state", [&](uint64_t x0, size_t cnt, c64* slot) {
         for (size_t i = 0; i < cnt; i++) slot[i] = c64{re[x0 + i], im[x0 + i]};
-        hipError_t e = hipMemcpyAsync(h->sv + x0, slot, cnt * sizeof(c64), hipMemcpyHostToDevice, h->stream);
-        if (e == hipSuccess) e = hipEventRecord(h->io_ev[w], h->stream);
-        return e == hipSuccess ? hipEventSynchronize(h->io_ev[w]) : e;
     });
 }
 
@@ -1156,16 +1193,11 @@ svmi_status svmi_get_state(svmi_handle h, double* re, double* im)
     SVMI_TRY(use_device(h));
     if (!re || !im) return fail(SVMI_ERR_ARG, "null state array");
     const uint64_t dim_user = 1ull << h->n;
-    return io_chunks(h, dim_user, "get_state", [&](uint64_t x0, size_t cnt, c64* slot, int w) -> hipError_t {
-        hipError_t e = hipMemcpyAsync(slot, h->sv + x0, cnt * sizeof(c64), hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipEventRecord(h->io_ev[w], h->stream);
-        if (e == hipSuccess) e = hipEventSynchronize(h->io_ev[w]);
-        if (e == hipSuccess)
-            for (size_t i = 0; i < cnt; i++) {
-                re[x0 + i] = slot[i].re;
-                im[x0 + i] = slot[i].im;
-            }
-        return e;
+    return io_chunks(h, dim_user, h->sv, false, "get_state", [&](uint64_t x0, size_t cnt, c64* slot) {
+        for (size_t i = 0; i < cnt; i++) {
+            re[x0 + i] = slot[i].re;
+            im[x0 + i] = slot[i].im;
+        }
     });
 }
 
