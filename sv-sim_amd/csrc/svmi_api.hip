@@ -941,17 +941,19 @@ svmi_status pauli_device(svmi_handle h, const c64* psi, const svmi_pauli_term* t
     return SVMI_OK;
 }
 
-// Host copies of the state (AoS device <-> SoA host) in chunks through pinned
-// slots.  From 8 chunks on four workers take a quarter each (neighbours in the
-// host arrays, whose large pages they then fault in alone): a worker's share of
-// the (un)interleaving and of the page faults of a new host array runs while
-// the others' chunks are on the bus.  Below, starting threads costs more than
-// it saves, and one worker fills a slot while the slots before it are copied.
-// A state of 2^21 amplitudes: set 1.9 -> 0.9 ms, get 3.5 -> 1.0 ms (one slot
-// allocated per call, one thread).
+// Host copies of the state (AoS device <-> SoA host) in chunks through a ring of
+// pinned slots: one is (un)interleaved while the others are on the bus.  A state
+// of 2^21 amplitudes: set 2.2 -> 1.2 ms, get into new arrays 3.6 -> 3.0 ms (one
+// slot allocated per call).  From 2^22 amplitudes on get_state takes four
+// workers, a quarter of the host arrays each (so that no two fault in the same
+// large page), mainly for the page faults of new arrays: 2^23 amplitudes 10.6 ->
+// 5.1 ms.  Smaller states are left to the caller's thread: in a quiet process
+// four workers read 2^21 amplitudes in 1.5 ms, but beside other threads (a
+// program that also runs torch) their wake-ups cost more than they save: set and
+// get 4.9 ms with one slot per call, 5.4-7.3 with workers, 3.8 without.
 constexpr size_t kChunk = size_t(1) << 17;   // amplitudes of a slot (2 MiB)
 constexpr int kIoSlots = 4;
-constexpr uint64_t kIoThreadedChunks = 8;
+constexpr uint64_t kIoThreadedChunks = 32;
 
 // The slots of a call come from a pool of the process: pinning a set and
 // faulting in its 8 MiB costs up to 4 ms (set_state of 19 qubits on a new
@@ -1018,7 +1020,7 @@ svmi_status io_chunks(svmi_handle h, uint64_t dim, c64* dev, bool to_device, con
     c64* slots = nullptr;
     SVMI_HIP(g_io.take(&slots));
     const uint64_t chunks = (dim + kChunk - 1) / kChunk;
-    const int workers = chunks >= kIoThreadedChunks ? kIoSlots : 1, ring = kIoSlots / workers;
+    const int workers = !to_device && chunks >= kIoThreadedChunks ? kIoSlots : 1, ring = kIoSlots / workers;
     std::atomic<int> err{int(hipSuccess)};
     const auto work = [&](int w) {
         hipError_t e = hipSetDevice(h->device);

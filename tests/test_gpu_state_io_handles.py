@@ -1,6 +1,6 @@
-"""GPU: set_state / get_state on new handles: one worker cycling through the
-slots (up to 7 chunks of 2^17 amplitudes), four with a quarter each (from 8 on),
-the slots of the process handed from one handle to the next.  Copies, so every
+"""GPU: set_state / get_state on new handles: the caller's thread cycling
+through the slots, from 32 chunks of 2^17 amplitudes on four workers with a
+quarter each, the slots of the process handed from one handle to the next.  Copies, so every
 bit must come back."""
 import numpy as np
 import pytest
