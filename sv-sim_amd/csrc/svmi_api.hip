@@ -175,7 +175,8 @@ struct DevBuf {
 // A program's tables in one device buffer, filled by one copy.
 struct DeviceProgram {
     DevBuf buf;
-    std::vector<unsigned char> host;   // the copy's source, until the upload's synchronisation
+    std::vector<unsigned char> host;   // the copy's source; kept up to kKept for the next upload
+    static constexpr size_t kKept = size_t(1) << 20;
     size_t o_ops = 0, o_coef = 0, o_lph = 0, o_lane = 0, o_wave = 0, o_io = 0;
     template <class T>
     size_t put(const std::vector<T>& v, size_t pad = 0)
@@ -210,6 +211,7 @@ struct DeviceProgram {
         SVMI_TRY(buf.ensure(host.size()));
         SVMI_HIP(hipMemcpyAsync(buf.p, host.data(), host.size(), hipMemcpyHostToDevice, st));
         SVMI_HIP(hipStreamSynchronize(st));
+        if (host.capacity() > kKept) std::vector<unsigned char>().swap(host);
         return SVMI_OK;
     }
     template <class T>
