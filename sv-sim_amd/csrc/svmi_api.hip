@@ -479,6 +479,11 @@ svmi_status verify_batch(const BatchPlan& bp)
     return SVMI_OK;
 }
 
+// Low qubits of a batch's tiles, an item's own or the table's, so that the tuner
+// measures what the table's users get: 3, as default_tile; 4 in tiles that could
+// not hold them and the widest op, which are refused as ever.
+int batch_low_qubits(int tile) { return tile >= 2 * kRegBits ? 3 : 4; }
+
 svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const double* expvals, const double* grads,
                         BatchPlan& bp)
 {
@@ -515,15 +520,14 @@ svmi_status build_batch(const svmi_batch_item* items, size_t n_items, const doub
                 PlanOptions of;
                 of.tile_qubits = it.fwd_tile ? it.fwd_tile : tu.fwd_tile;
                 of.op_overhead = it.op_cost ? it.op_cost - 1 : tu.op_cost;
-                if (!it.fwd_tile) of.low_qubits = 3;   // as default_tile
+                of.low_qubits = batch_low_qubits(of.tile_qubits);
                 plan_forward(it.gates, it.n_gates, ni[i], of, bp.fwd[i]);
                 std::vector<AdjEntry> entries;
                 adjoint_entries(it.gates, it.n_gates, it.param_slots, entries);
                 PlanOptions oa;
-                // (16 circuits of 20-22 qubits with backward tiles of 11 / 12: 15.1 / 14.5 ms)
-                oa.tile_qubits = it.adj_tile ? it.adj_tile : ni[i] >= 18 ? kMaxTileQubitsAdj : tu.adj_tile;
+                oa.tile_qubits = it.adj_tile ? it.adj_tile : ni[i] >= kBatchLargeAdj ? kMaxTileQubitsAdj : tu.adj_tile;
                 oa.op_overhead = of.op_overhead;
-                if (!it.adj_tile) oa.low_qubits = 3;
+                oa.low_qubits = batch_low_qubits(oa.tile_qubits);
                 build_adjoint_program(entries, ni[i], oa, bp.adj[i]);
                 plan_pauli(it.terms, it.n_terms, ni[i], kPauliTileQubits, true, 1, pauli[i]);
             }

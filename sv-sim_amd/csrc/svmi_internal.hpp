@@ -89,6 +89,9 @@ constexpr int kRegs = 1 << kRegBits;        // amplitudes per thread per group
 constexpr int kMaxTileQubits = 13;          // 512 threads, 64 KiB of exchange area: two tiles per CU
 constexpr int kMaxTileQubitsAdj = 12;       // two states (phi, lambda): the same threads and LDS
 constexpr int kMaxBatchAdjTile = 11;        // largest svmi_batch_item::adj_tile
+constexpr int kBatchLargeAdj = 18;          // from this many qubits on a batch's backward tiles have 12
+                                            // qubits unless the item says (16 circuits of 20-22 qubits
+                                            // with 11 / 12: 15.1 / 14.5 ms)
 // Two-state phases have 3 register bits; their fourth register "bit" is k,
 // the bit above the tile, which selects the state (phi at positions
 // [0, 2^k), lambda at [2^k, 2^(k+1))).  A thread's 16-amplitude group is then

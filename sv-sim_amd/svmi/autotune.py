@@ -5,10 +5,13 @@ gradient, planning included) on a batch of hardware-efficient-ansatz circuits
 of that size -- the gate pattern and observable of the batched workload, layer
 counts 2..10 -- and picks, by coordinate descent from the single-circuit
 settings, the fusion op cost, then the forward sweep tile, then the backward
-sweep tile.  A candidate replaces the current choice only when it is more than
-3 % faster (median of 3 runs).  The result is written as the C++ table
-sv-sim_amd/csrc/svmi_tuning.hpp (rebuild the library afterwards) and a JSON
-log of every measurement.
+sweep tile (below 18 qubits: from there on the engine's own is 12, more than an
+item can ask for, and every candidate runs with it).  A candidate replaces the
+current choice only when it is more than 3 % faster (median of 3 runs).  The
+result is written as the C++ table sv-sim_amd/csrc/svmi_tuning.hpp (rebuild the
+library afterwards) and a JSON log of every measurement.  Batches of one size
+say little about mixed ones: compare the two tables there before the new one
+stays (--out writes it elsewhere).
 
   python -m svmi.autotune [--nmin 4] [--nmax 22] [--out PATH] [--json PATH]
 
@@ -26,8 +29,13 @@ from svmi import workloads as W
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 DEFAULT_OUT = os.path.join(os.path.dirname(HERE), "csrc", "svmi_tuning.hpp")
-DEFAULT = {"fwd_tile": 12, "adj_tile": 11, "op_cost": 2}
 MAX_N = 30
+LARGE_ADJ = 18   # kBatchLargeAdj (csrc/svmi_internal.hpp)
+
+
+def default(n):
+    """The single-circuit settings."""
+    return {"fwd_tile": 13 if n >= 21 else 12, "adj_tile": 11, "op_cost": 2}
 
 
 def batch_for(n, seed):
@@ -43,6 +51,8 @@ def batch_for(n, seed):
 
 
 def time_batch(items, setting, reps=3):
+    if items[0]["n"] >= LARGE_ADJ:
+        setting = dict(setting, adj_tile=0)
     run = [dict(it, **setting) for it in items]
     svmi.batch_adjoint(run)
     ts = []
@@ -55,13 +65,13 @@ def time_batch(items, setting, reps=3):
 
 def tune_n(n, log):
     items = batch_for(n, seed=9000 + n)
-    best = dict(DEFAULT)
+    best = default(n)
     best_t = time_batch(items, best)
     log.append({"n": n, "setting": dict(best), "ms": best_t * 1e3})
     space = {
         "op_cost": [0, 1, 2, 4, 8],
         "fwd_tile": sorted({min(k, max(n, 4)) for k in (6, 8, 10, 12, 13)}),
-        "adj_tile": sorted({min(k, max(n, 4)) for k in (6, 8, 9, 10, 11)}),
+        "adj_tile": sorted({min(k, max(n, 4)) for k in (6, 8, 9, 10, 11)}) if n < LARGE_ADJ else [],
     }
     for key in ("op_cost", "fwd_tile", "adj_tile"):
         for v in space[key]:
@@ -79,12 +89,13 @@ def tune_n(n, log):
 def write_header(path, table, source):
     rows = []
     for n in range(4, MAX_N + 1):
-        e = table.get(n, DEFAULT)
+        e = table.get(n, default(n))
         rows.append(f"{{{n}, {e['fwd_tile']}, {e['adj_tile']}, {e['op_cost']}}}")
     body = ",\n    ".join(", ".join(rows[i:i + 6]) for i in range(0, len(rows), 6))
     text = f'''// svmi_tuning.hpp -- planning of batched circuits per qubit count.
 // Generated by svmi/autotune.py: {source}.
-// Sizes outside the tuned range keep the single-circuit settings.
+// Sizes outside the tuned range keep the single-circuit settings.  From
+// kBatchLargeAdj qubits on adj_tile is not read.
 #pragma once
 
 #include <stdint.h>
