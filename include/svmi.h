@@ -119,7 +119,7 @@ typedef enum svmi_option {
                                  form from a run of gates inside one phase (default 2)       */
     SVMI_OPT_PREFETCH = 10,   /* 0 or 1, no effect (see SVMI_OPT_PIPELINE)                    */
     SVMI_OPT_TILE_MAP = 11    /* 1 = CX and SWAP gates on two tile qubits that a phase does not
-                                 hold in registers relabel the tile's LDS indices instead of
+                                 hold in registers relabel the tile's positions instead of
                                  needing a phase (default; with SVMI_OPT_SPECIALIZE only below
                                  20 qubits); 0 = off                                         */
 } svmi_option;

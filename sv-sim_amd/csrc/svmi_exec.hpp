@@ -364,7 +364,7 @@ SVMI_HD inline void apply_rot(const DOpHdr& h, c64 (&a)[N], const c64* __restric
 #undef SVMI_ROT_SLOT
 }
 
-// h = the op's header (prefetched), op = the op in memory (diagonal tail),
+// h = the op's header, op = the op in memory (diagonal tail),
 // grp = the group index (goff with the register bits squeezed out).
 // vmask / vhi: the sweep's variant qubits (SweepInfo::exthi) and the tile
 // base's bits there, so a table over all of them finds its variant with one

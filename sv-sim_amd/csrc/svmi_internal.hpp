@@ -176,8 +176,8 @@ constexpr int kMaxPhaseFactors = 64;   // factor slots per sweep (LDS: 16 B each
 enum : uint8_t { DOP_TO_PSI = 1, DOP_TO_LAM = 2, DOP_TO_BOTH = 3 };
 
 // One device op (uniform across the workgroup).  Every field is a full
-// dword so the kernels fetch it with scalar loads; the kernels prefetch the
-// 40-byte header one op ahead and read the diagonal-op tail on demand.
+// dword so the kernels fetch it with scalar loads: the 40-byte header (the
+// latency builds one op ahead), the diagonal-op tail on demand.
 struct DOpHdr {
     uint32_t type;
     uint32_t smask;      // DENSE / GRAD_DENSE: register slot mask

@@ -6,17 +6,17 @@
 // of that dispatch, which costs register copies per op.  For a fixed circuit
 // the op list is known at upload, so each sweep can instead be emitted as
 // straight-line HIP code -- the steps of the interpreter (loads, exchanges,
-// stores of svmi_layout.cpp, with literal offsets) and, per op, a direct call of its template (svmi_internal.hpp) with register slots,
-// condition masks and coefficient offsets as literals -- and compiled with
-// hipRTC for the device.  The coefficients stay in the program's coefficient
+// stores of svmi_layout.cpp, with literal offsets) and, per op, a direct call of
+// its template (svmi_internal.hpp) with register slots, condition masks and
+// coefficient offsets as literals -- and compiled with hipRTC for the device.  The coefficients stay in the program's coefficient
 // array, so circuits that differ only in angles give the same source (and
 // hit hipRTC's cache).  Same arithmetic in the same order: the results equal
 // the interpreted sweeps'.
 //
-// Cost: compilation is serialised inside the process and takes from about
-// a second (QFT, 33 qubits, 6 sweeps) to tens of seconds (20 layers of a
-// dense u3 brickwall, 24 sweeps of 16x16 ops), so this pays for circuits
-// that run many times.
+// Cost: compilation is serialised inside the process and takes from about half
+// a second (QFT, 33 qubits, 6 sweeps) to a few (20 layers of a dense u3
+// brickwall of 30 qubits, 19 sweeps: 2.4 s), so this pays for circuits that run
+// many times.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -63,9 +63,8 @@ tile_factors(c64* xf, const SweepInfo& sw, const DOp* __restrict__ ops, const c6
     }
 }
 
-// LDS of a tile: exchange area (8 bytes per amplitude of every state, 16 where
-// whole amplitudes change threads) | phase
-// factors | gradient accumulators.
+// LDS of a tile: exchange area (8 bytes per amplitude of every state; SweepInfo::whole
+// adds as much) | phase factors | gradient accumulators.
 size_t sweep_smem_bytes(const SweepInfo& sw, int ns)
 {
     const size_t nwaves = (size_t(sweep_threads(sw.k, ns)) + 63) / 64;
@@ -291,7 +290,7 @@ sweep_tile(c64* __restrict__ s0, c64* __restrict__ s1, const SweepInfo& sw, cons
             c64* const to = stage + ((p + 1 - ph_begin) & 1u) * sw.stage;
 #pragma unroll
             for (uint32_t i = 0; i < kPre; i++)
-                if (stid + snt * i < pre_n) to[stid + snt * i] = c64{pre[i].re, pre[i].im};   // (by value: see k_pauli)
+                if (stid + snt * i < pre_n) to[stid + snt * i] = c64{pre[i].re, pre[i].im};   // (copied whole, pre[] stays in scratch memory)
             for (uint32_t i = stid + snt * kPre; i < pre_n; i += snt) to[i] = coef[pre_c + i];
             __syncthreads();
         }

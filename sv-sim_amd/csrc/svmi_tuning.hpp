@@ -1,7 +1,7 @@
 // svmi_tuning.hpp -- planning of batched circuits per qubit count.
-// 4 to 12 qubits: by svmi/autotune.py (AMD Radeon Graphics (gfx950), 2026-12-02).
-// From 13 on the forward tiles and op costs were set by hand for the sweeps that
-// hold their tile in registers, on batches of mixed sizes: what the tuner finds
+// By svmi/autotune.py (AMD Radeon Graphics (gfx950), n = 4..22, 2026-12-02).
+// From 13 on the tiles were set by hand for the sweeps that hold their tile in
+// registers, on batches of mixed sizes: what the tuner finds
 // for batches of one size (its candidates differ by less than its runs there)
 // runs 96 circuits of 10-20 qubits in 12.9 ms instead of 12.2, 32 of 12-18 in
 // 5.3 instead of 5.0.  So compare its output on mixed batches before it takes
@@ -19,7 +19,7 @@ struct BatchTuning {
     uint8_t op_cost;    // fusion op cost
 };
 
-constexpr const char* kBatchTuningSource = "AMD Radeon Graphics (gfx950), n = 4..12 2026-12-02; by hand from 13";
+constexpr const char* kBatchTuningSource = "AMD Radeon Graphics (gfx950), n = 4..22 2026-12-02; tiles by hand from 13";
 constexpr BatchTuning kBatchTuning[] = {
     {4, 12, 11, 1}, {5, 12, 11, 0}, {6, 12, 11, 0}, {7, 12, 11, 1}, {8, 12, 11, 0}, {9, 9, 11, 0},
     {10, 12, 10, 0}, {11, 12, 11, 0}, {12, 12, 11, 0}, {13, 13, 11, 0}, {14, 13, 11, 1}, {15, 13, 11, 1},
