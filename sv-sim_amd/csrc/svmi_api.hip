@@ -3,6 +3,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <cmath>
@@ -766,7 +768,7 @@ struct svmi_sim {
     std::string jit_error;     // why the last specialisation failed (the sweeps then interpret)
     PlanOptions opt;
     bool profile = false;
-    hipEvent_t io_ev[4] = {};      // set_state / get_state: a worker's copy is done
+    hipEvent_t io_ev[8] = {};      // set_state / get_state: the copy of a slot is done
     std::vector<hipEvent_t> prof_events;
     std::vector<double> step_ms;   // with profiling: per-step times of the last program run
     svmi_stats stats{};
@@ -947,23 +949,25 @@ svmi_status pauli_device(svmi_handle h, const c64* psi, const svmi_pauli_term* t
     return SVMI_OK;
 }
 
-// Host copies of the state (AoS device <-> SoA host) in chunks through a ring of
-// pinned slots: one is (un)interleaved while the others are on the bus.  A state
-// of 2^21 amplitudes: set 2.2 -> 1.2 ms, get into new arrays 3.6 -> 3.0 ms (one
-// slot allocated per call).  From 2^22 amplitudes on get_state takes four
-// workers, a quarter of the host arrays each (so that no two fault in the same
-// large page), mainly for the page faults of new arrays: 2^23 amplitudes 10.6 ->
-// 5.1 ms.  Smaller states are left to the caller's thread: in a quiet process
-// four workers read 2^21 amplitudes in 1.5 ms, but beside other threads (a
-// program that also runs torch) their wake-ups cost more than they save: set and
-// get 4.9 ms with one slot per call, 5.4-7.3 with workers, 3.8 without.
+// Host copies of the state (AoS device <-> SoA host) in chunks through pinned
+// slots, two per worker: one is (un)interleaved while the other is on the bus.
+// A run of chunks is 2 MiB of either host array, so that no two workers fault in
+// the same large page of a new array.  The caller's thread takes runs from the
+// first on; from 4 runs on helpers are started that take runs as well, if they
+// get to run in time: where the cores are busy (a program that has just run
+// numpy or torch leaves their threads spinning) a new thread waits milliseconds
+// for one, and is not waited for.  A state of 2^21 amplitudes, set and get: one
+// slot allocated per call 5.9 ms, the caller's thread alone 4.2, with helpers
+// 2.8; with spinning threads beside it 4.9, 3.8 and 3.9-4.4 (helpers that were
+// waited for: 5.4-7.3).
 constexpr size_t kChunk = size_t(1) << 17;   // amplitudes of a slot (2 MiB)
-constexpr int kIoSlots = 4;
-constexpr uint64_t kIoThreadedChunks = 32;
+constexpr uint64_t kIoRun = 2;               // chunks
+constexpr int kIoWorkers = 4, kIoSlots = 2 * kIoWorkers;
+constexpr uint64_t kIoThreadedRuns = 4;
 
 // The slots of a call come from a pool of the process: pinning a set and
-// faulting in its 8 MiB costs up to 4 ms (set_state of 19 qubits on a new
-// handle 3.7 ms, from the pool 0.27).  At most kIoKept idle sets are kept while
+// faulting in its 16 MiB costs milliseconds (set_state of 19 qubits on a new
+// handle with 8 MiB 3.7 ms, from the pool 0.29).  At most kIoKept idle sets are kept while
 // there are handles, one of them for the programs that make one handle after
 // another.
 struct IoPool {
@@ -1015,6 +1019,38 @@ struct IoPool {
 };
 IoPool g_io;
 
+// The runs of one call.  A helper holds this and touches nothing else of the call
+// unless it has a run; the call returns when no run is left and none is held.
+struct IoJob {
+    std::mutex mu;
+    std::condition_variable idle;
+    uint64_t next = 0, runs = 0;
+    int held = 0;
+    hipError_t err = hipSuccess;
+
+    bool take(uint64_t* run)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        if (err != hipSuccess || next == runs) return false;
+        *run = next++;
+        held++;
+        return true;
+    }
+    void done(hipError_t e)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        if (e != hipSuccess) err = e;
+        if (--held == 0) idle.notify_one();
+    }
+    hipError_t finish()
+    {
+        std::unique_lock<std::mutex> lk(mu);
+        next = runs;
+        idle.wait(lk, [&] { return held == 0; });
+        return err;
+    }
+};
+
 // to_device: pack(first, count, slot) fills a slot, which goes to dev + first;
 // else dev + first comes to a slot, which pack takes.
 template <class F>
@@ -1026,57 +1062,63 @@ svmi_status io_chunks(svmi_handle h, uint64_t dim, c64* dev, bool to_device, con
     c64* slots = nullptr;
     SVMI_HIP(g_io.take(&slots));
     const uint64_t chunks = (dim + kChunk - 1) / kChunk;
-    const int workers = !to_device && chunks >= kIoThreadedChunks ? kIoSlots : 1, ring = kIoSlots / workers;
-    std::atomic<int> err{int(hipSuccess)};
-    const auto work = [&](int w) {
-        hipError_t e = hipSetDevice(h->device);
-        const uint64_t c0 = chunks * uint64_t(w) / uint64_t(workers), c1 = chunks * uint64_t(w + 1) / uint64_t(workers);
+    // a run through worker w's slots
+    const auto move = [&](uint64_t run, int w) -> hipError_t {
+        hipError_t e = hipSuccess;
+        const uint64_t c0 = run * kIoRun, c1 = std::min(c0 + kIoRun, chunks);
         const auto count = [&](uint64_t c) { return size_t(std::min<uint64_t>(kChunk, dim - c * kChunk)); };
-        const auto index = [&](uint64_t c) { return w * ring + int((c - c0) % uint64_t(ring)); };
+        const auto slot = [&](uint64_t c) { return slots + size_t(2 * w + int(c & 1)) * kChunk; };
+        const auto event = [&](uint64_t c) { return h->io_ev[2 * w + int(c & 1)]; };
         const auto copy = [&](uint64_t c) {
-            c64 *slot = slots + size_t(index(c)) * kChunk, *at = dev + c * kChunk;
-            e = hipMemcpyAsync(to_device ? at : slot, to_device ? slot : at, count(c) * sizeof(c64),
+            c64* at = dev + c * kChunk;
+            e = hipMemcpyAsync(to_device ? at : slot(c), to_device ? slot(c) : at, count(c) * sizeof(c64),
                                to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, h->stream);
-            if (e == hipSuccess) e = hipEventRecord(h->io_ev[index(c)], h->stream);
+            if (e == hipSuccess) e = hipEventRecord(event(c), h->stream);
         };
         const auto wait = [&](uint64_t c) {
-            if (e == hipSuccess) e = hipEventSynchronize(h->io_ev[index(c)]);
-        };
-        const auto go = [&]() { return e == hipSuccess && err == int(hipSuccess); };
-        uint64_t issued = c0;   // chunks whose copies were given to the stream
-        if (to_device) {
-            for (uint64_t c = c0; c < c1 && go(); c++) {
-                if (c >= c0 + uint64_t(ring)) wait(c - uint64_t(ring));
-                if (e != hipSuccess) break;
-                pack(c * kChunk, count(c), slots + size_t(index(c)) * kChunk);
-                copy(c);
-                issued = c + 1;
-            }
-        } else {
-            for (uint64_t c = c0; c < c1 && go(); c++) {
-                while (issued < c1 && issued < c + uint64_t(ring) && e == hipSuccess) copy(issued++);
-                wait(c);
-                if (e == hipSuccess) pack(c * kChunk, count(c), slots + size_t(index(c)) * kChunk);
-            }
-        }
-        // the slots are given back with no copy under way
-        for (uint64_t c = issued > c0 + uint64_t(ring) ? issued - uint64_t(ring) : c0; c < issued; c++) {
-            const hipError_t s = hipEventSynchronize(h->io_ev[index(c)]);
+            const hipError_t s = hipEventSynchronize(event(c));
             if (e == hipSuccess) e = s;
+        };
+        uint64_t issued = c0, waited = c0;   // chunks whose copies were given to the stream, and are done
+        if (!to_device)
+            while (issued < c1 && issued < c0 + 2 && e == hipSuccess) copy(issued++);
+        for (uint64_t c = c0; c < c1 && e == hipSuccess; c++) {
+            if (to_device) {
+                if (c >= c0 + 2) wait(waited++);
+                if (e != hipSuccess) break;
+                pack(c * kChunk, count(c), slot(c));
+                copy(issued++);
+            } else {
+                wait(waited++);
+                if (e != hipSuccess) break;
+                pack(c * kChunk, count(c), slot(c));
+                if (issued < c1) copy(issued++);
+            }
         }
-        if (e != hipSuccess) err = int(e);
+        while (waited < issued) wait(waited++);   // the slots are free again
+        return e;
     };
-    std::vector<std::thread> pool;
-    try {
-        for (int w = 1; w < workers; w++) pool.emplace_back(work, w);
-    } catch (const std::exception&) {   // no more threads: this one takes the missing workers' chunks
+    const auto job = std::make_shared<IoJob>();
+    job->runs = (chunks + kIoRun - 1) / kIoRun;
+    if (job->runs >= kIoThreadedRuns) {
+        const int device = h->device;
+        const auto* mv = &move;
+        try {
+            for (int w = 1; w < kIoWorkers; w++)
+                std::thread([job, mv, w, device] {
+                    uint64_t run;
+                    for (bool first = true; job->take(&run); first = false) {
+                        hipError_t e = first ? hipSetDevice(device) : hipSuccess;
+                        if (e == hipSuccess) e = (*mv)(run, w);
+                        job->done(e);
+                    }
+                }).detach();
+        } catch (const std::exception&) {   // no more threads: fewer helpers
+        }
     }
-    const int started = int(pool.size()) + 1;
-    work(0);
-    for (int w = started; w < workers; w++) work(w);
-    for (auto& t : pool) t.join();
+    for (uint64_t run; job->take(&run);) job->done(move(run, 0));
+    const hipError_t e = job->finish();
     g_io.give(slots);
-    const hipError_t e = hipError_t(err.load());
     if (e != hipSuccess) return fail(SVMI_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
     return SVMI_OK;
 }
